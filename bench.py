@@ -58,7 +58,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_solve_xi_1025x257.json")
 
 def measured_traffic():
     """HBM bytes per xi-solve launch from the committed rocprofv3 --pmc runs
-    (FETCH_SIZE + WRITE_SIZE of k_solve_bc, each scaled by the counter's
+    (FETCH_SIZE + WRITE_SIZE of the solve kernel, each scaled by the counter's
     reading for a copy of known size); None when that file is absent"""
     try:
         with open(TRAFFIC_FILE) as f:
@@ -168,7 +168,7 @@ def main():
         "config": {"workload": "LNS3D implicit AF step: lrhs3D + xi/eta block-penta line solves + "
                                "update, complex double, factors formed once",
                    "nx": NX, "ny": NY, "beta": BETA, "Ma": p.Ma, "Re": p.Re, "cfl": p.cflmax},
-        "roofline": {"bound": "hbm", "kernel": "k_solve_tw<double,6,1,false,4,true> (xi lines: 257 lines x 1025 rows, twisted, column halves)",
+        "roofline": {"bound": "hbm", "kernel": "k_line_solve<double,6,4,true,false> (xi lines: 257 lines x 1025 rows, twisted)",
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic(),
                      "bytes_per_launch": bytes_launch,

@@ -423,10 +423,11 @@ int lns3d_graph_synchronize(lns3d_graph *g);
 int lns3d_graph_destroy(lns3d_graph *g);
 /* autotuner of the line solves: times every solve-kernel variant on
  * synthetic lines of n rows x lines and uses the fastest for plans of that
- * shape created later.  Variants: 0 one line per workgroup, 1 four lines,
- * 2 twisted (two chains per line, n >= 16), 3 two lines, 4 three lines,
- * 5 twisted with chain steps taken in pairs, 6 twisted with each row's
- * columns split over the two halves of a wave.  times_ms (may be NULL)
+ * shape created later.  Variants: 0 plain lines and 2 twisted lines (two
+ * chains per line, n >= 16), each with the form of the streaming solve that a
+ * rule on the shape picks; with a pinned form 3 and 5 (six-row chunks), 4
+ * and 6 (small LDS footprint, plain and twisted) and 1 (plain, the smallest
+ * chunks; complex float: the longest).  times_ms (may be NULL)
  * receives LNS3D_TUNE_VARIANTS timings in ms (-1: not applicable).  No
  * counterpart in the reference. */
 #define LNS3D_TUNE_VARIANTS 7

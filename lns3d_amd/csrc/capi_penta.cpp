@@ -59,10 +59,10 @@ extern "C" int lns3d_penta_create(int kind, int layout, int nsys, int nrows, int
   h->layout = layout;
   h->nsys = nsys;
   h->nrows = nrows;
-  int rc = penta_plan_create(&h->plan, kind, exact, nrows, nsys, precision);
+  int rc = penta_plan_create(&h->plan, kind, exact, nrows, nsys, precision, true);
   if (!rc && kind == 1 && precision == 1) {
     h->has64 = true;
-    rc = penta_plan_create(&h->plan64, kind, exact, nrows, nsys, 0);
+    rc = penta_plan_create(&h->plan64, kind, exact, nrows, nsys, 0, true);
   }
   if (rc) {
     penta_plan_destroy(&h->plan);

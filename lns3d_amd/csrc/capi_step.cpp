@@ -117,8 +117,8 @@ extern "C" int lns3d_ctx_create(const lns3d_params *p, lns3d_ctx **out) {
       hipMalloc(&c->r, (size_t)P * 5 * 16) != hipSuccess ||
       hipMalloc(&c->scal, 4096 * sizeof(double)) != hipSuccess)
     return bail(fail(LNS3D_EHIP, "hipMalloc work"));
-  rc = penta_plan_create(&c->px, p->xper, p->periodic_exact, p->nx, p->ny, 0);
-  if (!rc) rc = penta_plan_create(&c->py, p->yper, p->periodic_exact, p->ny, p->nx, 0);
+  rc = penta_plan_create(&c->px, p->xper, p->periodic_exact, p->nx, p->ny, 0, false);
+  if (!rc) rc = penta_plan_create(&c->py, p->yper, p->periodic_exact, p->ny, p->nx, 0, false);
   if (rc) return bail(rc);
   *out = c;
   return 0;
@@ -514,9 +514,9 @@ extern "C" int lns3d_factor(lns3d_ctx *c) {
       // bottom-up): take the tuned complex-float variant when it is of the
       // same family, else the family's default.
       auto family_variant = [](const PentaPlan &d, int n, long lines) {
-        const int v = penta_variant_for(n, lines, 1);
+        const int v = penta_variant_for(n, lines, 1, false);
         if (penta_twisted(v) == (d.h >= 0)) return v;
-        return d.h >= 0 ? (int)PENTA_TWISTED_PAIRS : (lines >= 512 ? (int)PENTA_PLAIN3 : (int)PENTA_PLAIN1);
+        return d.h >= 0 ? (int)PENTA_TWISTED : (int)PENTA_PLAIN1;
       };
       // periodic lines: complex-float records rounded from the complex-double ones
       rc = penta_plan_create_variant(&c->px32, c->p.xper, 0, c->p.nx, c->p.ny, 1,
@@ -899,7 +899,7 @@ extern "C" int lns3d_ctx_bytes(const lns3d_params *p, size_t *bytes) {
   auto plan = [&](int periodic, size_t es) {
     size_t x = P * 125 * 16;                                  // LU working copy
     if (periodic) x += 2 * P * 50 * 16;
-    else x += P * 126 * es + P * 2 * 150 * es / 32 + P * 100 * 16 / 32 + P * 26 * es;   // + pair side blocks
+    else x += P * 126 * es + P * 2 * 150 * es / 32 + P * 100 * 16 / 32 + P * 26 * es;   // (26: room)
     return x;
   };
   b += plan(p->xper, 16) + plan(p->yper, 16);

@@ -23,13 +23,13 @@
 //     (cpenta1bc.f:499-847); the per-row critical path becomes one 5x5
 //     matvec.  Boundary rows 0,1 and n-2,n-1 carry extra blocks, kept in a
 //     per-line tail record.
-//  3. k_solve_tw (twisted lines) / k_solve_bc: waves 1-3 stream chunks of
-//     records into a double-buffered LDS ring and compute the parallel parts
-//     (Linv b, Uinv y); wave 0 runs the serial recurrences, one line or one
-//     chain per 16-lane DPP row, lanes 0..4 owning one component each.
+//  3. k_line_solve (line_solve.hpp): one wave runs two chains of rows (a
+//     twisted line's halves, or two plain lines), one component's real or
+//     imaginary part per lane; three waves stream the records through an LDS
+//     ring and compute the parallel parts (Linv b, Uinv y).
 //  Periodic lines: k_records_per forms the same records from the bordered
 //  LU plus two border blocks per row (p2: rows n-2, n-1 in column i; qp:
-//  row i in columns n-2, n-1), and k_solve_per streams them like k_solve_bc
+//  row i in columns n-2, n-1), and k_solve_per streams them through a ring
 //  with the border sums formed by the loader waves.  k_solve_lines (one lane
 //  per line, the reference's substitution order on the LU working copy) is
 //  kept as the order-exact solve behind lns3d_penta_solve_reference_order.
@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "line_solve.hpp"
 #include "penta.hpp"
 
 namespace lns3d {
@@ -338,9 +339,10 @@ __global__ void k_solve_lines(LineGeom g, const cx<T> *mat_, const cx<T> *per_, 
 
 // ---------------------------------------------------------------------------
 // stage 2: records for the fast non-periodic solve
-// fwd[(line*n + i)*60 + f]: f = m*10 + q -> N2(m,q); m*10 + 5 + q -> N1(m,q);
-//                           50 + k -> strict lower of Linv, k = l*(l-1)/2 + q
-// bwd[(line*n + i)*66 + f] (one complex of padding): f = m*10 + q -> Q4(m,q); m*10 + 5 + q -> Q5(m,q);
+// fwd[(line*n + i)*60 + ...]: 50 complex of N2 and N1, a component's rows as
+//                           20 reals (rec_pos); 50 + k -> strict lower of
+//                           Linv, k = l*(l-1)/2 + q
+// bwd[(line*n + i)*66 + ...] (one complex of padding): Q4 and Q5 likewise;
 //                           50 + k -> upper of Uinv (row-major, incl. diagonal)
 // tail[line*150 + ...]: 0 row n-2 N(col n-5); 25 row n-1 N(col n-5);
 //                       50 row n-1 N(col n-4); 75 row 0 Q(col 3);
@@ -424,10 +426,15 @@ __global__ __launch_bounds__(256) void k_records_rows(LineGeom g, const cx<TF> *
   cx<TR> *B = bwd + idx * 66;
   cx<TR> *Tl = tail + (line * nchain + t) * 150;
   if (valid && act) {
-    F[m * 10 + q] = Nent(i - dir);
-    F[m * 10 + 5 + q] = Nent(i - 2 * dir);
-    B[m * 10 + q] = Qent(i + dir);
-    B[m * 10 + 5 + q] = Qent(i + 2 * dir);
+    auto put = [&](cx<TR> *rec, int older, cx<TR> v) {
+      TR *w = reinterpret_cast<TR *>(rec) + m * 20 + rec_pos(older, q);
+      w[0] = v.re;
+      w[10] = v.im;
+    };
+    put(F, 0, Nent(i - dir));
+    put(F, 1, Nent(i - 2 * dir));
+    put(B, 0, Qent(i + dir));
+    put(B, 1, Qent(i + 2 * dir));
     // forward blocks of the chain's last two rows outside the band: columns
     // n-5, n-4 (plain) or the bottom chain's last rows h+2, h+3 (twisted);
     // the bottom chain of a twisted factor has none (zeros)
@@ -453,93 +460,6 @@ __global__ __launch_bounds__(256) void k_records_rows(LineGeom g, const cx<TF> *
     } else {
       B[65] = cx<TR>{0, 0};
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Twisted lines take their chain steps in pairs where no hand-off or boundary
-// block is involved.  In processing order a step is u_s = c_s + W2_s u_{s-1}
-// + W1_s u_{s-2} (forward W2 = N2, W1 = N1; backward W2 = Q4, W1 = Q5).  The
-// second step of a pair written in the same inputs as the first,
-//   u_{s+1} = c' + W2' u_{s-1} + W1' u_{s-2},
-//   W2' = W1_{s+1} + W2_{s+1} W2_s,  W1' = W2_{s+1} W1_s,  c' = c_{s+1} + W2_{s+1} c_s,
-// lets the solve form both at once (lanes 0-4 and 5-9 of a DPP row).  The
-// factor rewrites the second step's record with W2', W1' and keeps
-// M = W2_{s+1} Linv_s (forward) / W2_{s+1} Uinv_s (backward) in a side array
-// (xf / xb, 25 complex per pair), so that the solve's loader waves form
-// c' = Linv_{s+1} b_{s+1} + M b_s (forward; backward with Uinv and the
-// forward result) from the staged right-hand sides in one pass.
-//
-// Pairs (s, s+1), s even, of chunk k (steps [kR, min(kR+R, len0))) lie in
-// [p_end, m_end); the same rule on both sides, as it depends on the solve's
-// chunk size R.
-__host__ __device__ inline void tw_pair_range(int R, int k, bool fw, int len0, int len1, int &p_end,
-                                              int &m_end) {
-  const int p0 = fw ? 0 : 4;                                   // even, after the backward hand-off
-  const int main_hi = fw ? len1 - 2 : (len0 - 5 < len1 - 3 ? len0 - 5 : len1 - 3);
-  const int s_begin = k * R, s_end = (k * R + R < len0) ? k * R + R : len0;
-  p_end = s_begin > (p0 < s_end ? p0 : s_end) ? s_begin : (p0 < s_end ? p0 : s_end);
-  const int hi = main_hi < s_end ? main_hi : s_end;
-  m_end = p_end + ((hi > p_end ? hi - p_end : 0) / 6) * 6;
-}
-// chunk size of the twisted solve for a record precision
-constexpr int tw_chunk(bool single) { return single ? 12 : 6; }
-
-// the pair rewrite at factor time: one 32-lane group per (line, chain, pass,
-// pair), lane (m, q) of lanes 0..24 forms entry (m, q) of W2', W1' and M
-template <typename TR>
-__global__ __launch_bounds__(256) void k_pair_records(int n, int h, long L, int R, cx<TR> *fwd, cx<TR> *bwd,
-                                                      cx<TR> *xf, cx<TR> *xb) {
-  const int len0 = h + 2, len1 = n - h - 2, npair = (len0 + 1) / 2;
-  const int grp = threadIdx.x >> 5, gl = threadIdx.x & 31;
-  const long id = (long)blockIdx.x * 8 + grp;     // ((line * 2 + chain) * 2 + pass) * npair + pair
-  const long total = L * 4 * npair;
-  const long idc = id < total ? id : total - 1;
-  const int q2 = (int)(idc % npair), pass = (int)((idc / npair) % 2), cc = (int)((idc / npair / 2) % 2);
-  const long line = idc / npair / 4;
-  const bool fw = pass == 0;
-  const int s = 2 * q2;
-  int p_end, m_end;
-  tw_pair_range(R, s / R, fw, len0, len1, p_end, m_end);
-  const bool is_pair = id < total && s >= p_end && s + 1 < m_end;
-  // chain rows of steps s, s+1 and their records
-  const int coff = cc * len0;
-  const int j0 = fw ? s : len0 - 1 - s + cc * (len1 + 2 - len0);
-  const int j1 = fw ? j0 + 1 : j0 - 1;
-  const int stride = fw ? 60 : 66;
-  cx<TR> *base = fw ? fwd : bwd;
-  cx<TR> *r0 = base + (line * n + coff + (is_pair ? j0 : 0)) * stride;
-  cx<TR> *r1 = base + (line * n + coff + (is_pair ? j1 : 0)) * stride;
-  cx<TR> *x = (fw ? xf : xb) + ((line * 2 + cc) * npair + q2) * 25;
-  const int m = gl / 5, q = gl % 5;
-  cx<double> w2n{0, 0}, w1n{0, 0}, mx{0, 0};
-  if (is_pair && gl < 25) {
-    // M(m, q) = (W2_{s+1} Linv_s)(m, q) forward (Linv: unit lower, strict
-    // part at 50 + l(l-1)/2 + c), (W2_{s+1} Uinv_s)(m, q) backward (Uinv:
-    // upper incl. diagonal at 50 + 5k - k(k-1)/2 + (c - k))
-#pragma unroll
-    for (int k = 0; k < 5; k++) {
-      const cx<double> a{(double)r1[m * 10 + k].re, (double)r1[m * 10 + k].im};
-      cx<TR> lk{0, 0};
-      if (fw) lk = k == q ? cx<TR>{1, 0} : (k > q ? r0[50 + k * (k - 1) / 2 + q] : cx<TR>{0, 0});
-      else if (k <= q) lk = r0[50 + 5 * k - k * (k - 1) / 2 + (q - k)];
-      mx = cfma(a, cx<double>{(double)lk.re, (double)lk.im}, mx);
-    }
-    w2n = cx<double>{(double)r1[m * 10 + 5 + q].re, (double)r1[m * 10 + 5 + q].im};
-#pragma unroll
-    for (int k = 0; k < 5; k++) {
-      const cx<double> a{(double)r1[m * 10 + k].re, (double)r1[m * 10 + k].im};
-      const cx<double> b2{(double)r0[k * 10 + q].re, (double)r0[k * 10 + q].im};
-      const cx<double> b1{(double)r0[k * 10 + 5 + q].re, (double)r0[k * 10 + 5 + q].im};
-      w2n = cfma(a, b2, w2n);
-      w1n = cfma(a, b1, w1n);
-    }
-  }
-  wave_sync();
-  if (is_pair && gl < 25) {
-    x[m * 5 + q] = cx<TR>{(TR)mx.re, (TR)mx.im};
-    r1[m * 10 + q] = cx<TR>{(TR)w2n.re, (TR)w2n.im};
-    r1[m * 10 + 5 + q] = cx<TR>{(TR)w1n.re, (TR)w1n.im};
   }
 }
 
@@ -814,7 +734,6 @@ __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *l
 //     (forward) or d_i = Uinv_i y_i (backward).
 // A chunk's copies so have two iterations to arrive while the compute wave
 // works through the chunks before it.
-typedef __attribute__((address_space(3))) void lds_void;
 
 template <typename T>
 __device__ __forceinline__ void copy_rows_to_lds(const cx<T> *src, long src_elems_left, cx<T> *dst,
@@ -830,20 +749,6 @@ __device__ __forceinline__ void copy_rows_to_lds(const cx<T> *src, long src_elem
     if (ec < 0) ec = 0;
     __builtin_amdgcn_global_load_lds((const void *)(src + ec),
                                      (lds_void *)(dst + (long)b * 64 * PER_LANE), 16, 0, 0);
-  }
-}
-
-// one wave copies nelem complex values src[0..nelem) into LDS at dst, 1 KB
-// (16 B per lane) per instruction; lanes past the end are masked off (nelem
-// is even for complex float, so no lane copies past the end)
-template <typename T>
-__device__ __forceinline__ void dma_rows(const cx<T> *src, cx<T> *dst, int nelem, int lane) {
-  constexpr int PER_LANE = 16 / sizeof(cx<T>);
-  for (int b = 0; b * 64 * PER_LANE < nelem; b++) {
-    const int e = (b * 64 + lane) * PER_LANE;
-    if (e < nelem)
-      __builtin_amdgcn_global_load_lds((const void *)(src + e), (lds_void *)(dst + b * 64 * PER_LANE),
-                                       16, 0, 0);
   }
 }
 
@@ -875,69 +780,6 @@ __device__ __forceinline__ void parallel_part(double2 *bp, const cx<T> *rp, int 
         acc = cfma(Ui[q], cx<T>{(T)yq.x, (T)yq.y}, acc);
       }
   }
-  *reinterpret_cast<cx<T> *>(bp + mm) = acc;
-}
-
-// The workgroup barrier of the loader waves: their LDS writes are complete
-// (lgkmcnt 0) but the copies they have in flight are not waited for, as a
-// __syncthreads fence would (it treats global_load_lds as pending LDS
-// writes).  The empty asm statements keep the compiler from moving memory
-// accesses across the barrier.
-__device__ __forceinline__ void loader_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);     // lgkmcnt(0); vmcnt, expcnt not waited for
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// the parallel part of a row, plus M b_prev for the second step of a pair
-// (M: the pair's side block, b_prev: the staged right-hand side of the first
-// step).  One straight-line path for every lane of a round, so that all of
-// them read before any writes.
-template <typename T>
-__device__ __forceinline__ void parallel_part_x(double2 *bp, const cx<T> *rp, const cx<T> *M,
-                                                const double2 *bprev, int mm, bool fw, bool second) {
-  cx<T> acc{0, 0};
-  double2 bz[5];
-  cx<T> mz[5];
-#pragma unroll
-  for (int q = 0; q < 5; q++) {
-    bz[q] = bprev[q];
-    mz[q] = second ? M[mm * 5 + q] : cx<T>{0, 0};
-  }
-  if (fw) {
-    const int base = 50 + mm * (mm - 1) / 2;
-    const double2 bm = bp[mm];
-    double2 bq[4];
-    cx<T> l[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      bq[q] = bp[q];
-      l[q] = rp[min(base + q, 59)];
-    }
-    acc = cx<T>{(T)bm.x, (T)bm.y};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const cx<T> w = q < mm ? l[q] : cx<T>{0, 0};
-      acc = cfma(w, cx<T>{(T)bq[q].x, (T)bq[q].y}, acc);
-    }
-  } else {
-    const int base = 50 + mm * 5 - mm * (mm - 1) / 2;
-    double2 yq[5];
-    cx<T> u[5];
-#pragma unroll
-    for (int q = 0; q < 5; q++) {
-      yq[q] = bp[min(mm + q, 4)];
-      u[q] = rp[min(base + q, 64)];
-    }
-#pragma unroll
-    for (int q = 0; q < 5; q++) {
-      const cx<T> w = q < 5 - mm ? u[q] : cx<T>{0, 0};
-      acc = cfma(w, cx<T>{(T)yq[q].x, (T)yq[q].y}, acc);
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 5; q++) acc = cfma(mz[q], cx<T>{(T)bz[q].x, (T)bz[q].y}, acc);
   *reinterpret_cast<cx<T> *>(bp + mm) = acc;
 }
 
@@ -976,679 +818,6 @@ __device__ __forceinline__ void compute_pass(int nchunk, Body body) {
     body(k);
     __syncthreads();
   }
-}
-
-// the solve of workgroup bid (lines bid G .. bid G + cnt - 1, cnt <= G)
-template <typename T, int R, int G>
-__device__ __forceinline__ void solve_bc(long bid, int n, long L, const cx<T> *__restrict__ fwd,
-                                         const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ tail,
-                                         double2 *rhs, long sL, long sR) {
-  constexpr int NBUF = 4, BUFE = R * 66;                        // LDS record rows of one line
-  static_assert(R % 6 == 0, "a chunk is whole groups of six rows");
-  __shared__ __attribute__((aligned(16))) cx<T> rec[NBUF][G][BUFE];
-  __shared__ double2 bst[NBUF][G][R][5];    // rhs rows, then c (or d) in place
-  const long line0 = bid * G;
-  const int cnt = (int)min((long)G, L - line0);
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  // cnt lines in this workgroup; DPP row r (16 lanes) of the compute wave
-  // runs the recurrence of line g = r mod cnt (rows past the last line repeat
-  // one and store the same values).  Lane m of a row owns component m (lanes
-  // past 4 duplicate component 4).  LDS slots past cnt are not loaded.
-  const int g = (lane >> 4) % cnt;
-  const int m = min(lane & 15, 4);
-  auto line_of = [&](int gg) { return line0 + min(gg, cnt - 1); };
-  const long line = line_of(g);
-  const int nchunk = (n + R - 1) / R;
-  double2 *X = rhs + line * sL * 5;
-  const long rs = sR * 5;
-  const cx<T> *tl = tail + line * 150;
-  // rows of chunk k, ascending as they sit in LDS: [lo, lo + nr); forward
-  // chunks run up from row 0, backward chunks down from row n-1
-  auto chunk = [&](int k, bool fw, int &lo, int &nr) {
-    if (fw) {
-      lo = k * R;
-      nr = min(R, n - lo);
-    } else {
-      const int top = n - 1 - k * R;
-      nr = min(R, top + 1);
-      lo = top - nr + 1;
-    }
-  };
-
-  if (wave != 0) {
-    // ---- loader waves ----
-    auto issue = [&](int k, bool fw) {
-      const int buf = k % NBUF;
-      int lo, nr;
-      chunk(k, fw, lo, nr);
-#pragma unroll
-      for (int gg = 0; gg < G; gg++) {
-        if (gg >= cnt) break;
-        const long r0 = line_of(gg) * n + lo;
-        if (fw) dma_rows(fwd + r0 * 60, rec[buf][gg], nr * 60, lane);
-        else dma_rows(bwd + r0 * 66, rec[buf][gg], nr * 66, lane);
-      }
-      double2 *dst = &bst[buf][0][0][0];
-#pragma unroll
-      for (int b = 0; b * 64 < G * R * 5; b++) {
-        const int e = b * 64 + lane, gg = e / (R * 5), j = (e / 5) % R, q = e % 5;
-        if (e < G * R * 5 && gg < cnt && j < nr)
-          __builtin_amdgcn_global_load_lds(
-              (const void *)(rhs + line_of(gg) * sL * 5 + (long)(lo + j) * rs + q),
-              (lds_void *)(dst + b * 64), 16, 0, 0);
-      }
-    };
-    auto prep = [&](int k, bool fw) {
-      const int buf = k % NBUF;
-      int lo, nr;
-      chunk(k, fw, lo, nr);
-      for (int r0 = 0; r0 < G * R; r0 += 12) {     // 12 rows (60 lanes) at a time
-        const int rr = r0 + lane / 5, gg = rr / R, j = rr % R;
-        if (lane < 60 && rr < G * R && gg < cnt && j < nr)
-          parallel_part(bst[buf][gg][j], rec[buf][gg] + j * (fw ? 60 : 66), lane % 5, fw);
-      }
-    };
-    stream_pass<NBUF>(nchunk, wave - 1, [&](int k) { issue(k, true); }, [&](int k) { prep(k, true); });
-    stream_pass<NBUF>(nchunk, wave - 1, [&](int k) { issue(k, false); }, [&](int k) { prep(k, false); });
-    return;
-  }
-
-  // ---- compute wave: the recurrence on lanes 0..4 (lane m = component m)
-  // Row i is split into the part that needs the newest value,
-  //   y_i = a0_i + W2_i * y_{i-1}          (products summed as a tree)
-  // and the part formed one row ahead, off the critical path,
-  //   a0_i = c_i + W1_i * y_{i-2} (+ boundary-row blocks).
-  // Record rows are read from LDS two rows ahead of use into three rotating
-  // register sets (W2 parts and W1+c parts separately).  The newest two
-  // values live in yA/yB, broadcast to every lane, with roles alternating.
-  // The recurrence wave issues first on its SIMD: where it shares the SIMD
-  // with loader waves (two workgroups on a CU) they would split its issue
-  // slots (1-4% of the solve time).
-  __builtin_amdgcn_s_setprio(3);
-  cx<T> yA[5], yB[5];
-  cx<T> w2s[3][5], w1s[3][5], cs[3];
-  // rows kept for the boundary-row blocks: y_{n-5}, y_{n-4} (forward),
-  // x_3, x_4 (backward), as broadcast values
-  cx<T> s0[5], s1[5];
-  // the term in the newest value: two FMA accumulators (four independent
-  // chains over re and im), 22 instructions
-  auto crit = [&](const cx<T> (&w)[5], const cx<T> (&yn)[5], cx<T> a0) -> cx<T> {
-    cx<T> a = cfma(w[0], yn[0], a0), b = cmul(w[1], yn[1]);
-    a = cfma(w[2], yn[2], a);
-    b = cfma(w[3], yn[3], b);
-    a = cfma(w[4], yn[4], a);
-    return a + b;
-  };
-  auto pre0 = [&](const cx<T> (&w)[5], cx<T> c, const cx<T> (&yo)[5]) -> cx<T> {
-    cx<T> a = cfma(w[0], yo[0], c), b = cmul(w[1], yo[1]);
-    a = cfma(w[2], yo[2], a);
-    b = cfma(w[3], yo[3], b);
-    a = cfma(w[4], yo[4], a);
-    return a + b;
-  };
-  // blocks of the boundary rows outside the two-row band
-  auto bnd = [&](int i, bool fwd_pass) -> cx<T> {
-    cx<T> b{0, 0};
-    if (fwd_pass) {
-      if (i >= n - 2) {      // rows n-2, n-1: blocks in columns n-5, n-4
-        const cx<T> *Xa = tl + (i == n - 2 ? 0 : 25) + m * 5;
-#pragma unroll
-        for (int q = 0; q < 5; q++) b = cfma(Xa[q], s0[q], b);
-        if (i == n - 1)
-#pragma unroll
-          for (int q = 0; q < 5; q++) b = cfma(tl[50 + m * 5 + q], s1[q], b);
-      }
-    } else if (i <= 1) {     // rows 1, 0: blocks in columns 3, 4
-      const cx<T> *Qa = tl + (i == 1 ? 125 : 100) + m * 5;
-#pragma unroll
-      for (int q = 0; q < 5; q++) b = cfma(Qa[q], s1[q], b);
-      if (i == 0)
-#pragma unroll
-        for (int q = 0; q < 5; q++) b = cfma(tl[75 + m * 5 + q], s0[q], b);
-    }
-    return b;
-  };
-  auto keep = [&](const cx<T> (&y)[5], int i, bool fwd_pass) {
-    if (i == (fwd_pass ? n - 5 : 3))
-#pragma unroll
-      for (int q = 0; q < 5; q++) s0[q] = y[q];
-    if (i == (fwd_pass ? n - 4 : 4))
-#pragma unroll
-      for (int q = 0; q < 5; q++) s1[q] = y[q];
-  };
-  // one chunk: rows of buffer kk in processing order j = 0..nr-1 (row in
-  // the buffer = j forward, nr-1-j backward; grid row = ibase +/- j).  Rows
-  // are processed in branch-free groups of six; the remainder and the last
-  // five rows of a pass (which carry the boundary-row blocks) take a plain
-  // one-row-at-a-time path.
-  auto run_chunk = [&](const cx<T> *B, int stride, int kk, int nr, int ibase, bool fwd_pass) {
-    auto rix = [&](int j) { return fwd_pass ? j : nr - 1 - j; };     // j < nr at every call
-    auto gi = [&](int j) { return fwd_pass ? ibase + j : ibase - j; };
-    auto ldW2 = [&](int j, cx<T> (&w)[5]) {
-      const cx<T> *p = B + rix(j) * stride + m * 10;
-#pragma unroll
-      for (int q = 0; q < 5; q++) w[q] = p[q];
-    };
-    auto ldW1 = [&](int j, cx<T> (&w)[5], cx<T> &c) {
-      const int r = rix(j);
-      const cx<T> *p = B + r * stride + m * 10 + 5;
-#pragma unroll
-      for (int q = 0; q < 5; q++) w[q] = p[q];
-      c = *reinterpret_cast<const cx<T> *>(&bst[kk][g][r][m]);
-    };
-    int before_tail = fwd_pass ? n - 5 - ibase : ibase - 4;
-    before_tail = max(0, min(nr, before_tail));
-    const int nmain = (before_tail / 6) * 6;
-    double2 *xp = X + (long)gi(0) * rs + m;
-    const long xstep = fwd_pass ? rs : -rs;
-    if (nmain > 0) {
-      ldW2(0, w2s[0]);
-      ldW2(1, w2s[1]);
-      ldW1(0, w1s[0], cs[0]);
-      ldW1(1, w1s[1], cs[1]);
-      ldW1(2, w1s[2], cs[2]);
-      cx<T> a0 = pre0(w1s[0], cs[0], yA);
-      // rows two and three ahead are read only while they lie in this
-      // chunk's groups (the next chunk starts by reading its own first rows)
-      auto sub = [&](int j, bool more, auto U) {
-        constexpr int u = decltype(U)::value;
-        constexpr int u0 = u % 3, u1 = (u + 1) % 3, u2 = (u + 2) % 3;
-        cx<T>(&yn)[5] = (u % 2 == 0) ? yB : yA;      // newest value, y_{i-1}
-        cx<T>(&yd)[5] = (u % 2 == 0) ? yA : yB;      // receives y_i
-        cx<T> y = crit(w2s[u0], yn, a0);
-        a0 = pre0(w1s[u1], cs[u1], yn);
-        *xp = make_double2(y.re, y.im);    // lanes of one component store the same value
-        xp += xstep;
-        if (u + 2 < 6 || more) ldW2(j + 2, w2s[u2]);
-        if (u + 3 < 6 || more) ldW1(j + 3, w1s[u0], cs[u0]);
-        row_bcast5(y, yd);
-      };
-      for (int j = 0; j < nmain; j += 6) {
-        const bool more = j + 6 < nmain;
-        sub(j, more, std::integral_constant<int, 0>());
-        sub(j + 1, more, std::integral_constant<int, 1>());
-        sub(j + 2, more, std::integral_constant<int, 2>());
-        sub(j + 3, more, std::integral_constant<int, 3>());
-        sub(j + 4, more, std::integral_constant<int, 4>());
-        sub(j + 5, more, std::integral_constant<int, 5>());
-      }
-    }
-    for (int j = nmain; j < nr; j++) {
-      const int i = gi(j);
-      cx<T> w1[5], w2[5], c;
-      ldW1(j, w1, c);
-      ldW2(j, w2);
-      cx<T> y = crit(w2, yB, pre0(w1, c, yA) + bnd(i, fwd_pass));
-      *xp = make_double2(y.re, y.im);
-      xp += xstep;
-      row_bcast5(y, yA);                 // y_{i-2} is dead
-#pragma unroll
-      for (int q = 0; q < 5; q++) { cx<T> t = yA[q]; yA[q] = yB[q]; yB[q] = t; }
-      keep(yB, i, fwd_pass);
-    }
-  };
-
-  // forward: y_i = c_i + N1 y_{i-2} + N2 y_{i-1}; backward: x_i = d_i +
-  // Q4 x_{i+1} + Q5 x_{i+2}
-#pragma unroll
-  for (int q = 0; q < 5; q++) { yA[q] = cx<T>{0, 0}; yB[q] = cx<T>{0, 0}; }
-  compute_pass(nchunk, [&](int k) {
-    int lo, nr;
-    chunk(k, true, lo, nr);
-    run_chunk(rec[k % NBUF][g], 60, k % NBUF, nr, lo, true);
-  });
-#pragma unroll
-  for (int q = 0; q < 5; q++) { yA[q] = cx<T>{0, 0}; yB[q] = cx<T>{0, 0}; }
-  compute_pass(nchunk, [&](int k) {
-    int lo, nr;
-    chunk(k, false, lo, nr);
-    run_chunk(rec[k % NBUF][g], 66, k % NBUF, nr, lo + nr - 1, false);
-  });
-}
-
-template <typename T, int R, int G>
-__global__ __launch_bounds__(256) void k_solve_bc(int n, long L, const cx<T> *__restrict__ fwd,
-                                                 const cx<T> *__restrict__ bwd,
-                                                 const cx<T> *__restrict__ tail, double2 *rhs,
-                                                 long sL, long sR) {
-  solve_bc<T, R, G>(blockIdx.x, n, L, fwd, bwd, tail, rhs, sL, sR);
-}
-
-// ---------------------------------------------------------------------------
-// stage 3, twisted lines: the factor eliminated rows n-1..h+2 bottom-up and
-// then rows 0..h+1 top-down, so each line is two recurrences of about n/2
-// rows ("chains"): chain 0 runs rows 0..h+1, chain 1 rows n-1..h+2.  They
-// run in lockstep on two DPP rows of the compute wave (G lines per
-// workgroup, 2G chains).  Forward: chain 1 finishes first and hands its last
-// two values (rows h+2, h+3) to chain 0, whose last two rows carry those
-// columns.  Backward: chain 0 starts at row h+1; chain 1 starts two steps
-// later from chain 0's x_{h+1}, x_h.
-// HALF (one line per workgroup, single steps): the DPP rows that would
-// repeat the two chains instead take half of each row's columns (below).
-template <typename T, int R, int G, bool PAIRS, int NBUF, bool HALF>
-__device__ __forceinline__ void solve_tw(long bid, int n, int h, long L, const cx<T> *__restrict__ fwd,
-                                         const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ tail,
-                                         const cx<T> *__restrict__ xf, const cx<T> *__restrict__ xb,
-                                         double2 *rhs, long sL, long sR) {
-  constexpr int C = 2 * G;
-  constexpr int BUFE = R * 66;
-  static_assert(R % 6 == 0, "a chunk is whole groups of six rows");
-  static_assert(!HALF || (G == 1 && !PAIRS), "column halves: one line per workgroup, single steps");
-  __shared__ __attribute__((aligned(16))) cx<T> rec[NBUF][C][BUFE];
-  __shared__ double2 bst[NBUF][C][R][5];   // rhs rows, then c (or d) in place
-  constexpr int XE = PAIRS ? (R / 2) * 25 + 1 : 1;   // side blocks of a chunk's pairs (+1: copy padding)
-  __shared__ __attribute__((aligned(16))) cx<T> xtr[NBUF][C][XE];
-  __shared__ cx<T> xch[G][2][5];     // values handed between the chains of a line
-  __shared__ cx<T> kept[C][2][5];    // x at chain rows 3, 4 (backward boundary blocks)
-  // zero rows standing in for the staged c rows in the column half without c
-  __shared__ double2 zrows[HALF ? R : 1][5];
-  const long line0 = bid * G;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int ch = (lane >> 4) % C;    // chain of this DPP row (rows past 2G repeat)
-  const int g = ch >> 1, t = ch & 1;
-  const int m = min(lane & 15, 4);
-  const int hq = lane >> 5;          // column half (HALF): DPP rows 0, 1 and rows 2, 3
-  auto line_of = [&](int gg) { return min(line0 + gg, L - 1); };
-  const long line = line_of(g);
-  const int len0 = h + 2, len1 = n - h - 2;          // len0 >= len1 + 2
-  // chain tt (0 or 1) in arithmetic form: a select here becomes a per-lane
-  // table in scratch, whose loads would wait on the loaders' copies
-  auto clen = [&](int tt) { return len0 + tt * (len1 - len0); };
-  auto coff = [&](int tt) { return tt * len0; };
-  auto real_row = [&](int tt, int j) { return j + tt * (n - 1 - 2 * j); };
-  const int len = clen(t);
-  const long rs = sR * 5;
-  double2 *X = rhs + line * sL * 5;
-  const cx<T> *tl = tail + (line * 2 + t) * 150;
-  const int nchunk = (len0 + R - 1) / R;             // steps per pass: len0
-  const int npair = (len0 + 1) / 2;                  // pair slots per chain in xf / xb
-  // chain row at step s of the backward pass
-  auto bj = [&](int tt, int s) { return len0 - 1 - s + tt * (len1 + 2 - len0); };
-  // rows of chunk k held in the LDS buffer for chain tt: [jlo, jlo + nr)
-  auto chunk_rows = [&](int tt, int k, bool fw, int &jlo, int &nr) {
-    const int l = clen(tt);
-    if (fw) {
-      jlo = k * R;
-      nr = max(0, min(R, l - jlo));
-    } else {
-      int jhi = min(l - 1, bj(tt, k * R));
-      jlo = max(0, bj(tt, k * R + R - 1));
-      nr = max(0, jhi - jlo + 1);
-    }
-  };
-
-  if (wave != 0) {
-    // ---- loader waves ----
-    auto issue = [&](int k, bool fw) {
-      const int buf = k % NBUF;
-#pragma unroll
-      for (int cc = 0; cc < C; cc++) {
-        int jlo, nr;
-        chunk_rows(cc & 1, k, fw, jlo, nr);
-        const long r0 = line_of(cc >> 1) * n + coff(cc & 1) + jlo;
-        if (fw) dma_rows(fwd + r0 * 60, rec[buf][cc], nr * 60, lane);
-        else dma_rows(bwd + r0 * 66, rec[buf][cc], nr * 66, lane);
-      }
-      int p_end, m_end;
-      tw_pair_range(R, k, fw, len0, len1, p_end, m_end);
-      if (PAIRS && m_end > p_end) {
-        const int ne = (m_end - p_end) / 2 * 25;
-#pragma unroll
-        for (int cc = 0; cc < C; cc++)
-          dma_rows((fw ? xf : xb) + ((line_of(cc >> 1) * 2 + (cc & 1)) * npair + p_end / 2) * 25, xtr[buf][cc],
-                   (ne + 1) & ~1, lane);
-      }
-      double2 *dst = &bst[buf][0][0][0];
-#pragma unroll
-      for (int b = 0; b * 64 < C * R * 5; b++) {
-        const int e = b * 64 + lane, cc = e / (R * 5), j = (e / 5) % R, q = e % 5;
-        int jlo, nr;
-        chunk_rows(cc & 1, k, fw, jlo, nr);
-        if (e < C * R * 5 && j < nr)
-          __builtin_amdgcn_global_load_lds(
-              (const void *)(rhs + line_of(cc >> 1) * sL * 5 + (long)real_row(cc & 1, jlo + j) * rs + q),
-              (lds_void *)(dst + b * 64), 16, 0, 0);
-      }
-    };
-    auto prep = [&](int k, bool fw) {
-      const int buf = k % NBUF;
-      int p_end, m_end;
-      tw_pair_range(R, k, fw, len0, len1, p_end, m_end);
-      for (int r0 = 0; r0 < C * R; r0 += 12) {     // 12 rows (60 lanes) at a time (a chain's rows
-        const int rr = r0 + lane / 5, cc = rr / R, j = rr % R;   // never straddle two rounds)
-        int jlo, nr;
-        chunk_rows(cc & 1, k, fw, jlo, nr);
-        // the step of LDS row j, and whether it is the second of a pair
-        const int st = fw ? k * R + j : bj(cc & 1, 0) - (jlo + j);
-        const bool second = PAIRS && (st & 1) && st - 1 >= p_end && st < m_end;
-        const int jp = second ? (fw ? j - 1 : j + 1) : j;   // LDS row of step st - 1
-        if (lane < 60 && rr < C * R && j < nr) {
-          if constexpr (PAIRS)
-            parallel_part_x(bst[buf][cc][j], rec[buf][cc] + j * (fw ? 60 : 66),
-                            xtr[buf][cc] + (second ? (st - 1 - p_end) / 2 : 0) * 25, bst[buf][cc][jp], lane % 5,
-                            fw, second);
-          else
-            parallel_part(bst[buf][cc][j], rec[buf][cc] + j * (fw ? 60 : 66), lane % 5, fw);
-        }
-      }
-    };
-    stream_pass<NBUF>(nchunk, wave - 1, [&](int k) { issue(k, true); }, [&](int k) { prep(k, true); });
-    stream_pass<NBUF>(nchunk, wave - 1, [&](int k) { issue(k, false); }, [&](int k) { prep(k, false); });
-    return;
-  }
-
-  // ---- compute wave (same recurrence as k_solve_bc, per chain) ----
-  __builtin_amdgcn_s_setprio(3);   // as in solve_bc
-  cx<T> yA[5], yB[5];
-  cx<T> w2s[3][5], w1s[3][5], cs[3];
-  cx<T> s0[5], s1[5];
-  // HALF: the two newest values (lane m: component m), always current, and
-  // their split broadcasts, current while `split` holds
-  cx<T> vA{0, 0}, vB{0, 0}, SA[3], SB[3];
-  bool split = false;
-  if (HALF) {
-    for (int e = lane; e < R * 5; e += 64) zrows[e / 5][e % 5] = make_double2(0.0, 0.0);
-    wave_sync();
-  }
-  // split broadcast of v into S, in place: slot k = component 3 hq + k of
-  // the chain; slot 2 of the upper half is never written and holds zero
-  auto split_bcast = [&](cx<T> v, cx<T> (&S)[3]) {
-    S[0] = row_bcast_rows<3, 0xC>(row_bcast_rows<0, 0x3>(S[0], v), v);
-    S[1] = row_bcast_rows<4, 0xC>(row_bcast_rows<1, 0x3>(S[1], v), v);
-    S[2] = row_bcast_rows<2, 0x3>(S[2], v);
-  };
-  // the term in the newest value: two FMA accumulators (four independent
-  // chains over re and im), 22 instructions
-  auto crit = [&](const cx<T> (&w)[5], const cx<T> (&yn)[5], cx<T> a0) -> cx<T> {
-    cx<T> a = cfma(w[0], yn[0], a0), b = cmul(w[1], yn[1]);
-    a = cfma(w[2], yn[2], a);
-    b = cfma(w[3], yn[3], b);
-    a = cfma(w[4], yn[4], a);
-    return a + b;
-  };
-  auto pre0 = [&](const cx<T> (&w)[5], cx<T> c, const cx<T> (&yo)[5]) -> cx<T> {
-    cx<T> a = cfma(w[0], yo[0], c), b = cmul(w[1], yo[1]);
-    a = cfma(w[2], yo[2], a);
-    b = cfma(w[3], yo[3], b);
-    a = cfma(w[4], yo[4], a);
-    return a + b;
-  };
-  // one step of a pair: c + W2 yn + W1 yo, in four independent FMA chains
-  auto pair_eval = [&](const cx<T> (&w2)[5], const cx<T> (&w1)[5], cx<T> c, const cx<T> (&yn)[5],
-                       const cx<T> (&yo)[5]) -> cx<T> {
-    cx<T> a = cfma(w1[0], yo[0], c), b = cmul(w2[0], yn[0]);
-#pragma unroll
-    for (int q = 1; q < 5; q++) {
-      a = cfma(w1[q], yo[q], a);
-      b = cfma(w2[q], yn[q], b);
-    }
-    return a + b;
-  };
-  auto run_pass = [&](bool fw) {
-    const int stride = fw ? 60 : 66;
-#pragma unroll
-    for (int q = 0; q < 5; q++) { yA[q] = cx<T>{0, 0}; yB[q] = cx<T>{0, 0}; }
-    vA = vB = cx<T>{0, 0};
-    split = false;
-    compute_pass(nchunk, [&](int k) {
-      {
-        const int kk = k % NBUF;
-        const cx<T> *B = rec[kk][ch];
-        int jlo, nr;
-        chunk_rows(t, k, fw, jlo, nr);
-        const int s_begin = k * R, s_end = min(k * R + R, len0);
-        // buffer row of step s (clamped into the chunk's rows)
-        auto brow = [&](int s) {
-          int b = fw ? s - s_begin : bj(t, s) - jlo;
-          return max(0, min(max(nr, 1) - 1, b));
-        };
-        // the same inside the main range, where every step's row is in the
-        // buffer for both chains
-        auto brow_m = [&](int s) { return fw ? s - s_begin : bj(t, s) - jlo; };
-        auto ldW2 = [&](int s, cx<T> (&w)[5]) {
-          const cx<T> *pp = B + brow(s) * stride + m * 10;
-#pragma unroll
-          for (int q = 0; q < 5; q++) w[q] = pp[q];
-        };
-        auto ldW1 = [&](int s, cx<T> (&w)[5], cx<T> &c) {
-          const int r = brow(s);
-          const cx<T> *pp = B + r * stride + m * 10 + 5;
-#pragma unroll
-          for (int q = 0; q < 5; q++) w[q] = pp[q];
-          c = *reinterpret_cast<const cx<T> *>(&bst[kk][ch][r][m]);
-        };
-        auto jrow = [&](int s) { return fw ? s : bj(t, s); };
-        // one step on the plain path: hand-offs, boundary blocks, inactive chains
-        auto plain = [&](int s) {
-          const int j = jrow(s);
-          const bool act = j >= 0 && j < len;
-          if (HALF) {          // vA, vB are the state; yA, yB live only within a plain step
-            row_bcast5(vA, yA);
-            row_bcast5(vB, yB);
-            split = false;
-          }
-          if (!fw && t == 1 && s == 2) {            // chain 1 starts from x_h, x_{h+1}
-#pragma unroll
-            for (int q = 0; q < 5; q++) { yA[q] = xch[g][0][q]; yB[q] = xch[g][1][q]; }
-            if (HALF) { vA = xch[g][0][m]; vB = xch[g][1][m]; }
-          }
-          if (fw && t == 0 && j == len0 - 2) {      // columns h+2, h+3 from chain 1
-#pragma unroll
-            for (int q = 0; q < 5; q++) { s0[q] = xch[g][0][q]; s1[q] = xch[g][1][q]; }
-          }
-          if (!fw && j == 1) {
-#pragma unroll
-            for (int q = 0; q < 5; q++) { s0[q] = kept[ch][0][q]; s1[q] = kept[ch][1][q]; }
-          }
-          cx<T> w1[5], w2[5], c;
-          ldW1(s, w1, c);
-          ldW2(s, w2);
-          cx<T> b{0, 0};
-          if (fw) {
-            if (t == 0 && j >= len0 - 2) {
-              const cx<T> *Xa = tl + (j == len0 - 2 ? 0 : 25) + m * 5;
-#pragma unroll
-              for (int q = 0; q < 5; q++) b = cfma(Xa[q], s0[q], b);
-              if (j == len0 - 1)
-#pragma unroll
-                for (int q = 0; q < 5; q++) b = cfma(tl[50 + m * 5 + q], s1[q], b);
-            }
-          } else if (j >= 0 && j <= 1) {
-            const cx<T> *Qa = tl + (j == 1 ? 125 : 100) + m * 5;
-#pragma unroll
-            for (int q = 0; q < 5; q++) b = cfma(Qa[q], s1[q], b);
-            if (j == 0)
-#pragma unroll
-              for (int q = 0; q < 5; q++) b = cfma(tl[75 + m * 5 + q], s0[q], b);
-          }
-          cx<T> y = crit(w2, yB, pre0(w1, c, yA) + b);
-          if (act) X[(long)real_row(t, j) * rs + m] = make_double2(y.re, y.im);
-          row_bcast5(y, yA);
-#pragma unroll
-          for (int q = 0; q < 5; q++) { cx<T> tt = yA[q]; yA[q] = yB[q]; yB[q] = tt; }
-          if (HALF) { vA = vB; vB = y; }
-          if (act) {
-            if (fw && t == 1 && j == len1 - 1) xch[g][0][m] = y;     // z_{h+2}
-            if (fw && t == 1 && j == len1 - 2) xch[g][1][m] = y;     // z_{h+3}
-            if (!fw && t == 0 && j == len0 - 1) xch[g][1][m] = y;    // x_{h+1}
-            if (!fw && t == 0 && j == len0 - 2) xch[g][0][m] = y;    // x_h
-            if (!fw && (j == 3 || j == 4)) kept[ch][j - 3][m] = y;
-          }
-        };
-        int p_end, m_end;
-        tw_pair_range(R, k, fw, len0, len1, p_end, m_end);
-        for (int s = s_begin; s < p_end; s++) plain(s);
-        if (PAIRS && m_end > p_end) {
-          // pairs of steps (s, s+1): lanes 0-4 step s, lanes 5-9 step s+1
-          // (its record and parallel part rewritten for the pair), lanes
-          // 10-15 repeat lane 9; both from y_{s-2} (yA), y_{s-1} (yB).
-          // Coefficients two pairs ahead in three rotating register sets.
-          const int pl = min(lane & 15, 9), prow = pl >= 5 ? 1 : 0, pm = pl - 5 * prow;
-          auto ldP = [&](int st, cx<T> (&w2)[5], cx<T> (&w1)[5], cx<T> &c) {
-            const int r = brow(st + prow);
-            const cx<T> *pp = B + r * stride + pm * 10;
-#pragma unroll
-            for (int q = 0; q < 5; q++) { w2[q] = pp[q]; w1[q] = pp[5 + q]; }
-            c = *reinterpret_cast<const cx<T> *>(&bst[kk][ch][r][pm]);
-          };
-          const long xstep = ((t == 0) == fw) ? rs : -rs;
-          double2 *xq = X + (long)real_row(t, jrow(p_end + prow)) * rs + pm;
-          ldP(p_end, w2s[0], w1s[0], cs[0]);
-          ldP(p_end + 2, w2s[1], w1s[1], cs[1]);
-          auto psub = [&](int st, auto U) {
-            constexpr int u = decltype(U)::value, u2 = (u + 2) % 3;
-            const cx<T> y = pair_eval(w2s[u], w1s[u], cs[u], yB, yA);
-            *xq = make_double2(y.re, y.im);
-            xq += 2 * xstep;
-            ldP(st + 4, w2s[u2], w1s[u2], cs[u2]);
-            row_bcast5_at<0>(y, yA);
-            row_bcast5_at<5>(y, yB);
-          };
-          for (int st = p_end; st < m_end; st += 6) {
-            psub(st, std::integral_constant<int, 0>());
-            psub(st + 2, std::integral_constant<int, 1>());
-            psub(st + 4, std::integral_constant<int, 2>());
-          }
-        }
-        if (HALF && m_end > p_end) {
-          // Columns split over the wave's halves: half hq of a chain sums
-          // columns 3 hq + k (k = 0, 1, 2) of each block row, slot 2 of the
-          // upper half meeting a zero broadcast; the upper half adds c.  The
-          // halves' partial rows are added across the wave (half_sum), so both
-          // halves hold y and broadcast it.  Steps two and three ahead are
-          // read only while they lie in the main range.
-          if (!split) {
-            SA[2] = SB[2] = cx<T>{0, 0};
-            split_bcast(vA, SA);
-            split_bcast(vB, SB);
-            split = true;
-          }
-          const int qb = 3 * hq;
-          const double2 *cb = hq ? &bst[kk][ch][0][m] : &zrows[0][m];   // row r: cb + 5 r
-          auto ldW2h = [&](int s, cx<T> (&w)[3]) {
-            const cx<T> *pp = B + brow_m(s) * stride + m * 10 + qb;
-#pragma unroll
-            for (int k = 0; k < 3; k++) w[k] = pp[k];
-          };
-          auto ldW1h = [&](int s, cx<T> (&w)[3], cx<T> &c) {
-            const int r = brow_m(s);
-            const cx<T> *pp = B + r * stride + m * 10 + 5 + qb;
-#pragma unroll
-            for (int k = 0; k < 3; k++) w[k] = pp[k];
-            c = *reinterpret_cast<const cx<T> *>(cb + 5 * r);
-          };
-          // a + b: the half's part of c + W1 y_{i-2}, formed a step ahead
-          auto pre0h = [&](const cx<T> (&w)[3], cx<T> c, const cx<T> (&S)[3], cx<T> &a, cx<T> &b) {
-            a = cfma(w[0], S[0], c);
-            b = cmul(w[1], S[1]);
-            a = cfma(w[2], S[2], a);
-          };
-          auto crith = [&](const cx<T> (&w)[3], const cx<T> (&S)[3], cx<T> a, cx<T> b) -> cx<T> {
-            a = cfma(w[0], S[0], a);
-            b = cfma(w[1], S[1], b);
-            a = cfma(w[2], S[2], a);
-            return half_sum(a + b);
-          };
-          cx<T> w2h[3][3], w1h[3][3], chh[3];
-          double2 *xp = X + (long)real_row(t, jrow(p_end)) * rs + m;
-          const long xstep = ((t == 0) == fw) ? rs : -rs;
-          ldW2h(p_end, w2h[0]);
-          ldW2h(p_end + 1, w2h[1]);
-          ldW1h(p_end, w1h[0], chh[0]);
-          ldW1h(p_end + 1, w1h[1], chh[1]);
-          ldW1h(p_end + 2, w1h[2], chh[2]);
-          cx<T> pa, pb;
-          pre0h(w1h[0], chh[0], SA, pa, pb);
-          auto subh = [&](int s, bool more, auto U) {
-            constexpr int u = decltype(U)::value;
-            constexpr int u0 = u % 3, u1 = (u + 1) % 3, u2 = (u + 2) % 3;
-            cx<T>(&Sn)[3] = (u % 2 == 0) ? SB : SA;      // y_{i-1}
-            cx<T>(&Sd)[3] = (u % 2 == 0) ? SA : SB;      // receives y_i
-            const cx<T> y = crith(w2h[u0], Sn, pa, pb);
-            pre0h(w1h[u1], chh[u1], Sn, pa, pb);
-            *xp = make_double2(y.re, y.im);
-            xp += xstep;
-            if (u + 2 < 6 || more) ldW2h(s + 2, w2h[u2]);
-            if (u + 3 < 6 || more) ldW1h(s + 3, w1h[u0], chh[u0]);
-            split_bcast(y, Sd);
-            if constexpr (u == 4) vA = y;
-            if constexpr (u == 5) vB = y;
-          };
-          for (int s = p_end; s < m_end; s += 6) {
-            const bool more = s + 6 < m_end;
-            subh(s, more, std::integral_constant<int, 0>());
-            subh(s + 1, more, std::integral_constant<int, 1>());
-            subh(s + 2, more, std::integral_constant<int, 2>());
-            subh(s + 3, more, std::integral_constant<int, 3>());
-            subh(s + 4, more, std::integral_constant<int, 4>());
-            subh(s + 5, more, std::integral_constant<int, 5>());
-          }
-        }
-        if (!PAIRS && !HALF && m_end > p_end) {
-          // one step at a time in groups of six (no pair rewrite); steps two
-          // and three ahead are read only while they lie in the main range
-          auto ldW2m = [&](int s, cx<T> (&w)[5]) {
-            const cx<T> *pp = B + brow_m(s) * stride + m * 10;
-#pragma unroll
-            for (int q = 0; q < 5; q++) w[q] = pp[q];
-          };
-          auto ldW1m = [&](int s, cx<T> (&w)[5], cx<T> &c) {
-            const int r = brow_m(s);
-            const cx<T> *pp = B + r * stride + m * 10 + 5;
-#pragma unroll
-            for (int q = 0; q < 5; q++) w[q] = pp[q];
-            c = *reinterpret_cast<const cx<T> *>(&bst[kk][ch][r][m]);
-          };
-          int j0 = jrow(p_end);
-          double2 *xp = X + (long)real_row(t, j0) * rs + m;
-          const long xstep = ((t == 0) == fw) ? rs : -rs;
-          ldW2m(p_end, w2s[0]);
-          ldW2m(p_end + 1, w2s[1]);
-          ldW1m(p_end, w1s[0], cs[0]);
-          ldW1m(p_end + 1, w1s[1], cs[1]);
-          ldW1m(p_end + 2, w1s[2], cs[2]);
-          cx<T> a0 = pre0(w1s[0], cs[0], yA);
-          auto sub = [&](int s, bool more, auto U) {
-            constexpr int u = decltype(U)::value;
-            constexpr int u0 = u % 3, u1 = (u + 1) % 3, u2 = (u + 2) % 3;
-            cx<T>(&yn)[5] = (u % 2 == 0) ? yB : yA;
-            cx<T>(&yd)[5] = (u % 2 == 0) ? yA : yB;
-            cx<T> y = crit(w2s[u0], yn, a0);
-            a0 = pre0(w1s[u1], cs[u1], yn);
-            *xp = make_double2(y.re, y.im);
-            xp += xstep;
-            if (u + 2 < 6 || more) ldW2m(s + 2, w2s[u2]);
-            if (u + 3 < 6 || more) ldW1m(s + 3, w1s[u0], cs[u0]);
-            row_bcast5(y, yd);
-          };
-          for (int s = p_end; s < m_end; s += 6) {
-            const bool more = s + 6 < m_end;
-            sub(s, more, std::integral_constant<int, 0>());
-            sub(s + 1, more, std::integral_constant<int, 1>());
-            sub(s + 2, more, std::integral_constant<int, 2>());
-            sub(s + 3, more, std::integral_constant<int, 3>());
-            sub(s + 4, more, std::integral_constant<int, 4>());
-            sub(s + 5, more, std::integral_constant<int, 5>());
-          }
-        }
-        for (int s = m_end; s < s_end; s++) plain(s);
-      }
-    });
-  };
-  run_pass(true);
-  run_pass(false);
-}
-
-template <typename T, int R, int G, bool PAIRS, int NBUF, bool HALF = false>
-__global__ __launch_bounds__(256, 2) void k_solve_tw(int n, int h, long L, const cx<T> *__restrict__ fwd,
-                                                 const cx<T> *__restrict__ bwd,
-                                                 const cx<T> *__restrict__ tail,
-                                                 const cx<T> *__restrict__ xf,
-                                                 const cx<T> *__restrict__ xb, double2 *rhs,
-                                                 long sL, long sR) {
-  solve_tw<T, R, G, PAIRS, NBUF, HALF>(blockIdx.x, n, h, L, fwd, bwd, tail, xf, xb, rhs, sL, sR);
 }
 
 // ---------------------------------------------------------------------------
@@ -2046,6 +1215,7 @@ __global__ void k_zero_i32(int *x, long n) {
 
 // ---------------------------------------------------------------------------
 // host side
+constexpr unsigned LDS_PER_CU = 160 * 1024;
 static int grid_for(long n, int b) { return (int)((n + b - 1) / b); }
 
 static int check_launch_grid(long total) { return (int)std::min<long>(grid_for(total, 256), 4096); }
@@ -2112,14 +1282,20 @@ int penta_check_result(PentaPlan *pl, hipStream_t s, long *bad_lines, long *firs
 static std::mutex g_tune_mu;
 static std::map<std::tuple<int, long, int>, int> g_tuned;
 
-int penta_variant_for(int n, long lines, int prec) {
+// Twisted lines (two chains per line, one line per workgroup) up to 512
+// lines: below that the chain's length is what a solve takes.  Above, plain
+// lines (two per workgroup) where the caller may ask for the reference's
+// substitution order, which needs factors in row order; else twisted lines
+// from 160 rows on.  Measured, plain / twisted us: 513 lines of 257 rows
+// 73 / 63, 1025 of 257 133 / 120, 1025 of 129 62 / 69, 1025 of 65 33 / 40.
+int penta_variant_for(int n, long lines, int prec, bool row_order) {
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(std::make_tuple(n, lines, prec));
     if (it != g_tuned.end()) return it->second;
   }
-  if (n >= 16 && lines < 512) return prec ? PENTA_TWISTED_PAIRS : PENTA_TWISTED_HALF;
-  return lines >= 512 ? PENTA_PLAIN3 : PENTA_PLAIN1;
+  const bool tw = n >= 16 && (lines < 512 || (!row_order && n >= 160));
+  return tw ? PENTA_TWISTED : PENTA_PLAIN1;
 }
 
 int penta_tune_set(int n, long lines, int prec, int variant) {
@@ -2131,10 +1307,10 @@ int penta_tune_set(int n, long lines, int prec, int variant) {
   return 0;
 }
 
-int penta_plan_create(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec) {
+int penta_plan_create(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec, bool row_order) {
   const int n = periodic ? n_rows - 1 : n_rows;
   return penta_plan_create_variant(pl, periodic, exact, n_rows, lines, prec,
-                                   periodic ? PENTA_PLAIN1 : penta_variant_for(n, lines, prec));
+                                   periodic ? PENTA_PLAIN1 : penta_variant_for(n, lines, prec, row_order));
 }
 
 int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec,
@@ -2152,7 +1328,7 @@ int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows
   size_t ne = (size_t)pl->np * 125 * lines;
   LNS3D_CHECK(hipMalloc(&pl->lu, ne * sizeof(cx<double>)));
   pl->per = pl->per2 = nullptr;
-  pl->fwd = pl->bwd = pl->tail = pl->mid = pl->p2 = pl->qp = pl->xf = pl->xb = pl->flags = nullptr;
+  pl->fwd = pl->bwd = pl->tail = pl->mid = pl->p2 = pl->qp = pl->flags = nullptr;
   if (periodic) {
     // complex-float plans take their records from a complex-double plan
     // (penta_records_narrow): no bordered LU of their own
@@ -2171,13 +1347,6 @@ int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows
     LNS3D_CHECK(hipMalloc(&pl->bwd, (size_t)pl->n * 66 * lines * es));
     LNS3D_CHECK(hipMalloc(&pl->tail, (size_t)150 * lines * (pl->h >= 0 ? 2 : 1) * es));
     if (pl->h >= 0) LNS3D_CHECK(hipMalloc(&pl->mid, (size_t)100 * lines * sizeof(cx<double>)));
-    if (pl->variant == PENTA_TWISTED_PAIRS) {
-      // 25 per (line, chain, pair), plus one complex past the end (a copy of
-      // an odd count of complex float moves 16 B at a time)
-      const size_t nx = ((size_t)lines * 2 * ((pl->h + 3) / 2) * 25 + 2) * es;
-      LNS3D_CHECK(hipMalloc(&pl->xf, nx));
-      LNS3D_CHECK(hipMalloc(&pl->xb, nx));
-    }
   }
   return 0;
 }
@@ -2192,11 +1361,9 @@ void penta_plan_destroy(PentaPlan *pl) {
   if (pl->mid) (void)hipFree(pl->mid);
   if (pl->p2) (void)hipFree(pl->p2);
   if (pl->qp) (void)hipFree(pl->qp);
-  if (pl->xf) (void)hipFree(pl->xf);
-  if (pl->xb) (void)hipFree(pl->xb);
   if (pl->flags) (void)hipFree(pl->flags);
   pl->lu = pl->per = pl->per2 = pl->fwd = pl->bwd = pl->tail = pl->mid = pl->p2 = pl->qp = nullptr;
-  pl->xf = pl->xb = pl->flags = nullptr;
+  pl->flags = nullptr;
 }
 
 int penta_import(PentaPlan *pl, const void *ref_mat, long sLm, long sRm, hipStream_t s) {
@@ -2221,18 +1388,6 @@ int penta_factor_records_only(PentaPlan *pl, hipStream_t s) {
                        (const cx<double> *)pl->lu, (cx<double> *)pl->fwd, (cx<double> *)pl->bwd,
                        (cx<double> *)pl->tail);
   LNS3D_CHECK(hipGetLastError());
-  if (pl->variant == PENTA_TWISTED_PAIRS) {   // the pair rewrite for the solve's chunk size
-    const long groups = pl->L * 4 * ((pl->h + 3) / 2);
-    if (pl->prec)
-      hipLaunchKernelGGL((k_pair_records<float>), dim3(grid_for(groups, 8)), dim3(256), 0, s, pl->n, pl->h, pl->L,
-                         tw_chunk(true), (cx<float> *)pl->fwd, (cx<float> *)pl->bwd, (cx<float> *)pl->xf,
-                         (cx<float> *)pl->xb);
-    else
-      hipLaunchKernelGGL((k_pair_records<double>), dim3(grid_for(groups, 8)), dim3(256), 0, s, pl->n, pl->h, pl->L,
-                         tw_chunk(false), (cx<double> *)pl->fwd, (cx<double> *)pl->bwd, (cx<double> *)pl->xf,
-                         (cx<double> *)pl->xb);
-    LNS3D_CHECK(hipGetLastError());
-  }
   return 0;
 }
 
@@ -2278,48 +1433,92 @@ int penta_factor(PentaPlan *pl, hipStream_t s) {
   return penta_factor_records_only(pl, s);
 }
 
-// non-periodic solve kernels by variant.  Chunks of R rows, four LDS
-// buffers: twisted lines and one line per workgroup use longer chunks (one
-// workgroup per line holds more rows); two, three or four lines per
-// workgroup take chunks of six rows so that two or more workgroups fit a CU.
-template <typename T>
-static void launch_solve_bc(const PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
-  constexpr bool D = sizeof(T) == 8;
-  const auto *f = (const cx<T> *)pl->fwd;
-  const auto *b = (const cx<T> *)pl->bwd;
-  const auto *t = (const cx<T> *)pl->tail;
-  auto *x = (double2 *)rhs;
-  auto wgs = [&](int G) { return dim3((unsigned)((pl->L + G - 1) / G)); };
-  switch (pl->variant) {
-    // twisted lines, a ring of four buffers (five measured slower: the wave
-    // preparing a chunk then also starts the next copies).  The kernel is
-    // bounded to 256 VGPRs per wave: above that only one workgroup fits a CU,
-    // and the 257th line of a 257-line solve would run alone after the rest.
-    case PENTA_TWISTED:        // one step at a time
-      hipLaunchKernelGGL((k_solve_tw<T, D ? 6 : 12, 1, false, 4>), wgs(1), dim3(256), 0, s, pl->n, pl->h, pl->L, f,
-                         b, t, (const cx<T> *)pl->xf, (const cx<T> *)pl->xb, x, sL, sR);
-      break;
-    case PENTA_TWISTED_HALF:   // one step at a time, columns split over the wave's halves
-      hipLaunchKernelGGL((k_solve_tw<T, D ? 6 : 12, 1, false, 4, true>), wgs(1), dim3(256), 0, s, pl->n, pl->h,
-                         pl->L, f, b, t, (const cx<T> *)pl->xf, (const cx<T> *)pl->xb, x, sL, sR);
-      break;
-    case PENTA_TWISTED_PAIRS:  // pairs of steps (factor-time rewrite)
-      static_assert(tw_chunk(!D) == (D ? 6 : 12), "the pair rewrite assumes the solve's chunk size");
-      hipLaunchKernelGGL((k_solve_tw<T, D ? 6 : 12, 1, true, 4>), wgs(1), dim3(256), 0, s, pl->n, pl->h, pl->L, f, b,
-                         t, (const cx<T> *)pl->xf, (const cx<T> *)pl->xb, x, sL, sR);
-      break;
-    case PENTA_PLAIN2:
-      hipLaunchKernelGGL((k_solve_bc<T, D ? 6 : 12, 2>), wgs(2), dim3(256), 0, s, pl->n, pl->L, f, b, t, x, sL, sR);
-      break;
-    case PENTA_PLAIN3:
-      hipLaunchKernelGGL((k_solve_bc<T, 6, 3>), wgs(3), dim3(256), 0, s, pl->n, pl->L, f, b, t, x, sL, sR);
-      break;
-    case PENTA_PLAIN4:
-      hipLaunchKernelGGL((k_solve_bc<T, 6, 4>), wgs(4), dim3(256), 0, s, pl->n, pl->L, f, b, t, x, sL, sR);
-      break;
-    default:
-      hipLaunchKernelGGL((k_solve_bc<T, D ? 12 : 24, 1>), wgs(1), dim3(256), 0, s, pl->n, pl->L, f, b, t, x, sL, sR);
+// Forms of the line solve: rows of a chunk and buffers of its ring, and
+// whether the right-hand sides stay in LDS.  Resident right-hand sides spare
+// the forward result's way to memory and back (160 of 2320 B per row); longer
+// chunks spare barriers (complex float, whose chunks are half the bytes);
+// small rings let more workgroups share a CU.
+enum { LINES_RES6, LINES_RING6, LINES_RES3, LINES_RING3, LINES_RES12, LINES_RING12 };
+template <int R_, int NBUF_, bool RES_> struct LineForm {
+  static constexpr int R = R_, NBUF = NBUF_;
+  static constexpr bool RES = RES_;
+};
+// f(T{}, LineForm, TW) with the types of a form
+template <typename F> static auto with_line_form(int form, int prec, bool tw, F f) {
+  auto fam = [&](auto t, auto lf) {
+    return tw ? f(t, lf, std::true_type()) : f(t, lf, std::false_type());
+  };
+  switch (form) {
+    case LINES_RES6: return prec ? fam(float{}, LineForm<6, 4, true>()) : fam(double{}, LineForm<6, 4, true>());
+    case LINES_RES3: return fam(double{}, LineForm<3, 4, true>());
+    case LINES_RING3: return fam(double{}, LineForm<3, 5, false>());
+    case LINES_RES12: return fam(float{}, LineForm<12, 4, true>());
+    case LINES_RING12: return fam(float{}, LineForm<12, 4, false>());
+    default: return prec ? fam(float{}, LineForm<6, 4, false>()) : fam(double{}, LineForm<6, 4, false>());
   }
+}
+static unsigned line_lds(int form, int prec, bool tw, int n) {
+  return with_line_form(form, prec, tw, [&](auto t, auto lf, auto TW) {
+    return LineSolve<decltype(t), lf.R, lf.NBUF, TW.value, lf.RES>::lds_bytes(n);
+  });
+}
+
+// The form for `lines` lines of n rows solved by one launch.  What matters is
+// how many workgroups share a CU (256 CUs, LDS_PER_CU of LDS each): while all
+// lines run at once a solve takes as long as its chain, so one or two per CU
+// take the form with the shortest step; more lines stream at the memory's
+// rate and take the form that moves least.  Measured at lines x rows, us
+// (complex double unless said):
+//   twisted  RES6 / RING6: 65x129 19 / 20, 127x384 43 / 44, 256x1025 117 / 124,
+//            257x257 36 / 37; 1025 lines of 257: RES6 120, RES3 126, RING3 132;
+//            513 of 257: RES3 63, RES6 75; 700 of 600: RING3 189, RING6 207
+//   plain    1025 of 65: RES3 33, RES6 41; 513 of 257: RING6 73, RING3 79;
+//            1025 of 257: RING3 133, RING6 151
+//   complex float, twisted: 257x1025 RING12 85, RING6 101; 127x384 RES12 35,
+//            RES6 41; 1025 of 257: RES6 74, RING6 83; 33x65 RES6 11.6, RES12 12.7
+static int line_form(int variant, int n, long lines, int prec, bool tw) {
+  // workgroups of a form that a CU holds
+  auto fit = [&](int form) { return (int)(LDS_PER_CU / line_lds(form, prec, tw, n)); };
+  const long wg = tw ? lines : (lines + 1) / 2;
+  const int need = wg <= 256 ? 1 : wg <= 512 ? 2 : 3;      // to run all at once, up to three
+  // variants that pin a form
+  const int small = prec ? (fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING6) : (fit(LINES_RES3) >= 3 ? LINES_RES3 : LINES_RING3);
+  switch (variant) {
+    case PENTA_PLAIN2: case PENTA_TWISTED_PAIRS: return LINES_RING6;
+    case PENTA_PLAIN3: case PENTA_TWISTED_HALF: return small;
+    case PENTA_PLAIN4: return prec ? LINES_RING12 : LINES_RING3;
+    default: break;
+  }
+  if (need < 3) {
+    if (prec && n >= 96) return fit(LINES_RES12) >= need ? LINES_RES12 : LINES_RING12;
+    return fit(LINES_RES6) >= need ? LINES_RES6 : LINES_RING6;
+  }
+  if (prec) return fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING6;
+  if (fit(LINES_RES3) >= 3 && (!tw || n < 128 || wg <= 768)) return LINES_RES3;
+  return tw && fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING3;
+}
+
+// a kernel's dynamic LDS above the default 64 KB has to be asked for
+template <typename K> static int allow_lds(K k, unsigned lds) {
+  if (lds > 64 * 1024)
+    LNS3D_CHECK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_PER_CU));
+  return 0;
+}
+
+static int launch_line_solve(const PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
+  const bool tw = pl->h >= 0;
+  const int form = line_form(pl->variant, pl->n, pl->L, pl->prec, tw);
+  return with_line_form(form, pl->prec, tw, [&](auto t, auto lf, auto TW) {
+    using T = decltype(t);
+    auto k = k_line_solve<T, lf.R, lf.NBUF, TW.value, lf.RES>;
+    const unsigned lds = line_lds(form, pl->prec, tw, pl->n);
+    const int rc = allow_lds(k, lds);
+    if (rc) return rc;
+    const long wg = tw ? pl->L : (pl->L + 1) / 2;
+    hipLaunchKernelGGL(k, dim3((unsigned)wg), dim3(256), lds, s, pl->n, pl->h, pl->L,
+                       (const cx<T> *)pl->fwd, (const cx<T> *)pl->bwd, (const cx<T> *)pl->tail, (double2 *)rhs, sL, sR);
+    return 0;
+  });
 }
 
 int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
@@ -2341,8 +1540,8 @@ int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
     if (pl->prec) per(float{});
     else per(double{});
   } else {
-    if (pl->prec) launch_solve_bc<float>(pl, rhs, sL, sR, s);
-    else launch_solve_bc<double>(pl, rhs, sL, sR, s);
+    const int rc = launch_line_solve(pl, rhs, sL, sR, s);
+    if (rc) return rc;
   }
   LNS3D_CHECK(hipGetLastError());
   return 0;
@@ -2363,23 +1562,14 @@ __device__ __forceinline__ int batch_member(const int *off, int count) {
   return lo;
 }
 
-template <typename T, int R, int G>
-__global__ __launch_bounds__(256) void kb_solve_bc(const PentaBatchItem *items, const int *off, int count,
-                                                  int which) {
+template <typename T, int R, int NBUF, bool TW, bool RES>
+__global__ __launch_bounds__(256, 2) void kb_line_solve(const PentaBatchItem *items, const int *off, int count,
+                                                       int which) {
+  extern __shared__ __attribute__((aligned(16))) char sm[];
   const int k = batch_member(off, count);
   const PentaBatchItem &b = items[k];
-  solve_bc<T, R, G>((long)blockIdx.x - off[k], b.n, b.L, (const cx<T> *)b.fwd, (const cx<T> *)b.bwd,
-                    (const cx<T> *)b.tail, b.rhs[which], b.sL, b.sR);
-}
-
-template <typename T, int R, int G, bool PAIRS, int NBUF, bool HALF = false>
-__global__ __launch_bounds__(256, 2) void kb_solve_tw(const PentaBatchItem *items, const int *off, int count,
-                                                     int which) {
-  const int k = batch_member(off, count);
-  const PentaBatchItem &b = items[k];
-  solve_tw<T, R, G, PAIRS, NBUF, HALF>((long)blockIdx.x - off[k], b.n, b.h, b.L, (const cx<T> *)b.fwd,
-                                       (const cx<T> *)b.bwd, (const cx<T> *)b.tail, (const cx<T> *)b.xf,
-                                       (const cx<T> *)b.xb, b.rhs[which], b.sL, b.sR);
+  LineSolve<T, R, NBUF, TW, RES>::run(sm, (long)blockIdx.x - off[k], b.n, b.h, b.L, (const cx<T> *)b.fwd,
+                                      (const cx<T> *)b.bwd, (const cx<T> *)b.tail, b.rhs[which], b.sL, b.sR);
 }
 
 template <typename T, int R, int G>
@@ -2396,9 +1586,7 @@ __global__ __launch_bounds__(256) void kb_solve_per(const PentaBatchItem *items,
 constexpr int BATCH_PERIODIC1 = 1001, BATCH_PERIODIC4 = 1004;
 
 // lines per workgroup of a batch group's solve kernel
-static int variant_lines(int v) {
-  return v == PENTA_PLAIN2 ? 2 : v == PENTA_PLAIN3 ? 3 : (v == PENTA_PLAIN4 || v == BATCH_PERIODIC4) ? 4 : 1;
-}
+static int group_lines(const PentaBatchGroup &g) { return g.form < 0 ? (g.variant == BATCH_PERIODIC4 ? 4 : 1) : g.tw ? 1 : 2; }
 
 int stage_upload(void *dev, const void *src, size_t bytes, std::vector<TableUpload> &ups) {
   void *h = nullptr;
@@ -2412,11 +1600,16 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
                       const long *sR, int count, std::vector<PentaBatchGroup> &out,
                       std::vector<TableUpload> &ups) {
   out.clear();
-  std::map<std::pair<int, int>, std::vector<int>> by;   // (variant, precision) -> members
+  long lines = 0;              // solved by one launch or another at a time
+  for (int k = 0; k < count; k++) lines += plans[k]->L;
+  // members that share a kernel: periodic lines by their kernel, the others
+  // by form and family (form -1: periodic)
+  std::map<std::tuple<int, int, int, int>, std::vector<int>> by;   // (form, variant of periodic lines, twisted, precision)
   for (int k = 0; k < count; k++) {
     const PentaPlan *pl = plans[k];
-    const int v = pl->periodic ? (pl->L > 512 ? BATCH_PERIODIC4 : BATCH_PERIODIC1) : pl->variant;
-    by[{v, pl->prec}].push_back(k);
+    const bool tw = pl->h >= 0;
+    if (pl->periodic) by[{-1, pl->L > 512 ? BATCH_PERIODIC4 : BATCH_PERIODIC1, 0, pl->prec}].push_back(k);
+    else by[{line_form(pl->variant, pl->n, lines, pl->prec, tw), 0, tw, pl->prec}].push_back(k);
   }
   for (auto &kv : by) {
     // longest lines first: their workgroups start in the first wave and the
@@ -2424,8 +1617,10 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
     std::stable_sort(kv.second.begin(), kv.second.end(),
                      [&](int a, int b) { return plans[a]->n > plans[b]->n; });
     PentaBatchGroup g;
-    g.variant = kv.first.first;
-    g.prec = kv.first.second;
+    g.form = std::get<0>(kv.first);
+    g.variant = std::get<1>(kv.first);
+    g.tw = std::get<2>(kv.first);
+    g.prec = std::get<3>(kv.first);
     g.count = (int)kv.second.size();
     std::vector<PentaBatchItem> items;
     std::vector<int> off(1, 0);
@@ -2438,8 +1633,6 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
       it.fwd = pl->fwd;
       it.bwd = pl->bwd;
       it.tail = pl->tail;
-      it.xf = pl->xf;
-      it.xb = pl->xb;
       it.p2 = pl->p2;
       it.qp = pl->qp;
       it.rhs[0] = rhs0[k];
@@ -2447,7 +1640,8 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
       it.sL = sL[k];
       it.sR = sR[k];
       items.push_back(it);
-      const long wg = (pl->L + variant_lines(g.variant) - 1) / variant_lines(g.variant);
+      const long wg = (pl->L + group_lines(g) - 1) / group_lines(g);
+      if (g.form >= 0) g.lds = std::max(g.lds, line_lds(g.form, g.prec, g.tw, pl->n));
       if ((long)off.back() + wg > 0x7fffffffL) return set_error(__FILE__, __LINE__, "batch too large");
       off.push_back(off.back() + (int)wg);
     }
@@ -2470,46 +1664,33 @@ void penta_batch_free(std::vector<PentaBatchGroup> &groups) {
   groups.clear();
 }
 
-template <typename T>
-static void launch_batch_group(const PentaBatchGroup &g, int which, hipStream_t s) {
-  constexpr bool D = sizeof(T) == 8;
+static int launch_batch_group(const PentaBatchGroup &g, int which, hipStream_t s) {
   const auto *it = (const PentaBatchItem *)g.items;
   const dim3 grid((unsigned)g.blocks), blk(256);
-  switch (g.variant) {
-    case PENTA_TWISTED:
-      hipLaunchKernelGGL((kb_solve_tw<T, D ? 6 : 12, 1, false, 4>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    case PENTA_TWISTED_HALF:
-      hipLaunchKernelGGL((kb_solve_tw<T, D ? 6 : 12, 1, false, 4, true>), grid, blk, 0, s, it, g.off, g.count,
-                         which);
-      break;
-    case PENTA_TWISTED_PAIRS:
-      hipLaunchKernelGGL((kb_solve_tw<T, D ? 6 : 12, 1, true, 4>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    case PENTA_PLAIN2:
-      hipLaunchKernelGGL((kb_solve_bc<T, D ? 6 : 12, 2>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    case PENTA_PLAIN3:
-      hipLaunchKernelGGL((kb_solve_bc<T, 6, 3>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    case PENTA_PLAIN4:
-      hipLaunchKernelGGL((kb_solve_bc<T, 6, 4>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    case BATCH_PERIODIC1:
-      hipLaunchKernelGGL((kb_solve_per<T, 30, 1>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    case BATCH_PERIODIC4:
+  if (g.form >= 0)
+    return with_line_form(g.form, g.prec, g.tw, [&](auto t, auto lf, auto TW) {
+      auto k = kb_line_solve<decltype(t), lf.R, lf.NBUF, TW.value, lf.RES>;
+      const int rc = allow_lds(k, g.lds);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k, grid, blk, g.lds, s, it, g.off, g.count, which);
+      return 0;
+    });
+  auto per = [&](auto t) {
+    using T = decltype(t);
+    if (g.variant == BATCH_PERIODIC4)
       hipLaunchKernelGGL((kb_solve_per<T, 6, 4>), grid, blk, 0, s, it, g.off, g.count, which);
-      break;
-    default:
-      hipLaunchKernelGGL((kb_solve_bc<T, D ? 12 : 24, 1>), grid, blk, 0, s, it, g.off, g.count, which);
-  }
+    else
+      hipLaunchKernelGGL((kb_solve_per<T, 30, 1>), grid, blk, 0, s, it, g.off, g.count, which);
+  };
+  if (g.prec) per(float{});
+  else per(double{});
+  return 0;
 }
 
 int penta_batch_solve(const std::vector<PentaBatchGroup> &groups, int which, hipStream_t s) {
   for (const auto &g : groups) {
-    if (g.prec) launch_batch_group<float>(g, which, s);
-    else launch_batch_group<double>(g, which, s);
+    const int rc = launch_batch_group(g, which, s);
+    if (rc) return rc;
     LNS3D_CHECK(hipGetLastError());
   }
   return 0;

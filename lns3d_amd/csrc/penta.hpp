@@ -33,8 +33,6 @@ struct PentaPlan {
   void *fwd = nullptr, *bwd = nullptr, *tail = nullptr;
   void *mid = nullptr;   // twisted factor: the bottom chain's share of the middle block
   void *p2 = nullptr, *qp = nullptr;   // periodic lines: border records (complex double)
-  void *xf = nullptr, *xb = nullptr;   // twisted lines: per step pair, the second row's
-                                       // original N2 (forward) / Q4 (backward) block
   void *flags = nullptr;   // per line: 1 when its factors hold a non-finite entry or a zero pivot
 };
 
@@ -43,38 +41,43 @@ struct PentaPlan {
 struct PentaBatchItem {
   int n, h;
   long L;
-  const void *fwd, *bwd, *tail, *xf, *xb;
+  const void *fwd, *bwd, *tail;
   const void *p2, *qp;     // periodic lines: the border records
   double2 *rhs[2];
   long sL, sR;
 };
 // the members of a batch that share a solve kernel; device tables
 struct PentaBatchGroup {
-  int variant = 0, prec = 0, count = 0;
+  int form = -1;           // form of the line solve; -1: periodic lines
+  int variant = 0;         // periodic lines: their kernel
+  int tw = 0, prec = 0, count = 0;
+  unsigned lds = 0;        // the most a member needs
   long blocks = 0;
   void *items = nullptr;   // PentaBatchItem[count]
   int *off = nullptr;      // first workgroup of each member, [count + 1]
 };
 
-// solve-kernel variants of non-periodic lines: one line per workgroup with a
-// deep LDS ring, two, three or four lines per workgroup, or twisted lines
-// (two chains): single steps, steps in pairs, or single steps with each
-// row's columns split over the two halves of the wave
+// solve-kernel variants of non-periodic lines: plain or twisted lines (two
+// chains per line), each with the form of the streaming solve that a rule on
+// the shape picks (PLAIN1, TWISTED), with a ring of six-row chunks (PLAIN2,
+// TWISTED_PAIRS), with a small LDS footprint (PLAIN3, TWISTED_HALF) or, plain
+// only, with the smallest (complex float: the longest) chunks (PLAIN4)
 enum { PENTA_PLAIN1 = 0, PENTA_PLAIN4 = 1, PENTA_TWISTED = 2, PENTA_PLAIN2 = 3, PENTA_PLAIN3 = 4,
        PENTA_TWISTED_PAIRS = 5, PENTA_TWISTED_HALF = 6, PENTA_NVARIANT = 7 };
 inline bool penta_twisted(int v) {
   return v == PENTA_TWISTED || v == PENTA_TWISTED_PAIRS || v == PENTA_TWISTED_HALF;
 }
 // the variant a plan of this shape uses: the autotuned one when
-// penta_tune has measured the shape, else a fixed rule
-int penta_variant_for(int n, long lines, int prec);
+// penta_tune has measured the shape, else a fixed rule; row_order: factors in
+// row order are kept for many lines (penta_solve_reference_order)
+int penta_variant_for(int n, long lines, int prec, bool row_order);
 // time every variant on synthetic lines of this shape (n rows, lines,
 // precision) and record the fastest; returns the chosen variant in *variant
 int penta_tune(int n, long lines, int prec, int *variant, float *times_ms);
 // record a variant for the shape without timing (later plans use it);
 // variant -1 drops the record (back to the fixed rule)
 int penta_tune_set(int n, long lines, int prec, int variant);
-int penta_plan_create(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec);
+int penta_plan_create(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec, bool row_order);
 int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec,
                               int variant);
 void penta_plan_destroy(PentaPlan *pl);

@@ -387,8 +387,8 @@ def ctx_bytes(p, precision=0) -> int:
 
 # line-solve variants the autotuner times (LNS3D_TUNE_VARIANTS)
 TUNE_VARIANTS = 7
-VARIANT_NAMES = ("1 line/WG", "4 lines/WG", "twisted", "2 lines/WG", "3 lines/WG", "twisted pairs",
-                 "twisted half")
+VARIANT_NAMES = ("plain", "plain, smallest chunks", "twisted", "plain, six-row chunks",
+                 "plain, small footprint", "twisted, six-row chunks", "twisted, small footprint")
 
 
 def tune_lines(n: int, lines: int, precision: int = 0):
