@@ -5,9 +5,10 @@
 // bordered).  Three stages:
 //
 //  1. Non-pivoted block LU.  Non-periodic lines: k_factor_chains, one wave
-//     per chain of rows with the rows being updated in an LDS window (lines
-//     of 16+ rows, when there are few lines, use a twisted order: two chains
-//     per line meeting in the middle).  Periodic lines: k_lu_per, one wave
+//     per chain of rows, the rows being updated in registers (interior rows)
+//     or in an LDS window (rows next to an end; lines of 16+ rows, when there
+//     are few lines, use a twisted order: two chains per line meeting in the
+//     middle).  Periodic lines: k_lu_per, one wave
 //     per line on a line-interleaved copy.  The storage of negated
 //     multipliers and the in-pivot order follow the reference
 //     (cpenta1bc.f:43-495, cpenta1p.f:46-654), including the periodic
@@ -66,13 +67,14 @@ struct LineGeom {
                  // rows n-1..h+2 bottom-up; -1: rows in order 0..n-1
 };
 
+// the slot of column c in row i of a line, -1 if it has none: slot k holds
+// column i - 2 + k, and the two rows next to an end hold the line's first or
+// last five columns, wrapped.  In arithmetic: a table would be a load from
+// memory for each look-up.
 __device__ __forceinline__ int bc_slot(int n, int i, int c) {
-  if (i == 0) { const int t[5] = {2, 3, 4, 0, 1}; return (c >= 0 && c <= 4) ? t[c] : -1; }
-  if (i == 1) { const int t[5] = {1, 2, 3, 4, 0}; return (c >= 0 && c <= 4) ? t[c] : -1; }
-  if (i == n - 2) { const int t[5] = {4, 0, 1, 2, 3}; int d = c - (n - 5); return (d >= 0 && d <= 4) ? t[d] : -1; }
-  if (i == n - 1) { const int t[5] = {3, 4, 0, 1, 2}; int d = c - (n - 5); return (d >= 0 && d <= 4) ? t[d] : -1; }
-  int d = c - i;
-  return (d >= -2 && d <= 2) ? d + 2 : -1;
+  const int lo = i < 2 ? 0 : i > n - 3 ? n - 5 : i - 2;
+  const int k = c - i + 2;
+  return (c < lo || c > lo + 4) ? -1 : k < 0 ? k + 5 : k > 4 ? k - 5 : k;
 }
 
 // where block (row i, column c) lives; false if structurally zero
@@ -464,8 +466,196 @@ __global__ __launch_bounds__(256) void k_records_rows(LineGeom g, const cx<TF> *
 }
 
 // ---------------------------------------------------------------------------
-// stage 1 for non-periodic lines: block LU with one wave per chain, the
-// rows v..v+4 of the chain in an LDS window.  A plain factor is one chain
+// A wave's elimination of one interior pivot row of a chain in registers.
+//
+// The pivot's window is 15 x 15: rows v..v+2 and columns v..v+2 as scalars.
+// Lane 16 g + j holds column j (15 idle) of row 0 and of the four rows
+//   slot 0: 1 + g;   slots 1-3: 5 + g + 4 (slot - 1)  (15 and 16 do not exist)
+// so that a row's 15 entries sit in one 16-lane row, where the multiplier of
+// column k reaches them as the DPP operand of the multiply-adds
+// (row_newbcast:k).  Pivot row k > 0 is passed from group k - 1 to the others
+// by v_permlane16/32_swap.  Every entry gets the operations of the generic
+// path in the same order: the in-block multipliers by cdiv, the partner rows'
+// by the pivot's reciprocal, then its updates by columns 0..4.
+template <int K> __device__ __forceinline__ double row_bcast(double x) {
+  const long long b = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0x150 + K, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x150 + K, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+// the value of 16-lane row G in all four
+template <int G> __device__ __forceinline__ double group_bcast(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  auto one = [](unsigned w) {
+    const auto a = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    const unsigned y = G < 2 ? a[0] : a[1];
+    const auto c = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+    return G % 2 == 0 ? c[0] : c[1];
+  };
+  const unsigned lo = one((unsigned)b), hi = one((unsigned)(b >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// fact = -1 / d and m = -a / d for a pivot d that all lanes hold: Smith's
+// algorithm with the wave's one branch, its quotients by reciprocals of the
+// denominators, corrected with their remainders (Markstein).  The denominators
+// lie between the pivot's larger part and twice that; near the ends of the
+// range they are divided by in full.
+__device__ __forceinline__ double pivot_recip(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(y, fma(-x, y, 1.0), y);
+}
+__device__ __forceinline__ double quotient(double a, double b, double y) {     // a / b, y = 1 / b
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+__device__ __forceinline__ void pivot_div(cx<double> d, cx<double> a, cx<double> &fact, cx<double> &m) {
+  const bool by_re = __any(fabs(d.re) >= fabs(d.im));
+  const double big = by_re ? fabs(d.re) : fabs(d.im);
+  if (__builtin_expect(__any(!(big > 0x1p-400 && big < 0x1p400)), 0)) {
+    fact = -crecip(d);
+    m = -cdiv(a, d);
+  } else if (by_re) {
+    const double r = quotient(d.im, d.re, pivot_recip(d.re)), den = fma(d.im, r, d.re), y = pivot_recip(den);
+    fact = cx<double>{quotient(-1, den, y), quotient(r, den, y)};
+    m = cx<double>{quotient(fma(-a.im, r, -a.re), den, y), quotient(fma(a.re, r, -a.im), den, y)};
+  } else {
+    const double r = quotient(d.re, d.im, pivot_recip(d.im)), den = fma(d.re, r, d.im), y = pivot_recip(den);
+    fact = cx<double>{quotient(-r, den, y), quotient(1, den, y)};
+    m = cx<double>{quotient(fma(-a.re, r, -a.im), den, y), quotient(fma(-a.im, r, a.re), den, y)};
+  }
+}
+
+struct PivotWindow {
+  cx<double> top;        // row 0
+  cx<double> s[4];       // slots 0-3
+
+  template <int K> __device__ __forceinline__ void step(int j, int g) {
+    cx<double> p = K == 0 ? top : cx<double>{group_bcast<(K + 3) % 4>(s[0].re), group_bcast<(K + 3) % 4>(s[0].im)};
+    cx<double> fact, m;
+    pivot_div(cx<double>{row_bcast<K>(p.re), row_bcast<K>(p.im)}, s[0], fact, m);
+    // column K becomes the multipliers
+    if (j == K) {
+      if (K < 4 && g >= K) s[0] = m;
+#pragma unroll
+      for (int t = 1; t < 4; t++) s[t] = cmul(s[t], fact);
+    }
+    // columns up to K, and in the block the rows up to the pivot, are final:
+    // they are updated by zeros
+    if (j <= K) p = cx<double>{0, 0};
+    cx<double> p0 = p;
+    if (g < K) p0 = cx<double>{0, 0};
+    // Lane K keeps its value throughout, so a slot is its own multiplier; the
+    // order leaves the two wait states between a write and its DPP read.
+#define LNS3D_PIV(ACC, M, P) "v_fmac_f64_dpp %" ACC ", " M ", %" P " row_newbcast:%12 row_mask:0xf bank_mask:0xf\n"
+    asm("s_nop 1\n"
+        LNS3D_PIV("0", "%0", "8") LNS3D_PIV("2", "%2", "10") LNS3D_PIV("4", "%4", "10") LNS3D_PIV("6", "%6", "10")
+        LNS3D_PIV("1", "%0", "9") LNS3D_PIV("3", "%2", "11") LNS3D_PIV("5", "%4", "11") LNS3D_PIV("7", "%6", "11")
+        LNS3D_PIV("0", "-%1", "9") LNS3D_PIV("2", "-%3", "11") LNS3D_PIV("4", "-%5", "11") LNS3D_PIV("6", "-%7", "11")
+        LNS3D_PIV("1", "%1", "8") LNS3D_PIV("3", "%3", "10") LNS3D_PIV("5", "%5", "10") LNS3D_PIV("7", "%7", "10")
+        : "+&v"(s[0].re), "+&v"(s[0].im), "+&v"(s[1].re), "+&v"(s[1].im), "+&v"(s[2].re), "+&v"(s[2].im),
+          "+&v"(s[3].re), "+&v"(s[3].im)
+        : "v"(p0.re), "v"(p0.im), "v"(p.re), "v"(p.im), "n"(K));
+#undef LNS3D_PIV
+  }
+};
+
+// The rows of a chain between its ends: pivots [vs, ve), chain row v at line
+// row v (dir 1) or n - 1 - v (dir -1).  The window moves down its diagonal
+// through the LDS array mx: an elimination leaves its trailing 10 x 10 there,
+// the 125 entries that the next window adds come from memory, read two pivots
+// ahead, and the 125 entries that are final go back, gathered in mx so that
+// two stores of whole blocks take them.  mx holds the first window on entry
+// and, in its first 10 rows and columns, the trailing part on return.  Entries
+// of rows and columns from zero_from on count as zero when they are first
+// read.  A chain is serial, so its time is latency: per pivot five divisions
+// in a row, the exchange through LDS, the multiply-adds of one wave.  Every
+// load and store of memory is unconditional (idle lanes repeat another's), so
+// that the wait for a window's entries counts past the stores in between.
+// 257 twisted lines of 513 rows: 1770 -> 530 to 660 us, 1.7 us a pivot (the same
+// elimination task by task in LDS took 5.8), of which its 450 vector
+// instructions take 1.0
+constexpr int MX_OUT = 17 * 16, MX_SIZE = MX_OUT + 125;     // 17 rows of 16, the final entries
+__device__ __forceinline__ void eliminate_interior(cx<double> *mx, cx<double> *lul, int n, int dir, int vs, int ve,
+                                                   int zero_from, int lane) {
+  const int j = min(lane & 15, 14), g = lane >> 4;           // lane 15 of a row repeats column 14
+  // block (v + dr, v + dc) of chain rows: its place in the line
+  auto place = [&](int v, int dr, int dc) {
+    return (dir > 0 ? v + dr : n - 1 - v - dr) * 125 + (2 + dir * (dc - dr)) * 25;
+  };
+  // this lane's two entries of what window v adds to window v - 1, and of
+  // what is final after pivot v
+  struct Entry { int from, at, low; } fr[2];      // low: the smaller of row and column
+  int fin[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int e = min(lane + 64 * h, 124), b = e / 25, in = e % 25;
+    const int dr = min(b, 2), dc = b < 2 ? 2 : b - 2;
+    fr[h] = Entry{place(0, dr, dc) + in, (dr * 5 + in / 5) * 16 + dc * 5 + in % 5, min(dr, dc)};
+    fin[h] = place(0, max(b - 2, 0), b < 3 ? b : 0) + in;
+  }
+  auto fetch = [&](int v, cx<double> (&x)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) x[h] = lul[fr[h].from + dir * v * 125];
+  };
+  // where this lane's entries go after a pivot: row 0 and slot 0 are final;
+  // of slots 1-3 columns 0-4 are, the rest moves up the diagonal
+  const int out0 = MX_OUT + (j / 5) * 25 + j % 5;
+  int to[4];
+#pragma unroll
+  for (int t = 1; t < 4; t++) {
+    const int r = 1 + g + 4 * t;
+    to[t] = r > 14 ? 15 * 16 + j : j < 5 ? MX_OUT + 75 + (r - 5) * 5 + j : (r - 5) * 16 + j - 5;
+  }
+  auto put_final = [&](int v, const cx<double> (&x)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) lul[fin[h] + dir * v * 125] = x[h];
+  };
+  // pivot v, with next the entries of window v + 1; those of window v + 2 are
+  // read into after.  Two sets in turn, as a copy from one to another
+  // would wait for the loads and the stores before them
+  auto pivot = [&](int v, cx<double> (&next)[2], cx<double> (&after)[2]) {
+    PivotWindow w;
+    w.top = mx[j];
+    w.s[0] = mx[(1 + g) * 16 + j];
+#pragma unroll
+    for (int t = 1; t < 4; t++) w.s[t] = mx[(1 + g + 4 * t) * 16 + j];
+    cx<double> done[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) done[h] = mx[MX_OUT + min(lane + 64 * h, 124)];
+    fetch(min(v + 2, ve - 1), after);
+    w.step<0>(j, g);
+    if (v > vs) put_final(v - 1, done);      // behind the first column, when they have come from LDS
+    w.step<1>(j, g);
+    w.step<2>(j, g);
+    w.step<3>(j, g);
+    w.step<4>(j, g);
+    wave_sync();
+    mx[out0] = w.top;
+    mx[out0 + 5 * (1 + g)] = w.s[0];
+#pragma unroll
+    for (int t = 1; t < 4; t++) mx[to[t]] = w.s[t];
+#pragma unroll
+    for (int h = 0; h < 2; h++)                                // after the last pivot nothing reads these
+      mx[fr[h].at] = v + 1 + fr[h].low >= zero_from ? cx<double>{0, 0} : next[h];
+    wave_sync();
+  };
+  cx<double> f1[2], f2[2];
+  fetch(min(vs + 1, ve - 1), f1);
+  wave_sync();
+  for (int v = vs; v < ve; v += 2) {
+    pivot(v, f1, f2);
+    if (v + 1 < ve) pivot(v + 1, f2, f1);
+  }
+  const cx<double> last[2] = {mx[MX_OUT + lane], mx[MX_OUT + min(lane + 64, 124)]};
+  put_final(ve - 1, last);
+}
+
+// ---------------------------------------------------------------------------
+// stage 1 for non-periodic lines: block LU with one wave per chain, interior
+// rows by eliminate_interior, the others with the rows v..v+4 of the chain in
+// an LDS window.  A plain factor is one chain
 // (rows 0..n-1).  The twisted factor runs two chains concurrently, rows
 // 0..h-1 top-down and rows n-1..h+2 bottom-up (the bottom one in reversed
 // indices, where the band looks the same); both update the 2x2 block of
@@ -481,7 +671,8 @@ constexpr int FW = 5;
 __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *lu, cx<double> *mid) {
   using T = double;
   __shared__ cx<T> win[2][FW][125];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ cx<T> mx[2][MX_SIZE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const long line = blockIdx.x;
   const int n = g.n, h = g.h;
   const bool tw = h >= 0;
@@ -516,9 +707,18 @@ __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *l
         win[w][vr % FW][e] = x;
       }
     };
-    auto load_row = [&](int vr) {
-      const cx<T> *src = lul + (long)real(vr) * 125;
-      put_row(vr, src[lane], lane + 64 < 125 ? src[lane + 64] : cx<T>{0, 0});
+    // rows v.. up to lim into the window, all loads before the first use
+    auto load_window = [&](int v) {
+      cx<T> x[FW][2];
+#pragma unroll
+      for (int r = 0; r < FW; r++) {
+        const cx<T> *src = lul + (long)real(min(v + r, lim)) * 125;
+        x[r][0] = src[lane];
+        x[r][1] = src[min(lane + 64, 124)];
+      }
+#pragma unroll
+      for (int r = 0; r < FW; r++)
+        if (v + r <= lim) put_row(v + r, x[r][0], x[r][1]);
     };
     // write back a row: own = all slots (pivot rows) or the chain's share
     auto store_row = [&](int vr, bool all) {
@@ -543,10 +743,36 @@ __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *l
         }
       }
     };
-    if (!preloaded)
-      for (int vr = v0; vr <= min(v0 + FW - 1, lim); vr++) load_row(vr);
+    if (!preloaded) load_window(v0);
     wsync();
+    // Pivots from 2 on whose partner rows v+1 and v+2 are interior rows of the
+    // line (and the chain's): the blocks right of them are columns v+1, v+2,
+    // and they go through registers.  The rows beside them keep the window.
+    const int vfast = min(v1, min(lim - 1, n - 5));
     for (int v = v0; v < v1; v++) {
+      if (v == 2 && v0 < 2 && vfast > 2) {
+        for (int e = lane; e < 225; e += 64) {
+          const int r = e / 15, c = e % 15;
+          mx[w][r * 16 + c] = B(v + r / 5, slot(v + r / 5, v + c / 5))[(r % 5) * 5 + c % 5];
+        }
+        // multipliers already formed in these rows
+        for (int e = lane; e < 75; e += 64) {
+          const int b = e / 25, vr = v + b / 2, vc = v - 2 + (b + 1) / 2, sl = slot(vr, vc);
+          lul[(long)real(vr) * 125 + sl * 25 + e % 25] = B(vr, sl)[e % 25];
+        }
+        wsync();
+        eliminate_interior(mx[w], lul, n, tt == 0 ? 1 : -1, v, vfast, tt == 1 && tw ? lim - 1 : n, lane);
+        __threadfence_block();
+        v = vfast;
+        load_window(v);
+        wsync();
+        for (int e = lane; e < 100; e += 64) {
+          const int r = e / 10, c = e % 10;
+          B(v + r / 5, slot(v + r / 5, v + c / 5))[(r % 5) * 5 + c % 5] = mx[w][r * 16 + c];
+        }
+        wsync();
+        if (v == v1) break;
+      }
       // row v+5 comes into the window when row v leaves it; its loads are
       // issued now, so that they arrive while row v is eliminated
       const bool pf_ok = v + FW <= lim;
@@ -556,138 +782,62 @@ __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *l
         pf0 = src[lane];
         pf1 = lane + 64 < 125 ? src[lane + 64] : cx<T>{0, 0};
       }
-      const int sd = slot(v, v);
-      cx<T> *D = B(v, sd);
-      // Interior pivot: rows v..v+4 (those up to lim) are interior rows of
-      // the line, and v+2 <= lim.  Then the right blocks are columns v+1,
-      // v+2 and the partners rows v+1, v+2, at slots fixed by the chain
-      // direction -- the generic path below with its lists in constants
-      // (the same operations on every element, in the same order).
-      const int sg = tt == 0 ? 1 : -1;
-      const bool fast = v >= 2 && v + 2 <= lim && min(v + 4, lim) <= n - 3;
-      if (fast) {
-        cx<T> *U0 = B(v, 2 + sg), *U1 = B(v, 2 + 2 * sg);
+      // Blocks right of the pivot (columns uc, slots us) and partner rows pr;
+      // filled and read with constant indices only, so that they stay in
+      // registers (a run-time index puts a local array in scratch).  Every
+      // loop over columns and tasks stays rolled, and a task decodes to an
+      // entry of whole blocks: this code runs four to eight times a chain, and
+      // its cost is fetching it (unrolled 200 of 660 us at 257 lines of 513)
+      cx<T> *D = B(v, slot(v, v));
+      int uc[4] = {0, 0, 0, 0}, us[4] = {0, 0, 0, 0}, pr[4] = {0, 0, 0, 0}, nu = 0, nparts = 0;
 #pragma unroll
-        for (int nc = 0; nc < 4; nc++) {
-          if (lane < 4 - nc) {
-            const int l = nc + 1 + lane;
-            D[l * 5 + nc] = -cdiv(D[l * 5 + nc], D[nc * 5 + nc]);
-          }
-          wsync();
-          const int nd = (4 - nc) * (4 - nc), ntask = nd + 2 * (4 - nc) * 5;
-          for (int k = lane; k < ntask; k += 64) {
-            if (k < nd) {
-              const int l = nc + 1 + k / (4 - nc), q = nc + 1 + k % (4 - nc);
-              D[l * 5 + q] = cfma(D[l * 5 + nc], D[nc * 5 + q], D[l * 5 + q]);
-            } else {
-              const int kk = k - nd, u = kk / ((4 - nc) * 5), rem = kk % ((4 - nc) * 5);
-              const int l = nc + 1 + rem / 5, q = rem % 5;
-              cx<T> *U = u ? U1 : U0;
-              U[l * 5 + q] = cfma(D[l * 5 + nc], U[nc * 5 + q], U[l * 5 + q]);
-            }
-          }
-          wsync();
+      for (int d = 1; d <= 4; d++) {
+        const int vc = v + d;
+        const int su = vc <= lim ? slot(v, vc) : -1;
+        const bool hp = vc <= lim && slot(vc, v) >= 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          if (su >= 0 && nu == i) { uc[i] = vc; us[i] = su; }
+          if (hp && nparts == i) pr[i] = vc;
         }
-        cx<T> *L0 = B(v + 1, 2 - sg), *L1 = B(v + 2, 2 - 2 * sg);
-#pragma unroll
-        for (int nc = 0; nc < 5; nc++) {
-          const cx<T> fact = crecip(D[nc * 5 + nc]);
-          if (lane < 10) {
-            cx<T> *Lb = lane < 5 ? L0 : L1;
-            const int mm = lane % 5;
-            Lb[mm * 5 + nc] = -(Lb[mm * 5 + nc] * fact);
-          }
-          wsync();
-          const int nl = 2 * 5 * (4 - nc), ntask = nl + 2 * 2 * 25;
-          for (int k = lane; k < ntask; k += 64) {
-            if (k < nl) {
-              const int pp = k / (5 * (4 - nc)), rem = k % (5 * (4 - nc));
-              const int mm = rem / (4 - nc), q = nc + 1 + rem % (4 - nc);
-              cx<T> *Lb = pp ? L1 : L0;
-              Lb[mm * 5 + q] = cfma(Lb[mm * 5 + nc], D[nc * 5 + q], Lb[mm * 5 + q]);
-            } else {
-              const int kk = k - nl, pp = kk / 50, rem = kk % 50;
-              const int u = rem / 25, mm = (rem % 25) / 5, q = rem % 5;
-              cx<T> *Lb = pp ? L1 : L0;
-              cx<T> *Dst = B(v + 1 + pp, 2 + sg * (u - pp));
-              const cx<T> *U = u ? U1 : U0;
-              Dst[mm * 5 + q] = cfma(Lb[mm * 5 + nc], U[nc * 5 + q], Dst[mm * 5 + q]);
-            }
-          }
-          wsync();
+        nu += su >= 0;
+        nparts += hp;
+      }
+      auto pick = [](const int (&a)[4], int i) { return i == 0 ? a[0] : i == 1 ? a[1] : i == 2 ? a[2] : a[3]; };
+      // in-block LU of D, its row operations applied to the right blocks
+#pragma unroll 1
+      for (int nc = 0; nc < 4; nc++) {
+        const int l = nc + 1 + lane;
+        if (l < 5) D[l * 5 + nc] = -cdiv(D[l * 5 + nc], D[nc * 6]);
+        wsync();
+#pragma unroll 1
+        for (int k = lane; k < (1 + nu) * 25; k += 64) {
+          const int b = k / 25, e = k % 25, l = e / 5, q = e % 5;
+          cx<T> *X = b == 0 ? D : B(v, pick(us, b - 1));
+          if (l > nc && (b > 0 || q > nc)) X[e] = cfma(D[l * 5 + nc], X[nc * 5 + q], X[e]);
         }
-      } else {
-        // blocks right of the pivot (columns uc, slots us) and partner rows
-        // (pr); filled and read with constant indices only, so that they stay
-        // in registers (a run-time index puts a local array in scratch)
-        int uc[4] = {0, 0, 0, 0}, us[4] = {0, 0, 0, 0}, pr[4] = {0, 0, 0, 0}, nu = 0, nparts = 0;
-#pragma unroll
-        for (int d = 1; d <= 4; d++) {
-          const int vc = v + d;
-          const int su = vc <= lim ? slot(v, vc) : -1;
-          const bool hp = vc <= lim && slot(vc, v) >= 0;
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            if (su >= 0 && nu == i) { uc[i] = vc; us[i] = su; }
-            if (hp && nparts == i) pr[i] = vc;
-          }
-          nu += su >= 0;
-          nparts += hp;
+        wsync();
+      }
+      // partner rows: the block in the pivot column becomes the multipliers
+#pragma unroll 1
+      for (int nc = 0; nc < 5; nc++) {
+        if (lane < nparts * 5) {
+          const int p = pick(pr, lane / 5);
+          cx<T> *x = B(p, slot(p, v)) + (lane % 5) * 5 + nc;
+          *x = -(*x * crecip(D[nc * 6]));
         }
-        auto pick = [](const int (&a)[4], int i) { return i == 0 ? a[0] : i == 1 ? a[1] : i == 2 ? a[2] : a[3]; };
-        // in-block LU of D, its row operations applied to the right blocks
-        // (loops over nc unrolled: the task decodes divide by constants)
-#pragma unroll
-        for (int nc = 0; nc < 4; nc++) {
-          if (lane < 4 - nc) {
-            const int l = nc + 1 + lane;
-            D[l * 5 + nc] = -cdiv(D[l * 5 + nc], D[nc * 5 + nc]);
-          }
-          wsync();
-          const int nd = (4 - nc) * (4 - nc), ntask = nd + nu * (4 - nc) * 5;
-          for (int k = lane; k < ntask; k += 64) {
-            if (k < nd) {
-              const int l = nc + 1 + k / (4 - nc), q = nc + 1 + k % (4 - nc);
-              D[l * 5 + q] = cfma(D[l * 5 + nc], D[nc * 5 + q], D[l * 5 + q]);
-            } else {
-              const int kk = k - nd, u = kk / ((4 - nc) * 5), rem = kk % ((4 - nc) * 5);
-              const int l = nc + 1 + rem / 5, q = rem % 5;
-              cx<T> *U = B(v, pick(us, u));
-              U[l * 5 + q] = cfma(D[l * 5 + nc], U[nc * 5 + q], U[l * 5 + q]);
-            }
-          }
-          wsync();
+        wsync();
+#pragma unroll 1
+        for (int k = lane; k < nparts * (1 + nu) * 25; k += 64) {
+          const int pp = k / ((1 + nu) * 25), b = k / 25 - pp * (1 + nu), e = k % 25, q = e % 5, p = pick(pr, pp);
+          cx<T> *Lb = B(p, slot(p, v));
+          const int sdst = b == 0 ? slot(p, v) : slot(p, pick(uc, b - 1));
+          if (sdst < 0 || (b == 0 && q <= nc)) continue;      // no such block (does not occur in the band); final
+          const cx<T> *X = b == 0 ? D : B(v, pick(us, b - 1));
+          cx<T> *x = B(p, sdst) + e;
+          *x = cfma(Lb[e - q + nc], X[nc * 5 + q], *x);
         }
-        // partner rows: the block in the pivot column becomes the multipliers
-#pragma unroll
-        for (int nc = 0; nc < 5; nc++) {
-          const cx<T> fact = crecip(D[nc * 5 + nc]);
-          if (lane < nparts * 5) {
-            cx<T> *Lb = B(pick(pr, lane / 5), slot(pick(pr, lane / 5), v));
-            const int mm = lane % 5;
-            Lb[mm * 5 + nc] = -(Lb[mm * 5 + nc] * fact);
-          }
-          wsync();
-          const int nl = nparts * 5 * (4 - nc), ntask = nl + nparts * nu * 25;
-          for (int k = lane; k < ntask; k += 64) {
-            if (k < nl) {
-              const int pp = k / (5 * (4 - nc)), rem = k % (5 * (4 - nc));
-              const int mm = rem / (4 - nc), q = nc + 1 + rem % (4 - nc);
-              cx<T> *Lb = B(pick(pr, pp), slot(pick(pr, pp), v));
-              Lb[mm * 5 + q] = cfma(Lb[mm * 5 + nc], D[nc * 5 + q], Lb[mm * 5 + q]);
-            } else {
-              const int kk = k - nl, pp = kk / (nu * 25), rem = kk % (nu * 25);
-              const int u = rem / 25, mm = (rem % 25) / 5, q = rem % 5;
-              const int sdst = slot(pick(pr, pp), pick(uc, u));
-              if (sdst < 0) continue;      // no such block (does not occur in the band)
-              cx<T> *Lb = B(pick(pr, pp), slot(pick(pr, pp), v));
-              cx<T> *Dst = B(pick(pr, pp), sdst);
-              const cx<T> *U = B(v, pick(us, u));
-              Dst[mm * 5 + q] = cfma(Lb[mm * 5 + nc], U[nc * 5 + q], Dst[mm * 5 + q]);
-            }
-          }
-          wsync();
-        }
+        wsync();
       }
       // row v is final: write it back and bring in row v+5
       store_row(v, true);
@@ -698,25 +848,29 @@ __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *l
     // rows the chain updated but did not pivot
     for (int vr = v1; vr <= min(v1 + FW - 1, lim); vr++) store_row(vr, !tw);
   };
-  if (!tw) {
-    chain(0, 0, 0, n, n - 1, false);
-    return;
+  // the chain of this wave, and then the two rows between the chains; one call
+  // site, so that the code exists once
+  int tt = tw ? wave : 0, v0 = 0, v1 = !tw ? n : wave == 0 ? h : n - h - 2, lim = !tw ? n - 1 : wave == 0 ? h + 1 : n - 1 - h;
+  for (bool middle_rows = false;; middle_rows = true) {
+    chain(tt, tt, v0, v1, lim, middle_rows);
+    if (!tw || middle_rows) return;
+    __syncthreads();
+    if (wave != 0) return;
+    // rows h, h+1 with both chains' updates of their 2x2 middle block summed,
+    // then their elimination
+    for (int rr = h; rr <= h + 1; rr++)
+      for (int e = lane; e < 125; e += 64) win[0][rr % FW][e] = lul[(long)rr * 125 + e];
+    wsync();
+    for (int e = lane; e < 100; e += 64) {
+      const int b = e / 25, r = h + b / 2, c = h + b % 2;
+      cx<T> &x = win[0][r % FW][bc_slot(n, r, c) * 25 + e % 25];
+      x = x + midl[e];
+    }
+    wsync();
+    v0 = h;
+    v1 = h + 2;
+    lim = h + 1;
   }
-  if (wave == 0) chain(0, 0, 0, h, h + 1, false);
-  else chain(1, 1, 0, n - h - 2, n - 1 - h, false);
-  __syncthreads();
-  if (wave != 0) return;
-  // rows h, h+1 with both chains' updates of their 2x2 middle block summed,
-  // then their elimination
-  for (int rr = h; rr <= h + 1; rr++)
-    for (int e = lane; e < 125; e += 64) win[0][rr % FW][e] = lul[(long)rr * 125 + e];
-  wsync();
-  for (int e = lane; e < 100; e += 64) {
-    const int b = e / 25, r = h + b / 2, c = h + b % 2;
-    cx<T> &x = win[0][r % FW][bc_slot(n, r, c) * 25 + e % 25];
-    x = x + midl[e];
-  }
-  chain(0, 0, h, h + 2, h + 1, true);
 }
 
 // ---------------------------------------------------------------------------
