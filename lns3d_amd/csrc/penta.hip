@@ -35,6 +35,7 @@
 //  per line, the reference's substitution order on the LU working copy) is
 //  kept as the order-exact solve behind lns3d_penta_solve_reference_order.
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -352,10 +353,12 @@ __global__ void k_solve_lines(LineGeom g, const cx<T> *mat_, const cx<T> *per_, 
 // Records of (line, chain row)s: eight per workgroup, 32 lanes each (a row
 // and its inverses in LDS; lane (m, q) = (l / 5, l % 5) of lanes 0..24 forms
 // entry (m, q) of a block).  The row's five LU blocks are read with
-// consecutive lanes on consecutive entries.
+// consecutive lanes on consecutive entries; with flags, the line's flag is set
+// on the way if one of them is unhealthy (a pass of its own over the factors
+// took 58 us at 257 lines of 513 rows).
 template <typename TF, typename TR>
 __global__ __launch_bounds__(256) void k_records_rows(LineGeom g, const cx<TF> *mat, cx<TR> *fwd, cx<TR> *bwd,
-                                                      cx<TR> *tail) {
+                                                      cx<TR> *tail, int *flags) {
   __shared__ cx<TF> rowb[8][125];
   __shared__ cx<TF> Lis[8][25], Uis[8][25];
   const int n = g.n;
@@ -375,7 +378,13 @@ __global__ __launch_bounds__(256) void k_records_rows(LineGeom g, const cx<TF> *
   const int i = t == 0 ? j : n - 1 - j;
   cx<TF> *rb = rowb[grp];
   const cx<TF> *src = mat + ((line * n + i) * 125);
-  for (int e = gl; e < 125; e += 32) rb[e] = src[e];
+  bool bad = false;                // the row's share of the line's health (k_check_factor)
+  for (int e = gl; e < 125; e += 32) {
+    const cx<TF> x = src[e];
+    rb[e] = x;
+    bad |= !(isfinite(x.re) && isfinite(x.im)) || (e / 25 == 2 && e % 25 % 6 == 0 && x.re == 0 && x.im == 0);
+  }
+  if (flags && bad) flags[line] = 1;
   const int m = gl / 5, q = gl % 5;
   const bool act = gl < 25;
   const int sd = bc_slot(n, i, i) * 25;
@@ -1331,8 +1340,8 @@ __global__ __launch_bounds__(256) void k_solve_per(int n, long L, const cx<T> *_
 // layout conversions between the reference's arrays and the working copy
 // ref mat (5,5,5,...) element (slot k, r, c) of (line l, row i) at
 //   ((i*sRm + l*sLm) * 125 + k + 5r + 25c)
-__global__ void k_import_mat(const double2 *ref, cx<double> *lu, int n, long L, long sLm, long sRm,
-                             int line_major) {
+// Periodic lines keep the line index fastest.
+__global__ void k_import_mat(const double2 *ref, cx<double> *lu, int n, long L, long sLm, long sRm) {
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;   // over (i, k, r, c, line)
   long total = (long)n * 125 * L;
   if (idx >= total) return;
@@ -1341,7 +1350,34 @@ __global__ void k_import_mat(const double2 *ref, cx<double> *lu, int n, long L, 
   int c = e % 5, r = (e / 5) % 5, k = (e / 25) % 5;
   long i = e / 125;
   double2 v = ref[(i * sRm + line * sLm) * 125 + k + 5 * r + 25 * c];
-  lu[line_major ? line * n * 125 + e : idx] = cx<double>{v.x, v.y};
+  lu[idx] = cx<double>{v.x, v.y};
+}
+// Non-periodic lines: a block row's 125 entries are consecutive on both sides,
+// so IMP rows a workgroup are read in order and leave in order, transposed in
+// LDS between.  Bound by memory, 4000 B a row: 257 lines of 513 rows (528 MB)
+// 437 us with reads of one entry per 2000 B, 95 us (5.6 TB/s) so.
+constexpr int IMP = 16;
+__global__ __launch_bounds__(256) void k_import_rows(const double2 *ref, double2 *lu, int n, int rows, long sLm, long sRm) {
+  __shared__ double2 buf[IMP * 125];
+  const int row0 = blockIdx.x * IMP, count = min(IMP, rows - row0) * 125;
+  constexpr int PER = (IMP * 125 + 255) / 256;
+  double2 v[PER];
+#pragma unroll
+  for (int t = 0; t < PER; t++) {
+    const int e = min((int)threadIdx.x + 256 * t, count - 1), row = row0 + e / 125;
+    v[t] = ref[((row % n) * sRm + (row / n) * sLm) * 125 + e % 125];
+  }
+#pragma unroll
+  for (int t = 0; t < PER; t++) {
+    const int e = threadIdx.x + 256 * t, in = e % 125, k = in % 5, r = (in / 5) % 5, c = in / 25;
+    if (e < count) buf[e - in + k * 25 + r * 5 + c] = v[t];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < PER; t++) {
+    const int e = threadIdx.x + 256 * t;
+    if (e < count) lu[(long)row0 * 125 + e] = buf[e];
+  }
 }
 
 // Factor health (the reference has no pivoting and no check: a zero pivot
@@ -1374,23 +1410,25 @@ static int grid_for(long n, int b) { return (int)((n + b - 1) / b); }
 
 static int check_launch_grid(long total) { return (int)std::min<long>(grid_for(total, 256), 4096); }
 
-int penta_check_launch(PentaPlan *pl, hipStream_t s) {
+static int clear_flags(PentaPlan *pl, hipStream_t s) {
   if (!pl->flags) LNS3D_CHECK(hipMalloc(&pl->flags, (size_t)pl->L * sizeof(int)));
   hipLaunchKernelGGL(k_zero_i32, dim3(grid_for(pl->L, 256)), dim3(256), 0, s, (int *)pl->flags, pl->L);
-  const long n = pl->n, L = pl->L;
-  if (pl->periodic) {
-    const long tl = (long)pl->np * 125 * L, tp = (long)pl->np * 50 * L;
-    hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tl)), dim3(256), 0, s,
-                       (const cx<double> *)pl->lu, tl, L, 0, 0L, 1, (int *)pl->flags);
-    hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tp)), dim3(256), 0, s,
-                       (const cx<double> *)pl->per, tp, L, 0, 0L, 0, (int *)pl->flags);
-    hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tp)), dim3(256), 0, s,
-                       (const cx<double> *)pl->per2, tp, L, 0, 0L, 0, (int *)pl->flags);
-  } else {
-    const long tl = n * 125 * L;
-    hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tl)), dim3(256), 0, s,
-                       (const cx<double> *)pl->lu, tl, L, 1, n * 125, 1, (int *)pl->flags);
-  }
+  LNS3D_CHECK(hipGetLastError());
+  return 0;
+}
+
+int penta_check_launch(PentaPlan *pl, hipStream_t s) {
+  if (!pl->periodic) return 0;       // k_records_rows has checked them
+  const int rc = clear_flags(pl, s);
+  if (rc) return rc;
+  const long L = pl->L;
+  const long tl = (long)pl->np * 125 * L, tp = (long)pl->np * 50 * L;
+  hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tl)), dim3(256), 0, s,
+                     (const cx<double> *)pl->lu, tl, L, 0, 0L, 1, (int *)pl->flags);
+  hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tp)), dim3(256), 0, s,
+                     (const cx<double> *)pl->per, tp, L, 0, 0L, 0, (int *)pl->flags);
+  hipLaunchKernelGGL(k_check_factor<double>, dim3(check_launch_grid(tp)), dim3(256), 0, s,
+                     (const cx<double> *)pl->per2, tp, L, 0, 0L, 0, (int *)pl->flags);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
@@ -1399,8 +1437,8 @@ int penta_check_launch(PentaPlan *pl, hipStream_t s) {
 // of the refined step): their entries, per line
 int penta_check_records_launch(PentaPlan *pl, hipStream_t s) {
   if (!pl->prec) return 0;
-  if (!pl->flags) LNS3D_CHECK(hipMalloc(&pl->flags, (size_t)pl->L * sizeof(int)));
-  hipLaunchKernelGGL(k_zero_i32, dim3(grid_for(pl->L, 256)), dim3(256), 0, s, (int *)pl->flags, pl->L);
+  const int rc = clear_flags(pl, s);
+  if (rc) return rc;
   const long n = pl->n, L = pl->L;
   const long tf = n * 60 * L, tb = n * 66 * L;
   hipLaunchKernelGGL(k_check_factor<float>, dim3(check_launch_grid(tf)), dim3(256), 0, s,
@@ -1521,29 +1559,36 @@ void penta_plan_destroy(PentaPlan *pl) {
 }
 
 int penta_import(PentaPlan *pl, const void *ref_mat, long sLm, long sRm, hipStream_t s) {
-  long total = (long)pl->np * 125 * pl->L;
-  hipLaunchKernelGGL(k_import_mat, dim3(grid_for(total, 256)), dim3(256), 0, s,
-                     (const double2 *)ref_mat, (cx<double> *)pl->lu, pl->np, pl->L, sLm, sRm,
-                     pl->periodic ? 0 : 1);
+  if (pl->periodic) {
+    hipLaunchKernelGGL(k_import_mat, dim3(grid_for((long)pl->np * 125 * pl->L, 256)), dim3(256), 0, s,
+                       (const double2 *)ref_mat, (cx<double> *)pl->lu, pl->np, pl->L, sLm, sRm);
+  } else {
+    const long rows = pl->np * pl->L;
+    if (rows > INT_MAX) return set_error(__FILE__, __LINE__, "penta_import: more rows than an index holds");
+    hipLaunchKernelGGL(k_import_rows, dim3(grid_for(rows, IMP)), dim3(256), 0, s, (const double2 *)ref_mat,
+                       (double2 *)pl->lu, pl->np, (int)rows, sLm, sRm);
+  }
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
 
-int penta_factor_records_only(PentaPlan *pl, hipStream_t s) {
+static int records_launch(PentaPlan *pl, int *flags, hipStream_t s) {
   if (pl->periodic) return set_error(__FILE__, __LINE__, "records are for non-periodic lines");
   LineGeom g{pl->n, pl->periodic, pl->exact, pl->L, pl->h};
   const int nb = grid_for(pl->L * (long)pl->n, 8);
   if (pl->prec)
     hipLaunchKernelGGL((k_records_rows<double, float>), dim3(nb), dim3(256), 0, s, g,
                        (const cx<double> *)pl->lu, (cx<float> *)pl->fwd, (cx<float> *)pl->bwd,
-                       (cx<float> *)pl->tail);
+                       (cx<float> *)pl->tail, flags);
   else
     hipLaunchKernelGGL((k_records_rows<double, double>), dim3(nb), dim3(256), 0, s, g,
                        (const cx<double> *)pl->lu, (cx<double> *)pl->fwd, (cx<double> *)pl->bwd,
-                       (cx<double> *)pl->tail);
+                       (cx<double> *)pl->tail, flags);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
+
+int penta_factor_records_only(PentaPlan *pl, hipStream_t s) { return records_launch(pl, nullptr, s); }
 
 __global__ void k_narrow(const cx<double> *src, cx<float> *dst, long count) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1584,7 +1629,8 @@ int penta_factor(PentaPlan *pl, hipStream_t s) {
   hipLaunchKernelGGL(k_factor_chains, dim3((unsigned)pl->L), dim3(pl->h >= 0 ? 128 : 64), 0, s, g,
                      (cx<double> *)pl->lu, (cx<double> *)pl->mid);
   LNS3D_CHECK(hipGetLastError());
-  return penta_factor_records_only(pl, s);
+  const int rc = clear_flags(pl, s);
+  return rc ? rc : records_launch(pl, (int *)pl->flags, s);
 }
 
 // Forms of the line solve: rows of a chunk and buffers of its ring, and

@@ -104,7 +104,8 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
 int penta_batch_solve(const std::vector<PentaBatchGroup> &groups, int which, hipStream_t s);
 void penta_batch_free(std::vector<PentaBatchGroup> &groups);
 // factor health: flag the lines whose LU (and border fill) holds a
-// non-finite entry or a zero pivot (launch after penta_factor), or whose
+// non-finite entry or a zero pivot (launch after penta_factor, which has
+// flagged non-periodic lines already), or whose
 // complex-float records hold a non-finite entry (after the records); then
 // count them (synchronises s)
 int penta_check_launch(PentaPlan *pl, hipStream_t s);
