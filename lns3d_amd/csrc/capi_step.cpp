@@ -694,7 +694,7 @@ extern "C" int lns3d_step(lns3d_ctx *c, void *v_dev, void *dv_dev) {
     if (!rc) rc = record_norm(c, r);
     if (!rc && c->impl == 2) rc = launch_copy(c->vhist, v_dev, n, c->stream);
     if (!rc) rc = solve_xy(c, c->px, c->py, r);
-    if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, c->stream);
+    if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
   } else {
     // corrector iterations (src/impdrv3d.f90:173-358): vold stays the field at
     // the start of the step; the factors are those of the first iteration
@@ -705,7 +705,7 @@ extern "C" int lns3d_step(lns3d_ctx *c, void *v_dev, void *dv_dev) {
       if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, mode, c->stream, c->vhist, c->vstart);
       if (!rc && it == 0) rc = record_norm(c, r);
       if (!rc) rc = solve_xy(c, c->px, c->py, r);
-      if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, c->stream);
+      if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
     }
     if (!rc && c->impl == 2) std::swap(c->vhist, c->vstart);   // this step's start is the next v2old
   }
@@ -727,7 +727,7 @@ extern "C" int lns3d_step_forced(lns3d_ctx *c, void *v_dev, const void *vold_dev
   int rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, 5, c->stream, nullptr,
                       vold_dev ? vold_dev : v_dev, f_dev);
   if (!rc) rc = solve_xy(c, c->px, c->py, r);
-  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, c->stream);
+  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
   return rc;
 }
 
@@ -827,7 +827,7 @@ extern "C" int lns3d_step_refined(lns3d_ctx *c, void *v_dev, void *dv_dev, doubl
   if (iters_out) *iters_out = it;
   if (resid_out) *resid_out = c->last_resid;
   if (!(c->last_resid == c->last_resid)) return fail(LNS3D_ENONFINITE, "refinement produced NaN");
-  rc = launch_update_bc(c->p, c->c, v_dev, dv, c->stream);
+  rc = launch_update_bc(c->p, c->c, v_dev, dv, nullptr, c->stream);
   if (!rc) c->lstep++;
   return rc;
 }
@@ -844,7 +844,7 @@ extern "C" int lns3d_step_fp32(lns3d_ctx *c, void *v_dev, void *dv_dev) {
   if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, 1, c->stream);
   if (!rc) rc = record_norm(c, r);
   if (!rc) rc = solve_xy(c, c->px32, c->py32, r);
-  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, c->stream);
+  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
   if (!rc) c->lstep++;
   return rc;
 }
@@ -867,17 +867,20 @@ extern "C" int lns3d_step_refined_fixed(lns3d_ctx *c, void *v_dev, void *dv_dev,
   if (!rc) rc = record_norm(c, rhs);
   if (!rc) rc = launch_copy(dv, rhs, n, c->stream);
   if (!rc) rc = solve_xy(c, c->px32, c->py32, dv);
+  // the last correction is added with the update of v, unless the check's
+  // residual needs dv whole before it
+  const void *last = corrections > 0 && !check ? c->t2 : nullptr;
   for (int k = 0; k < corrections && !rc; k++) {
     rc = launch_af_matvec(c->p, c->c, dv, c->t2, c->t1, c->stream);
     if (!rc) rc = launch_residual_norms(rhs, c->t2, n, c->scal + 8, c->stream);
     if (!rc) rc = solve_xy(c, c->px32, c->py32, c->t2);
-    if (!rc) rc = launch_axpy(dv, c->t2, n, c->stream);
+    if (!rc && (k < corrections - 1 || !last)) rc = launch_axpy(dv, c->t2, n, c->stream);
   }
   if (!rc && check) {
     rc = launch_af_matvec(c->p, c->c, dv, c->t2, c->t1, c->stream);
     if (!rc) rc = launch_residual_norms(rhs, c->t2, n, c->scal + 8, c->stream);
   }
-  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, dv, c->stream);
+  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, dv, last, c->stream);
   if (!rc) c->lstep++;
   return rc;
 }
@@ -987,7 +990,7 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
   const bool capturing = !rc;
   const hipStream_t s = gr->s;
   // members with the inviscid wall rows take bcfix on the final increment
-  // (as launch_update_bc): dv += t2, bcfix, v += dv instead of the fused update
+  // (as launch_update_bc): dv += t2 and bcfix come before the update
   const bool fix = !rc && gr->sb.blocks[SB_STAGE_BCFIX] > 0;
   for (int k = 0; k < nsteps && !rc; k++) {
     rc = step_batch_rhs(gr->sb, s);
@@ -1000,11 +1003,10 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
       if (!rc) rc = step_batch_vec(gr->sb, SB_SUB, s);
       if (!rc) rc = penta_batch_solve(gr->gx, 1, s);
       if (!rc) rc = penta_batch_solve(gr->gy, 1, s);
-      if (!rc) rc = step_batch_vec(gr->sb, q == corrections - 1 && !fix ? SB_UPDATE : SB_ADD_DV, s);
+      if (!rc && (q < corrections - 1 || fix)) rc = step_batch_vec(gr->sb, SB_ADD_DV, s);
     }
     if (!rc && fix) rc = step_batch_bcfix(gr->sb, s);
-    if (!rc && (corrections == 0 || fix)) rc = step_batch_vec(gr->sb, SB_ADD_V, s);
-    if (!rc) rc = step_batch_itrbc(gr->sb, s);
+    if (!rc) rc = step_batch_update(gr->sb, corrections > 0 && !fix, s);
   }
   if (capturing) {
     hipGraph_t g = nullptr;

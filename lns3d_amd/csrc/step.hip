@@ -1407,6 +1407,159 @@ int launch_itrbc(const lns3d_params &p, const Coeffs &c, void *v, hipStream_t s)
   return 0;
 }
 
+// The end of a step in one pass: dv += t2 (where t2 is given: a refined step's
+// correction), v += dv, then itrBC3D on v; the values are those of the three
+// kernels in turn.  A thread takes component d of the wall strip of column i
+// (the rows the wall's closures read, first 5 nx threads) or of one point
+// above it, so that every value a boundary value is formed from is the
+// thread's own; a value that a periodic direction repeats is written to both
+// places by the thread of the first.  right = 9 reads two neighbours: its
+// column is left to itrbc_lr after this kernel (bc_after_update).
+//
+// Bound by launches below about 500 x 250 points.  As three kernels it cost a
+// step 3 to 4 us more (us a step, complex double: 65x33 44.4 -> 41.2, 129x65
+// 57.8 -> 53.9, 384x127 99.9 -> 96.0; a captured march of 129x65 72 -> 66),
+// and a refined step, which also added its correction apart, 4.6 us (257x129
+// 154.5 -> 149.9).
+__host__ __device__ __forceinline__ int strip_rows(const lns3d_params &p, bool inviscid) {
+  if (p.yper || inviscid) return 1;
+  return (p.wall >= 1 && p.wall <= 3) || p.wallt == 1 ? 5 : 1;
+}
+__host__ __device__ __forceinline__ bool bc_after_update(const lns3d_params &p) { return !p.xper && p.right == 9; }
+// threads of a grid
+__host__ __device__ __forceinline__ long update_threads(const lns3d_params &p, bool inviscid) {
+  return 5L * p.nx * (p.ny - strip_rows(p, inviscid) + 1);
+}
+__device__ __forceinline__ void update_bc(long t, const lns3d_params &p, const double *ftop, const double *fside,
+                                          const double *fwall, int wlo, int whi, const double *bnb, double2 *v,
+                                          double2 *dv, const double2 *t2) {
+  using namespace st;
+  const int nx = p.nx, ny = p.ny;
+  const bool inviscid = bnb && !p.yper;
+  const int S = strip_rows(p, inviscid);
+  if (t >= update_threads(p, inviscid)) return;
+  const int w = 5 * nx;
+  // the row above the strip and the place in it (32-bit division where it serves)
+  long above;
+  int at;
+  if (t >> 32) {
+    above = t / w;
+    at = (int)(t - above * w);
+  } else {
+    above = (unsigned)t / (unsigned)w;
+    at = (int)((unsigned)t - (unsigned)above * (unsigned)w);
+  }
+  const int i = at / 5, d = at - 5 * i;
+  // v + dv at this thread's row j (dv completed first)
+  auto updated = [&](long j) {
+    const long q = j * w + at;
+    double2 b = dv[q];
+    if (t2) {
+      const double2 e = t2[q];
+      b = make_double2(b.x + e.x, b.y + e.y);
+      dv[q] = b;
+    }
+    const double2 a = v[q];
+    return z{a.x + b.x, a.y + b.y};
+  };
+  // the left and right columns, then the periodic copy
+  auto put = [&](long j, int dd, z u) {
+    double2 *row = v + j * w;
+    if (!p.xper) {
+      auto F = [&](int side) { return z{fside[2 * ((5L * side + dd) * ny + j)], fside[2 * ((5L * side + dd) * ny + j) + 1]}; };
+      if (i == 0) {
+        if (p.left == 0) u = z{0, 0};
+        if (p.left == 1 || p.left == 4 || p.left == 5) u = F(0);
+      }
+      if (i == nx - 1) {
+        if (p.right == 0) u = z{0, 0};
+        if (p.right == 4 || p.right == 5) u = F(1);
+      }
+    } else if (i == 0) {
+      row[5L * (nx - 1) + dd] = make_double2(u.re, u.im);
+    }
+    row[5L * i + dd] = make_double2(u.re, u.im);
+  };
+  const bool copied = p.xper && i == nx - 1;      // written by the thread of column 0
+  if (above > 0) {
+    const long j = S - 1 + above;
+    z u = updated(j);
+    if (copied) return;
+    if (j == ny - 1) {
+      if (p.yper) return;                         // written by the thread of row 0
+      u = z{0, 0};
+      if (p.top == 1) u = z{ftop[2 * (d * nx + i)], ftop[2 * (d * nx + i) + 1]};
+    }
+    put(j, d, u);
+    return;
+  }
+  if (p.yper) {
+    const z u = updated(0);
+    if (copied) return;
+    put(0, d, u);
+    put(ny - 1, d, u);
+    return;
+  }
+  const bool on = i >= wlo && i <= whi;           // the wall extent is:ie
+  if (bnb) {
+    // the rotation couples components 2 and 3: the thread of component 2
+    // takes both (there is no t2 here: dv is whole)
+    if (copied || (on && d == 2)) return;
+    const z u = updated(0);
+    if (on && d == 1) {
+      const double2 a = v[at + 1], b = dv[at + 1];
+      const double b1 = bnb[i], b2 = bnb[nx + i];
+      const z ub = sc(b2, u) - sc(b1, z{a.x + b.x, a.y + b.y});
+      put(0, 1, sc(b2, ub));
+      put(0, 2, sc(-b1, ub));
+    } else {
+      put(0, d, u);
+    }
+    return;
+  }
+  z u[5];
+  u[0] = updated(0);
+  if (S == 5) {
+#pragma unroll
+    for (int r = 1; r < 5; r++) u[r] = updated(r);
+  }
+  if (copied) return;
+  auto W = [&](int k, int x) { return z{fwall[2 * (k * nx + x)], fwall[2 * (k * nx + x) + 1]}; };
+  auto lin = [&]() { return sc(gc2, u[1]) + sc(gc3, u[2]) + sc(gc4, u[3]) + sc(gc5, u[4]); };
+  if (d >= 1 && d <= 3) {
+    if (p.wall == 3) u[0] = W(d - 1, i);
+    else if (on) u[0] = z{0, 0};
+  } else if (on && d == 0) {
+    if (p.wall == 1) {
+      const z s = lin();
+      u[0] = z{-s.re / gc1, -s.im / gc1};
+    }
+    if (p.wall == 2) u[0] = z{2.0 * u[1].re - u[2].re, 2.0 * u[1].im - u[2].im};
+    if (p.wall == 3) u[0] = sc(4.0, u[1]) - sc(6.0, u[2]) + sc(4.0, u[3]) - u[4];
+  } else if (on) {
+    if (p.wallt == 0) u[0] = p.wall == 3 ? W(3, i - wlo) : z{0, 0};
+    if (p.wallt == 1) {
+      const z s = lin();
+      if (p.wall == 3) {
+        const z e = W(4, i - wlo) - s;
+        u[0] = z{e.re / gc1, e.im / gc1};
+      } else {
+        u[0] = z{-s.re / gc1, -s.im / gc1};
+      }
+    }
+  }
+  put(0, d, u[0]);
+  if (S == 5) {
+#pragma unroll
+    for (int r = 1; r < 5; r++) put(r, d, u[r]);
+  }
+}
+__global__ __launch_bounds__(256) void k_update_bc(lns3d_params p, const double *ftop, const double *fside,
+                                                   const double *fwall, int wlo, int whi, const double *bnb,
+                                                   double2 *v, double2 *dv, const double2 *t2) {
+  update_bc((long)blockIdx.x * blockDim.x + threadIdx.x, p, ftop, fside, fwall, wlo, whi, bnb, v, dv, t2);
+}
+
 __global__ void k_copy2(double2 *dst, const double2 *src, long n) {
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) dst[t] = src[t];
@@ -1572,14 +1725,23 @@ int launch_axpy(void *x, const void *d, long n, hipStream_t s) {
   return 0;
 }
 
-int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, hipStream_t s) {
-  if (c.bnb && !p.yper) {      // inviscid: the increment's wall row back to x, y components
+int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, const void *t2, hipStream_t s) {
+  const bool inviscid = c.bnb && !p.yper;
+  if (inviscid) {              // the increment's wall row back to x, y components
+    if (t2) {
+      const int rc = launch_axpy(dv, t2, 5L * p.nx * p.ny, s);
+      if (rc) return rc;
+      t2 = nullptr;
+    }
     hipLaunchKernelGGL(k_bcfix, dim3(nblocks(p.nx, 128)), dim3(128), 0, s, p.nx, c.bnb, (double2 *)dv);
-    LNS3D_CHECK(hipGetLastError());
   }
-  int rc = launch_axpy(v, dv, 5L * p.nx * p.ny, s);
-  if (rc) return rc;
-  return launch_itrbc(p, c, v, s);
+  hipLaunchKernelGGL(k_update_bc, dim3(nblocks(update_threads(p, inviscid), 256)), dim3(256), 0, s, p,
+                     (const double *)c.ftop, (const double *)c.fside, (const double *)c.fwall, c.wlo, c.whi, c.bnb,
+                     (double2 *)v, (double2 *)dv, (const double2 *)t2);
+  if (bc_after_update(p))
+    hipLaunchKernelGGL(k_itrbc_lr, dim3(nblocks(p.ny, 128)), dim3(128), 0, s, p, (const double *)c.fside, (double2 *)v);
+  LNS3D_CHECK(hipGetLastError());
+  return 0;
 }
 
 // ==========================================================================
@@ -1926,36 +2088,30 @@ __global__ __launch_bounds__(256) void kb_line_op(const StepBatchItem *items, co
   line_op((long)blockIdx.x - off[k], dir == 1 ? b.ax : b.ay, b.c, dir, b.buf[xs], b.buf[ys]);
 }
 
+// the end of a step (update_bc), with the last correction t2 or without
+__global__ __launch_bounds__(256) void kb_update_bc(const StepBatchItem *items, const int *off, int count, int with_t2) {
+  const int k = step_member(off, count);
+  const StepBatchItem &b = items[k];
+  update_bc(((long)blockIdx.x - off[k]) * blockDim.x + threadIdx.x, b.p, b.c.ftop, b.c.fside, b.c.fwall, b.c.wlo,
+            b.c.whi, b.c.bnb, b.buf[SB_V], b.buf[SB_DV], with_t2 ? b.buf[SB_T2] : nullptr);
+}
+
 // elementwise stages over the 5P values of a member
 __global__ void kb_vec(const StepBatchItem *items, const int *off, int count, int op) {
   const int k = step_member(off, count);
   const StepBatchItem &b = items[k];
   const long t = ((long)blockIdx.x - off[k]) * blockDim.x + threadIdx.x;
   if (t >= 5 * b.P) return;
-  double2 *v = b.buf[SB_V], *dv = b.buf[SB_DV], *rhs = b.buf[SB_RHS], *t2 = b.buf[SB_T2];
+  double2 *dv = b.buf[SB_DV], *rhs = b.buf[SB_RHS], *t2 = b.buf[SB_T2];
   if (op == SB_COPY) {
     dv[t] = rhs[t];
   } else if (op == SB_SUB) {
     const double2 bb = rhs[t], yy = t2[t];
     t2[t] = make_double2(bb.x - yy.x, bb.y - yy.y);
-  } else if (op == SB_ADD_DV || op == SB_UPDATE) {
+  } else {   // SB_ADD_DV
     const double2 a = dv[t], c = t2[t];
-    const double2 d = make_double2(a.x + c.x, a.y + c.y);
-    dv[t] = d;
-    if (op == SB_UPDATE) {
-      const double2 x = v[t];
-      v[t] = make_double2(x.x + d.x, x.y + d.y);
-    }
-  } else {   // SB_ADD_V
-    const double2 x = v[t], d = dv[t];
-    v[t] = make_double2(x.x + d.x, x.y + d.y);
+    dv[t] = make_double2(a.x + c.x, a.y + c.y);
   }
-}
-
-__global__ void kb_itrbc_wall_top(const StepBatchItem *items, const int *off, int count) {
-  const int k = step_member(off, count);
-  const StepBatchItem &b = items[k];
-  itrbc_wall_top((long)blockIdx.x - off[k], b.p, b.c.ftop, b.c.fwall, b.c.wlo, b.c.whi, b.c.bnb, b.buf[SB_V]);
 }
 
 __global__ void kb_itrbc_lr(const StepBatchItem *items, const int *off, int count) {
@@ -1991,8 +2147,8 @@ static long stage_blocks(int stage, const lns3d_params &p) {
     case SB_STAGE_POINT: return nblocks(P, RT);
     case SB_STAGE_LINE: return nblocks(P, 256);
     case SB_STAGE_VEC: return nblocks(5 * P, 256);
-    case SB_STAGE_WALL: return nblocks(p.nx, 128);
-    default: return nblocks(p.ny, 128);
+    case SB_STAGE_LR: return bc_after_update(p) ? nblocks(p.ny, 128) : 0;
+    default: return 0;
   }
 }
 
@@ -2022,6 +2178,7 @@ int step_batch_build(const StepBatchMember *m, int count, StepBatch &out, std::v
     for (int sg = 0; sg < SB_NSTAGE; sg++) {
       const long nb = sg == SB_STAGE_NORM    ? (a.norm ? std::min<long>(nblocks(it.P, 256), NORM_BLOCKS) : 0)
                       : sg == SB_STAGE_BCFIX ? ((a.c.bnb && !a.p.yper) ? nblocks(a.p.nx, 128) : 0)
+                      : sg == SB_STAGE_UPDATE ? nblocks(update_threads(a.p, a.c.bnb && !a.p.yper), 256)
                                              : stage_blocks(sg, a.p);
       if ((long)off[sg].back() + nb > 0x7fffffffL) return set_error(__FILE__, __LINE__, "batch too large");
       off[sg].push_back(off[sg].back() + (int)nb);
@@ -2114,12 +2271,13 @@ int step_batch_norm(const StepBatch &b, long k, hipStream_t s) {
   return 0;
 }
 
-int step_batch_itrbc(const StepBatch &b, hipStream_t s) {
+int step_batch_update(const StepBatch &b, bool with_t2, hipStream_t s) {
   const auto *it = (const StepBatchItem *)b.items;
-  hipLaunchKernelGGL(kb_itrbc_wall_top, dim3((unsigned)b.blocks[SB_STAGE_WALL]), dim3(128), 0, s, it,
-                     b.off[SB_STAGE_WALL], b.count);
-  hipLaunchKernelGGL(kb_itrbc_lr, dim3((unsigned)b.blocks[SB_STAGE_LR]), dim3(128), 0, s, it, b.off[SB_STAGE_LR],
-                     b.count);
+  hipLaunchKernelGGL(kb_update_bc, dim3((unsigned)b.blocks[SB_STAGE_UPDATE]), dim3(256), 0, s, it,
+                     b.off[SB_STAGE_UPDATE], b.count, (int)with_t2);
+  if (b.blocks[SB_STAGE_LR] > 0)
+    hipLaunchKernelGGL(kb_itrbc_lr, dim3((unsigned)b.blocks[SB_STAGE_LR]), dim3(128), 0, s, it, b.off[SB_STAGE_LR],
+                       b.count);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }

@@ -105,9 +105,9 @@ int launch_residual_norm_noalloc(const double *dtl, const void *r, long P, doubl
 int launch_forced_norm(const lns3d_params &p, const Coeffs &c, const void *r, double *part, int *nb,
                        hipStream_t s);
 // ftop: the top = 1 wave (Coeffs::ftop), null for top = 0
-// v += dv and itrBC3D; for the inviscid deck bcfix turns dv's wall row back
-// to x, y components first (src/impdrv3d.f90:333-336)
-int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, hipStream_t s);
+// dv += t2 (unless null), v += dv and itrBC3D; for the inviscid deck bcfix
+// turns dv's wall row back to x, y components first (src/impdrv3d.f90:333-336)
+int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, const void *t2, hipStream_t s);
 int launch_itrbc(const lns3d_params &p, const Coeffs &c, void *v, hipStream_t s);
 // the wall normals bnb [2][nx] from the metric's n1, n2 on the wall row
 int launch_wall_normals(const lns3d_params &p, const Coeffs &c, double *bnb, hipStream_t s);
@@ -125,10 +125,9 @@ int launch_copy(void *dst, const void *src, long n, hipStream_t s);   // complex
 // tables built once).  Buffers of a member: v, dv, rhs (the step's
 // residual), t1, t2 (the correction), work (U_xi)
 enum { SB_V = 0, SB_DV, SB_RHS, SB_T1, SB_T2, SB_WORK };
-// elementwise stages: dv = rhs; t2 = rhs - t2; dv += t2; dv += t2 then
-// v += dv; v += dv
-enum { SB_COPY = 0, SB_SUB, SB_ADD_DV, SB_UPDATE, SB_ADD_V };
-enum { SB_STAGE_D1X = 0, SB_STAGE_POINT, SB_STAGE_LINE, SB_STAGE_VEC, SB_STAGE_WALL, SB_STAGE_LR, SB_STAGE_NORM,
+// elementwise stages: dv = rhs; t2 = rhs - t2; dv += t2
+enum { SB_COPY = 0, SB_SUB, SB_ADD_DV };
+enum { SB_STAGE_D1X = 0, SB_STAGE_POINT, SB_STAGE_LINE, SB_STAGE_VEC, SB_STAGE_UPDATE, SB_STAGE_LR, SB_STAGE_NORM,
        SB_STAGE_BCFIX, SB_NSTAGE };
 // norm (optional): the member's residual-norm output of norm_count slots;
 // step k of a captured sequence writes slot (norm_idx + k) mod norm_count
@@ -157,8 +156,9 @@ int step_batch_rhs(const StepBatch &b, hipStream_t s);
 // t2 = Lx (Ly dv) through t1 (launch_af_matvec)
 int step_batch_matvec(const StepBatch &b, hipStream_t s);
 int step_batch_vec(const StepBatch &b, int op, hipStream_t s);
-// itrBC3D of v (launch_itrbc)
-int step_batch_itrbc(const StepBatch &b, hipStream_t s);
+// dv += t2 (with_t2; no member with the inviscid wall rows then), v += dv and
+// itrBC3D of v (launch_update_bc)
+int step_batch_update(const StepBatch &b, bool with_t2, hipStream_t s);
 // the residual norm sqrt(sum |rhs|^2 / dtl^2) of every member with a norm
 // output, into its slot for step k (the bits of launch_residual_norm)
 int step_batch_norm(const StepBatch &b, long k, hipStream_t s);
