@@ -585,7 +585,7 @@ extern "C" int lns3d_assemble(lns3d_ctx *c, int dir, void *mat_dev) {
 
 extern "C" int lns3d_lrhs3d(lns3d_ctx *c, const void *v_dev, void *r_dev) {
   if (!c || !c->coeffs_ready || !v_dev || !r_dev) return fail(LNS3D_EINVAL, "lns3d_lrhs3d: bad arguments");
-  return launch_rhs(c->p, c->st, c->c, v_dev, r_dev, c->work, 0, c->stream);
+  return launch_rhs(c->p, c->st, c->c, v_dev, r_dev, 0, c->stream);
 }
 
 extern "C" int lns3d_itrbc3d(lns3d_ctx *c, void *v_dev) {
@@ -690,7 +690,7 @@ extern "C" int lns3d_step(lns3d_ctx *c, void *v_dev, void *dv_dev) {
   auto refactor = [&](int iter) { return refactor_for(c, iter); };
   if (c->niter == 1) {
     rc = refactor(1);
-    if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, two ? 2 : 1, c->stream, c->vhist);
+    if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, two ? 2 : 1, c->stream, c->vhist);
     if (!rc) rc = record_norm(c, r);
     if (!rc && c->impl == 2) rc = launch_copy(c->vhist, v_dev, n, c->stream);
     if (!rc) rc = solve_xy(c, c->px, c->py, r);
@@ -702,7 +702,7 @@ extern "C" int lns3d_step(lns3d_ctx *c, void *v_dev, void *dv_dev) {
     for (int it = 0; it < c->niter && !rc; it++) {
       const int mode = it == 0 ? (two ? 2 : 1) : (two ? 4 : 3);
       rc = refactor(it + 1);
-      if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, mode, c->stream, c->vhist, c->vstart);
+      if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, mode, c->stream, c->vhist, c->vstart);
       if (!rc && it == 0) rc = record_norm(c, r);
       if (!rc) rc = solve_xy(c, c->px, c->py, r);
       if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
@@ -724,7 +724,7 @@ extern "C" int lns3d_step_forced(lns3d_ctx *c, void *v_dev, const void *vold_dev
   if (c->impl != 1)
     return fail(LNS3D_EUNSUPPORTED, "lns3d_step_forced: the shift-invert steps are backward Euler (impl = 1)");
   void *r = dv_dev ? dv_dev : c->r;
-  int rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, 5, c->stream, nullptr,
+  int rc = launch_rhs(c->p, c->st, c->c, v_dev, r, 5, c->stream, nullptr,
                       vold_dev ? vold_dev : v_dev, f_dev);
   if (!rc) rc = solve_xy(c, c->px, c->py, r);
   if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
@@ -738,7 +738,7 @@ extern "C" int lns3d_forced_residual(lns3d_ctx *c, const void *v_dev, const void
                                      void *r_dev, double *norm_out) {
   if (!c || !c->coeffs_ready || !v_dev || !vold_dev || !f_dev || !r_dev || !norm_out)
     return fail(LNS3D_EINVAL, "lns3d_forced_residual: bad arguments");
-  int rc = launch_rhs(c->p, c->st, c->c, v_dev, r_dev, c->work, 5, c->stream, nullptr, vold_dev, f_dev);
+  int rc = launch_rhs(c->p, c->st, c->c, v_dev, r_dev, 5, c->stream, nullptr, vold_dev, f_dev);
   int nb = 0;
   if (!rc) rc = launch_forced_norm(c->p, c->c, r_dev, c->scal + 16, &nb, c->stream);
   if (rc) return rc;
@@ -801,7 +801,7 @@ extern "C" int lns3d_step_refined(lns3d_ctx *c, void *v_dev, void *dv_dev, doubl
   void *dv = dv_dev ? dv_dev : c->r;
   void *rhs = c->t3;            // the residual r of the step
   int rc = refactor_for(c, 1);
-  if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, rhs, c->work, 1, c->stream);
+  if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, rhs, 1, c->stream);
   if (rc) return rc;
   rc = launch_copy(dv, rhs, n, c->stream);
   if (rc) return rc;
@@ -841,7 +841,7 @@ extern "C" int lns3d_step_fp32(lns3d_ctx *c, void *v_dev, void *dv_dev) {
     return fail(LNS3D_ENOTFACTORED, "lns3d_step_fp32: needs precision = 1 and lns3d_factor");
   void *r = dv_dev ? dv_dev : c->r;
   int rc = refactor_for(c, 1);
-  if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, c->work, 1, c->stream);
+  if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, r, 1, c->stream);
   if (!rc) rc = record_norm(c, r);
   if (!rc) rc = solve_xy(c, c->px32, c->py32, r);
   if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, r, nullptr, c->stream);
@@ -863,7 +863,7 @@ extern "C" int lns3d_step_refined_fixed(lns3d_ctx *c, void *v_dev, void *dv_dev,
   void *dv = dv_dev ? dv_dev : c->r;
   void *rhs = c->t3;
   int rc = refactor_for(c, 1);
-  if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, rhs, c->work, 1, c->stream);
+  if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, rhs, 1, c->stream);
   if (!rc) rc = record_norm(c, rhs);
   if (!rc) rc = launch_copy(dv, rhs, n, c->stream);
   if (!rc) rc = solve_xy(c, c->px32, c->py32, dv);
@@ -967,7 +967,6 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
     a.rhs = (double2 *)c->t3;
     a.t1 = (double2 *)c->t1;
     a.t2 = (double2 *)c->t2;
-    a.work = (double2 *)c->work;
     a.norm = c->norm_out;
     a.norm_count = c->norm_count;
     a.norm_idx = c->norm_idx;

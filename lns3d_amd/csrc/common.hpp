@@ -98,6 +98,18 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The workgroup barrier of waves with copies in flight: their LDS accesses
+// are complete (lgkmcnt 0) but the copies (or loads into registers) are not
+// waited for, as a __syncthreads fence would (it treats global_load_lds as
+// pending LDS writes).  The empty asm statements keep the compiler from moving memory
+// accesses across the barrier.
+__device__ __forceinline__ void loader_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);     // lgkmcnt(0); vmcnt, expcnt not waited for
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // finite-difference coefficient tables of the scheme (src/stencil.f90)
 namespace st {
 constexpr double ga1 = 8.333333333333333333333E-02, ga2 = -6.666666666666666666667E-01,

@@ -30,18 +30,6 @@ namespace lns3d {
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// The workgroup barrier of waves with copies in flight: their LDS accesses
-// are complete (lgkmcnt 0) but the copies are not waited for, as a
-// __syncthreads fence would (it treats global_load_lds as pending LDS
-// writes).  The empty asm statements keep the compiler from moving memory
-// accesses across the barrier.
-__device__ __forceinline__ void loader_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);     // lgkmcnt(0); vmcnt, expcnt not waited for
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // A lane's share of a block-row product.  In a 16-lane row, lanes 0-4 hold the
 // real parts of the five components and lanes 5-9 the imaginary parts, of the
 // vector v and of the product.  With a = (re | im) and b = (im | re) of the

@@ -27,6 +27,19 @@ __device__ __forceinline__ double sc(double a, double x) { return a * x; }
 __device__ __forceinline__ z sc(double a, z x) { return {a * x.re, a * x.im}; }
 __device__ __forceinline__ double ld(const double *p) { return *p; }
 __device__ __forceinline__ z ld(const double2 *p) { double2 v = *p; return {v.x, v.y}; }
+// the same, and a real at a byte offset, from pointers known to be to device
+// memory: pointers read from a batch's tables compile to flat accesses
+// otherwise, which the LDS's counter waits for as well
+#define LNS3D_GLOBAL __attribute__((address_space(1)))
+typedef double vec2d __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ z ldg(const double2 *p) {
+  const vec2d v = *(const LNS3D_GLOBAL vec2d *)p;
+  return {v.x, v.y};
+}
+__device__ __forceinline__ double ldg_at(const double *p, unsigned o) {
+  return *(const LNS3D_GLOBAL double *)((const LNS3D_GLOBAL char *)p + o);
+}
+__device__ __forceinline__ void stg(double2 *p, double2 v) { *(LNS3D_GLOBAL vec2d *)p = vec2d{v.x, v.y}; }
 // right = 9 (src/rhsbc3d.f90:317-320, src/itrbc3d.f90:408-410): the value
 // exp(2 log a - log b) of the column from the two columns inside it, formed
 // as a^2 / b (the same value, zero for a = 0, not finite for b = 0)
@@ -78,11 +91,10 @@ __device__ __forceinline__ bool smooth_at(int N, int p, int sym, double sgn, con
   return false;
 }
 
-template <typename S, typename V>
-__device__ __forceinline__ V d1(int N, int per, int p, const double *g, double dinv,
-                                const S *base, long es, int sym = 0, double sgn = 1.0) {
+// (x(q) is the value at position q; d1 and d2 below read it from memory)
+template <typename V, typename X>
+__device__ __forceinline__ V d1_of(int N, int per, int p, const double *g, double dinv, X x, int sym, double sgn) {
   using namespace st;
-  auto x = [&](int q) { return ld(base + (long)q * es); };
   if (per) {
     int m = N - 1;
     if (p == N - 1) p = 0;
@@ -110,12 +122,16 @@ __device__ __forceinline__ V d1(int N, int per, int p, const double *g, double d
          sc(g[4], x(p + 2)) + sc(g[5], x(p + 3));
 }
 
-// second derivative, src/cgrad2.f90:134-326
 template <typename S, typename V>
-__device__ __forceinline__ V d2(int N, int per, int p, const double *d, double dsinv,
+__device__ __forceinline__ V d1(int N, int per, int p, const double *g, double dinv,
                                 const S *base, long es, int sym = 0, double sgn = 1.0) {
+  return d1_of<V>(N, per, p, g, dinv, [&](int q) { return ld(base + (long)q * es); }, sym, sgn);
+}
+
+// second derivative, src/cgrad2.f90:134-326
+template <typename V, typename X>
+__device__ __forceinline__ V d2_of(int N, int per, int p, const double *d, double dsinv, X x, int sym, double sgn) {
   using namespace st;
-  auto x = [&](int q) { return ld(base + (long)q * es); };
   if (per) {
     int m = N - 1;
     if (p == N - 1) p = 0;
@@ -142,6 +158,11 @@ __device__ __forceinline__ V d2(int N, int per, int p, const double *d, double d
                          sc(dd5, x(N - 5)));
   return sc(d[0], x(p - 3)) + sc(d[1], x(p - 2)) + sc(d[2], x(p - 1)) + sc(d[3], x(p)) +
          sc(d[4], x(p + 1)) + sc(d[5], x(p + 2)) + sc(d[6], x(p + 3));
+}
+template <typename S, typename V>
+__device__ __forceinline__ V d2(int N, int per, int p, const double *d, double dsinv,
+                                const S *base, long es, int sym = 0, double sgn = 1.0) {
+  return d2_of<V>(N, per, p, d, dsinv, [&](int q) { return ld(base + (long)q * es); }, sym, sgn);
 }
 
 Stencil make_stencil(const lns3d_params &p) {
@@ -918,182 +939,225 @@ int launch_assemble_ref(const lns3d_params &p, const Coeffs &c, int dir, void *m
 }
 
 // ==========================================================================
-// RHS: c1 = d/dxi v first (stored), then the point operator
-// one lane per (point, component), so a wave's stencil loads are contiguous
-__device__ __forceinline__ void rhs_d1x(long bid, int nx, int ny, int xper, const Stencil &st, const double2 *v,
-                                        double2 *c1) {
-  long t = bid * blockDim.x + threadIdx.x;
-  if (t >= 5L * nx * ny) return;
-  const long q = t / 5;
-  const int e = (int)(t - 5 * q);
-  const int i = q % nx, j = q / nx;
-  z g = d1<double2, z>(nx, xper, i, st.gx, st.dxinv, v + 5L * nx * j + e, 5, st.sym, e == 2 ? -1.0 : 1.0);
-  c1[t] = make_double2(g.re, g.im);
-}
-__global__ void k_rhs_d1x(int nx, int ny, int xper, Stencil st, const double2 *v, double2 *c1) {
-  rhs_d1x(xcd_tile(blockIdx.x, gridDim.x), nx, ny, xper, st, v, c1);
-}
-
-// The point operator works on tiles of RT consecutive grid points with one
-// workgroup of five waves.  Phase 1 stages the tile's U and U_xi and its 17
-// stencil derivatives (U_eta; U_xixi, U_xieta, U_etaeta of components 1-4) in
-// LDS; phase 2 has wave m form row m of the operator for the tile, so each
-// wave streams one row of every coefficient matrix ([25][P] layout, one
-// contiguous run of RT values per load).  Terms are accumulated in the order
-// of src/lrhs3d.f90:45-220 (U,xi and U,eta; U; U,xixi; U,xieta; U,etaeta;
-// A_i/B_i; D_i), then rbe3D and rhsBC3D (impdrv3d.f90:444-470,
-// src/rhsbc3d.f90:34-160, 200-215).
-constexpr int RT = 64;   // the interior path's task split (320 threads, 512 tasks) assumes 64
-static_assert(RT == 64, "k_rhs_point_t's interior path assumes tiles of 64 points");
-constexpr int NDER = 17;
+// RHS: the point operator on tiles of up to RT points of one grid row, one
+// workgroup of eight waves each.
+//
+// Phase 1, one lane per (column, component) of the tile and HALO columns to
+// either side: v and U_eta of the column into LDS, U_etaeta of the tile's own
+// points, from one gather of the rows j-3 .. j+3.  Phase 2, one lane per
+// (point, component): U_xi, U_xixi and U_xieta = d/dxi U_eta from LDS.  Phase
+// 3, one lane per (row of the operator, point): a run of lanes streams one row
+// of every coefficient matrix ([25][P] layout); these loads are issued before
+// phase 1's values are waited for, so that they are in flight through phases
+// 1 and 2.  Terms are accumulated in the order of src/lrhs3d.f90:45-220 (U,xi
+// and U,eta; U; U,xixi; U,xieta; U,etaeta; A_i/B_i; D_i), then rbe3D and
+// rhsBC3D (impdrv3d.f90:444-470, src/rhsbc3d.f90:34-160, 200-215).  U_xieta is
+// d/dxi of U_eta rather than d/deta of U_xi: the two operators commute, and
+// the row's own halo serves.
+//
+// Bound by the coefficients' stream, 1000 bytes a point of 1224: 1025x257 in
+// 69 us, 4.7 TB/s (copies reach 6.1), 24 grids of 65x33 to 513x257 in 166 us;
+// small grids by one pass through the phases (65x33 10 us).  Before, U_xi was
+// stored by a kernel of its own, the operator read it over seven rows and its
+// coefficients' loads came behind the stencils: 101, 255 and 15 us.
+// Eight waves, so that two workgroups fill a CU at 128 registers (of five-wave
+// ones, one a row of the operator, a CU held two: its first SIMD takes two
+// waves of each); RT is the widest tile with one task a lane in phase 1.
+constexpr int RHS_THREADS = 512, HALO = 4, RT = RHS_THREADS / 5 - 2 * HALO;
+// tiles of a row; they share its columns evenly
+__host__ __device__ __forceinline__ int rhs_row_tiles(int nx) { return (nx + RT - 1) / RT; }
 
 struct StepBatchItem;
-__device__ __forceinline__ int step_member(const int *off, int count);
-__device__ __forceinline__ void batch_point_args(const StepBatchItem *items, const int *off, int count,
-                                                 lns3d_params &p, Stencil &st, Coeffs &c, const double2 *&v,
-                                                 const double2 *&c1a, double2 *&r, long &tile);
+struct RhsMember {           // what the kernel reads of a staged batch's member
+  const lns3d_params *p;
+  const Stencil *st;
+  const Coeffs *c;
+  const double2 *v;
+  double2 *r;
+};
+__device__ __forceinline__ RhsMember rhs_member(const StepBatchItem *items, const int *off, int count, long &bid);
 
 // BATCH: the kernel of a staged batch (the member's deck, coefficients and
 // buffers replace the arguments, from items; its workgroups are numbered
-// from off[member]); otherwise one context with its tiles numbered per XCD.
-// The single-context kernel keeps the arguments as kernel arguments: its
-// body moved into a device function was measured 11% slower (78 to 90
-// VGPRs).
+// from off[member]).  Tiles are numbered per XCD: those of neighbouring rows,
+// which share v, on one L2.
 template <bool BATCH>
-__global__ __launch_bounds__(320) void k_rhs_point_t(lns3d_params p, Stencil st, Coeffs c, const double2 *v,
-                                                    const double2 *c1a, double2 *r, int with_rbe,
-                                                    const double2 *v2old, const double2 *vold,
-                                                    const double2 *forcing, const StepBatchItem *items,
-                                                    const int *off, int count) {
+__global__ __launch_bounds__(RHS_THREADS, 4) void k_rhs(lns3d_params p_, Stencil st_, Coeffs c_, const double2 *v_,
+                                                    double2 *r_, int with_rbe, const double2 *v2old,
+                                                    const double2 *vold, const double2 *forcing,
+                                                    const StepBatchItem *__restrict__ items, const int *__restrict__ off, int count) {
   using namespace st;
-  long tile;
-  if constexpr (BATCH) batch_point_args(items, off, count, p, st, c, v, c1a, r, tile);
-  else tile = xcd_tile(blockIdx.x, gridDim.x);   // tiles of one XCD: consecutive rows
-  __shared__ double2 sv[5 * RT], sg1[5 * RT], sd[NDER * RT], sr[5 * RT];
+  long bid = xcd_tile(blockIdx.x, gridDim.x);
+  RhsMember mb{&p_, &st_, &c_, v_, r_};
+  if constexpr (BATCH) mb = rhs_member(items, off, count, bid);
+  const lns3d_params &p = *mb.p;
+  const Stencil &st = *mb.st;
+  const Coeffs &c = *mb.c;
+  const double2 *v = mb.v;
+  double2 *r = mb.r;
+  constexpr int NC = RT + 2 * HALO;    // columns held
+  __shared__ double2 sv[5 * NC], su[5 * NC], s22[4 * NC], s1[5 * NC], s11[4 * NC], s12[4 * NC];
   const int nx = p.nx, ny = p.ny;
   const long P = (long)nx * ny;
-  const long q0 = tile * RT;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int npt = (int)min((long)RT, P - q0);
-  if (tid < 5 * npt) {
-    sv[tid] = v[5 * q0 + tid];
-    sg1[tid] = c1a[5 * q0 + tid];
+  const int nt = rhs_row_tiles(nx), j = (int)((unsigned)bid / (unsigned)nt), tt = (int)bid - j * nt;
+  const int wid = nx / nt, rem = nx - wid * nt;
+  const int i0 = tt * wid + min(tt, rem), npt = wid + (tt < rem);
+  const long q0 = (long)j * nx + i0;
+  const int tid = threadIdx.x;
+
+  // ---- phase 1: column slot cs holds column i0 - HALO + cs; periodic xi: the
+  // columns wrapped onto 0 .. nx-2, which makes every stencil an interior one,
+  // and slot 0, which no stencil reads, holds column nx-1 as it is
+  const int cs = min(tid / 5, NC - 1), e1 = tid - 5 * (tid / 5);
+  int col = i0 - HALO + cs;
+  if (p.xper) {
+    if (col < 0) col += nx - 1;
+    if (col >= nx - 1) col -= nx - 1;
+    if (cs == 0) col = nx - 1;
   }
-  // stencil derivatives into LDS, one lane per (point, component): slots
-  // 0-4 U_eta, 5-8 U_xixi, 9-12 U_xieta, 13-16 U_etaeta (components 1-4).
-  // A tile within one row whose points all lie inside both directions'
-  // closures (no periodic direction) takes the interior stencils without
-  // branches: U_eta and U_etaeta from one 7-row gather of v, then U_xixi or
-  // U_xieta, then U_xieta again (threads below 192), each summed in the
-  // interior formula's order (the bits of d1, d2).  Other tiles loop over
-  // the tasks, whose four kinds span multiples of 64, so each wave works on
-  // one kind at a time.
-  // (the staged batch's kernel keeps the task loop: the interior path raises
-  // it from 78 to 97 VGPRs, six to four waves per SIMD, and its small grids
-  // have few such tiles)
-  bool inner = false;
-  if (!BATCH && !p.xper && !p.yper && npt == RT) {
-    const int i0 = (int)(q0 % nx), j0 = (int)(q0 / nx);
-    const int i1 = (int)((q0 + RT - 1) % nx), j1 = (int)((q0 + RT - 1) / nx);
-    inner = j0 == j1 && j0 >= 3 && j0 <= ny - 4 && i0 >= 3 && i1 <= nx - 4;
+  col = min(max(col, 0), nx - 1);      // slots past the line's ends are not read
+  const long es = 5L * nx;
+  // rows of the interior stencil around row jp (the last row of a periodic
+  // direction is row 0 again)
+  const int yp = p.yper != 0, jp = yp && j == ny - 1 ? 0 : j;
+  const bool yin = p.yper || (j >= 3 && j <= ny - 4);
+  const double2 *vc = v + 5 * col + e1;
+  z x[7];
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    const int jr = jp + k - 3, lo = yp ? jr + ny - 1 : 0, hi = yp ? jr + 1 - ny : ny - 1;
+    x[k] = ldg(vc + (jr < 0 ? lo : jr >= ny - yp ? hi : jr) * es);
   }
-  if (inner) {
-    const long es = 5L * nx;
-    {
-      const int pt = tid / 5, e = tid - 5 * pt;
-      const double2 *b = v + 5 * (q0 + pt) + e;
-      z x[7];
-#pragma unroll
-      for (int k = 0; k < 7; k++) x[k] = ld(b + (k - 3) * es);
-      const z h1 = sc(st.gy[0], x[0]) + sc(st.gy[1], x[1]) + sc(st.gy[2], x[2]) + sc(st.gy[3], x[4]) +
-                   sc(st.gy[4], x[5]) + sc(st.gy[5], x[6]);
-      const z h3 = sc(st.dy[0], x[0]) + sc(st.dy[1], x[1]) + sc(st.dy[2], x[2]) + sc(st.dy[3], x[3]) +
-                   sc(st.dy[4], x[4]) + sc(st.dy[5], x[5]) + sc(st.dy[6], x[6]);
-      sd[e * RT + pt] = make_double2(h1.re, h1.im);
-      if (e >= 1) sd[(12 + e) * RT + pt] = make_double2(h3.re, h3.im);
-    }
-#pragma unroll
-    for (int sl = 0; sl < 2; sl++) {
-      // task u of 512: U_xixi (u < 256), then U_xieta; components 1-4
-      const int u0 = tid + 5 * 64 * sl, u = min(u0, 511);
-      const bool xx = u < 256;
-      const int w4 = u & 255, pt = w4 >> 2, e = 1 + (w4 & 3);
-      const double2 *b = (xx ? v : c1a) + 5 * (q0 + pt) + e;
-      const long s1 = xx ? 5L : es;
-      z x[7];
-#pragma unroll
-      for (int k = 0; k < 7; k++) x[k] = ld(b + (k - 3) * s1);
-      const double *wv = xx ? st.dx : st.gy;
-      z h = sc(wv[0], x[0]) + sc(wv[1], x[1]) + sc(wv[2], x[2]);
-      if (xx) h = h + sc(wv[3], x[3]);
-      const int o = xx ? 4 : 3;
-      h = h + sc(wv[o], x[4]) + sc(wv[o + 1], x[5]) + sc(wv[o + 2], x[6]);
-      if (u0 < 512) sd[((xx ? 4 : 8) + e) * RT + pt] = make_double2(h.re, h.im);
-    }
-  } else
-  for (int tsk = tid; tsk < 5 * RT + 3 * 4 * RT; tsk += 5 * 64) {
-    int kind, pt, e;
-    if (tsk < 5 * RT) { kind = 0; pt = tsk / 5; e = tsk - 5 * pt; }
-    else { const int u = tsk - 5 * RT; kind = 1 + u / (4 * RT); const int w4 = u % (4 * RT); pt = w4 / 4; e = 1 + w4 % 4; }
-    if (pt >= npt) continue;
-    const long qq = q0 + pt;
-    const int ii = (int)(qq % nx), jj = (int)(qq / nx);
-    z h;
-    if (kind == 0) {
-      h = d1<double2, z>(ny, p.yper, jj, st.gy, st.dyinv, v + 5L * ii + e, 5L * nx);
-      if (e == 4 && !c.bnb && (p.wallt == 1 || p.wallt == 2) && jj == 0) h = z{0, 0};   // src/cgradbc.f90:15 (Navier)
-    } else if (kind == 1) {
-      h = d2<double2, z>(nx, p.xper, ii, st.dx, st.dxsinv, v + 5L * nx * jj + e, 5, st.sym,
-                         e == 2 ? -1.0 : 1.0);
-    } else if (kind == 2) {
-      h = d1<double2, z>(ny, p.yper, jj, st.gy, st.dyinv, c1a + 5L * ii + e, 5L * nx);
-    } else {
-      h = d2<double2, z>(ny, p.yper, jj, st.dy, st.dysinv, v + 5L * ii + e, 5L * nx);
-    }
-    const int sl = kind == 0 ? e : 4 * kind + e;
-    sd[sl * RT + pt] = make_double2(h.re, h.im);
-  }
+
+  // ---- the coefficients of this lane's point (row m), used in phase 3.  The
+  // gather above is issued first (loads return in order); the compiler would
+  // sink it into the branch that uses it
+  asm volatile("" ::: "memory");
+  const bool on = tid < 5 * npt;
+  const int m = on ? (int)((unsigned)tid / (unsigned)npt) : 4, l = on ? tid - m * npt : npt - 1;
   const long q = q0 + l;
-  const int i = (int)(q % nx), j = (int)(q / nx);
-  __syncthreads();
-  if (l < npt) {
-    const int m = w;
-    auto S = [](double2 a) { return z{a.x, a.y}; };
-    auto g1 = [&](int e) { return S(sg1[5 * l + e]); };
-    auto g2 = [&](int e) { return S(sd[e * RT + l]); };
-    auto vq = [&](int e) { return S(sv[5 * l + e]); };
-    z a{0, 0};
+  const int i = i0 + l;
+  // byte offsets of 32 bits: five planes of 8 bytes a point stay below 4 GB
+  // (the other coefficients and the factors of a grid of 10^8 points would
+  // not fit the memory)
+  const unsigned oq = (unsigned)q * 8u, om = oq + (unsigned)(m * P) * 8u;
+  double cA[5], cB[5], cD[5], cI[5];
 #pragma unroll
-    for (int e = 0; e < 5; e++) a = a + sc(c.Ah[(long)(m + 5 * e) * P + q], g1(e));
+  for (int e = 0; e < 5; e++) cA[e] = ldg_at(c.Ah + 5 * e * P, om);
 #pragma unroll
-    for (int e = 0; e < 5; e++) a = a + sc(c.Bh[(long)(m + 5 * e) * P + q], g2(e));
+  for (int e = 0; e < 5; e++) cB[e] = ldg_at(c.Bh + 5 * e * P, om);
 #pragma unroll
-    for (int e = 0; e < 5; e++) a = a + sc(c.Dh[(long)(m + 5 * e) * P + q], vq(e));
+  for (int e = 0; e < 5; e++) cD[e] = ldg_at(c.Dh + 5 * e * P, om);
+#pragma unroll
+  for (int e = 0; e < 5; e++) cI[e] = ldg_at(c.Dhi + 5 * e * P, om);
+
+  {
+    z h1, h2;
+    if (yin) {
+      h1 = sc(st.gy[0], x[0]) + sc(st.gy[1], x[1]) + sc(st.gy[2], x[2]) + sc(st.gy[3], x[4]) + sc(st.gy[4], x[5]) +
+           sc(st.gy[5], x[6]);
+      h2 = sc(st.dy[0], x[0]) + sc(st.dy[1], x[1]) + sc(st.dy[2], x[2]) + sc(st.dy[3], x[3]) + sc(st.dy[4], x[4]) +
+           sc(st.dy[5], x[5]) + sc(st.dy[6], x[6]);
+    } else {
+      auto line = [&](int pos) { return ldg(vc + pos * es); };
+      h1 = d1_of<z>(ny, 0, j, st.gy, st.dyinv, line, 0, 1.0);
+      h2 = d2_of<z>(ny, 0, j, st.dy, st.dysinv, line, 0, 1.0);
+    }
+    const z own = jp != j ? ldg(vc + j * es) : x[3];
+    if (tid < 5 * NC) {
+      sv[tid] = make_double2(own.re, own.im);
+      su[tid] = make_double2(h1.re, h1.im);
+    }
+    if (e1 >= 1 && tid < 5 * NC) s22[(e1 - 1) * NC + cs] = make_double2(h2.re, h2.im);
+  }
+  loader_barrier();
+
+  // ---- the viscous entries of row m (m = 1: entries 0 and 4 with components
+  // 2 and 3; m = 2: 5 and 1; m = 3: 2 with 4; m = 4: 3 with 5), the spanwise
+  // cross entries and the time step, in flight through phase 2
+  const int w1 = m == 2 ? 5 : max(m - 1, 0), w2 = m == 2 ? 1 : 4;
+  const unsigned ow1 = oq + (unsigned)(w1 * P) * 8u, ow2 = oq + (unsigned)(w2 * P) * 8u;
+  double cV1[3], cV2[3] = {0, 0, 0}, cX[4] = {0, 0, 0, 0};
+  {
+    const double *Ws[3] = {c.V11, c.V12, c.V22};
+#pragma unroll
+    for (int t = 0; t < 3; t++) cV1[t] = ldg_at(Ws[t], ow1);
+    if (m == 1 || m == 2)
+#pragma unroll
+      for (int t = 0; t < 3; t++) cV2[t] = ldg_at(Ws[t], ow2);
+    if (m >= 1 && m <= 3)
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (m == 3 || (m == 1) == (k % 2 == 0)) cX[k] = ldg_at(c.ABhi + k * P, oq);
+  }
+  const double dt = with_rbe ? ldg_at(c.dtl, oq) : 0.0;
+
+  // ---- phase 2
+  const int pt = tid / 5, e2 = tid - 5 * pt;
+  if (pt < npt) {
+    const int ii = i0 + pt;
+    const double2 *vb = sv + 5 * (pt + HALO) + e2, *ub = su + 5 * (pt + HALO) + e2;
+    z hx, hxx, hxe;
+    if (p.xper || (i0 >= 3 && i0 + npt <= nx - 3)) {
+      auto first = [&](const double2 *b) {
+        return sc(st.gx[0], ld(b - 15)) + sc(st.gx[1], ld(b - 10)) + sc(st.gx[2], ld(b - 5)) +
+               sc(st.gx[3], ld(b + 5)) + sc(st.gx[4], ld(b + 10)) + sc(st.gx[5], ld(b + 15));
+      };
+      hx = first(vb);
+      hxe = first(ub);
+      hxx = sc(st.dx[0], ld(vb - 15)) + sc(st.dx[1], ld(vb - 10)) + sc(st.dx[2], ld(vb - 5)) + sc(st.dx[3], ld(vb)) +
+            sc(st.dx[4], ld(vb + 5)) + sc(st.dx[5], ld(vb + 10)) + sc(st.dx[6], ld(vb + 15));
+    } else {
+      const double sgn = e2 == 2 ? -1.0 : 1.0;
+      auto line = [&](const double2 *b) { return [=](int pos) { return ld(b + 5 * (pos - ii)); }; };
+      hx = d1_of<z>(nx, 0, ii, st.gx, st.dxinv, line(vb), st.sym, sgn);
+      hxe = d1_of<z>(nx, 0, ii, st.gx, st.dxinv, line(ub), st.sym, sgn);
+      hxx = d2_of<z>(nx, 0, ii, st.dx, st.dxsinv, line(vb), st.sym, sgn);
+    }
+    s1[e2 * NC + pt] = make_double2(hx.re, hx.im);
+    if (e2 >= 1) {
+      s11[(e2 - 1) * NC + pt] = make_double2(hxx.re, hxx.im);
+      s12[(e2 - 1) * NC + pt] = make_double2(hxe.re, hxe.im);
+    }
+  }
+  loader_barrier();
+
+  // ---- phase 3
+  const int ol = p.xper && i == nx - 1 ? 0 : l + HALO;    // the point's slot
+  auto S = [](double2 a) { return z{a.x, a.y}; };
+  auto g1 = [&](int e) { return S(s1[e * NC + l]); };
+  const bool heat = !c.bnb && (p.wallt == 1 || p.wallt == 2) && j == 0;     // src/cgradbc.f90:15 (Navier)
+  auto g2 = [&](int e) { return e == 4 && heat ? z{0, 0} : S(su[5 * ol + e]); };
+  auto vq = [&](int e) { return S(sv[5 * ol + e]); };
+  z a{0, 0};
+  if (on) {
+#pragma unroll
+    for (int e = 0; e < 5; e++) a = a + sc(cA[e], g1(e));
+#pragma unroll
+    for (int e = 0; e < 5; e++) a = a + sc(cB[e], g2(e));
+#pragma unroll
+    for (int e = 0; e < 5; e++) a = a + sc(cD[e], vq(e));
     if (m > 0) {
-      // viscous terms: slots 4+e (xixi), 8+e (xieta), 12+e (etaeta)
-      const double *Ws[3] = {c.V11, c.V12, c.V22};
 #pragma unroll
-      for (int tt = 0; tt < 3; tt++) {
-        const double *W = Ws[tt];
-        auto h = [&](int e) { return S(sd[(4 * tt + 4 + e) * RT + l]); };
-        if (m == 1) a = a - sc(W[q], h(1)) - sc(W[4 * P + q], h(2));
-        else if (m == 2) a = a - sc(W[5 * P + q], h(1)) - sc(W[P + q], h(2));
-        else if (m == 3) a = a - sc(W[2 * P + q], h(3));
-        else a = a - sc(W[3 * P + q], h(4));
+      for (int t = 0; t < 3; t++) {
+        auto h = [&](int e) {
+          return S(t == 0 ? s11[(e - 1) * NC + l] : t == 1 ? s12[(e - 1) * NC + l] : s22[(e - 1) * NC + ol]);
+        };
+        a = a - sc(cV1[t], h(m <= 2 ? 1 : m));
+        if (m <= 2) a = a - sc(cV2[t], h(2));
       }
     }
     if (m >= 1 && m <= 3) {
-      const double ab0 = c.ABhi[q], ab1 = c.ABhi[P + q], ab2 = c.ABhi[2 * P + q], ab3 = c.ABhi[3 * P + q];
       z ti;
-      if (m == 1) ti = sc(ab0, g1(3)) + sc(ab2, g2(3));
-      else if (m == 2) ti = sc(ab1, g1(3)) + sc(ab3, g2(3));
-      else ti = sc(ab0, g1(1)) + sc(ab1, g1(2)) + sc(ab2, g2(1)) + sc(ab3, g2(2));
+      if (m == 1) ti = sc(cX[0], g1(3)) + sc(cX[2], g2(3));
+      else if (m == 2) ti = sc(cX[1], g1(3)) + sc(cX[3], g2(3));
+      else ti = sc(cX[0], g1(1)) + sc(cX[1], g1(2)) + sc(cX[2], g2(1)) + sc(cX[3], g2(2));
       a = a + z{ti.im, -ti.re};                       // -i * ti
     }
     {
       z b{0, 0};
 #pragma unroll
-      for (int e = 0; e < 5; e++) b = b + sc(c.Dhi[(long)(m + 5 * e) * P + q], vq(e));
+      for (int e = 0; e < 5; e++) b = b + sc(cI[e], vq(e));
       a = a + z{-b.im, b.re};                         // + i * b
     }
     // sponge (src/lrhs3d.f90:222-282): sp1 v, then the inflow part sp2 (v - f)
@@ -1112,7 +1176,6 @@ __global__ __launch_bounds__(320) void k_rhs_point_t(lns3d_params p, Stencil st,
     // backward Euler: r = vold - v - dtl * r with vold = v (the field already
     // satisfies the boundary conditions when the step starts)
     if (with_rbe) {
-      const double dt = c.dtl[q];
       constexpr double onept33 = 1.3333333333333333333, pt33 = 3.3333333333333333333e-1;
       if (with_rbe == 2) {
         // two-step backward (src/impdrv3d.f90:473-501, rtb3D) with vold = v:
@@ -1205,46 +1268,42 @@ __global__ __launch_bounds__(320) void k_rhs_point_t(lns3d_params p, Stencil st,
           a = z{0, 0};
       }
     }
-    sr[5 * l + m] = make_double2(a.re, a.im);
   }
-  __syncthreads();
-  if (tid < 5 * npt) {
-    double2 o = sr[tid];
+  loader_barrier();
+  // the results go out through LDS, over s1, which has been read
+  if (on) s1[5 * l + m] = make_double2(a.re, a.im);
+  loader_barrier();
+  if (on) {
+    double2 o = s1[tid];
     // the inviscid wall rows (src/rhsbc3d.f90:108-118) on is:ie, rows 2 and 3
     // of the residual: the tangential momentum row rotated, the normal
     // velocity held at zero; the left and right columns keep their rows
-    const int pt = tid / 5, m = tid - 5 * pt;
-    const long qq = q0 + pt;
-    const int ii = (int)(qq % nx), jj = (int)(qq / nx);
-    if (c.bnb && with_rbe && !p.yper && jj == 0 && (m == 1 || m == 2) && ii >= c.wlo && ii <= c.whi) {
+    const int ii = i0 + pt;
+    if (c.bnb && with_rbe && !p.yper && j == 0 && (e2 == 1 || e2 == 2) && ii >= c.wlo && ii <= c.whi) {
       const bool lr = p.xper ? ii == nx - 1
                              : ((ii == 0 && (p.left == 0 || p.left == 1 || p.left == 4 || p.left == 5)) ||
                                 (ii == nx - 1 && (p.right == 0 || p.right == 4 || p.right == 5 || p.right == 8 ||
                                                   p.right == 9)));
       if (!lr) {
         const double b1 = c.bnb[ii], b2 = c.bnb[nx + ii];
-        if (m == 1) {
-          const z t = sc(b2, z{sr[5 * pt + 1].x, sr[5 * pt + 1].y}) - sc(b1, z{sr[5 * pt + 2].x, sr[5 * pt + 2].y});
+        if (e2 == 1) {
+          const z t = sc(b2, S(s1[5 * pt + 1])) - sc(b1, S(s1[5 * pt + 2]));
           o = make_double2(t.re, t.im);
         } else {
-          const z t = sc(b1, z{sv[5 * pt + 1].x, sv[5 * pt + 1].y}) + sc(b2, z{sv[5 * pt + 2].x, sv[5 * pt + 2].y});
+          const z t = sc(b1, S(sv[5 * (pt + HALO) + 1])) + sc(b2, S(sv[5 * (pt + HALO) + 2]));
           o = make_double2(-t.re, -t.im);
         }
       }
     }
-    r[5 * q0 + tid] = o;
+    stg(r + (5 * q0 + tid), o);
   }
 }
 
-int launch_rhs(const lns3d_params &p, const Stencil &st, const Coeffs &c, const void *v, void *r,
-               void *work, int with_rbe, hipStream_t s, const void *v2old, const void *vold,
-               const void *forcing) {
-  long P = (long)p.nx * p.ny;
-  hipLaunchKernelGGL(k_rhs_d1x, dim3(nblocks(5 * P, 256)), dim3(256), 0, s, p.nx, p.ny, p.xper, st,
-                     (const double2 *)v, (double2 *)work);
-  hipLaunchKernelGGL(k_rhs_point_t<false>, dim3(nblocks(P, RT)), dim3(5 * 64), 0, s, p, st, c, (const double2 *)v,
-                     (const double2 *)work, (double2 *)r, with_rbe, (const double2 *)v2old,
-                     (const double2 *)vold, (const double2 *)forcing, nullptr, nullptr, 0);
+int launch_rhs(const lns3d_params &p, const Stencil &st, const Coeffs &c, const void *v, void *r, int with_rbe,
+               hipStream_t s, const void *v2old, const void *vold, const void *forcing) {
+  hipLaunchKernelGGL(k_rhs<false>, dim3((unsigned)((long)rhs_row_tiles(p.nx) * p.ny)), dim3(RHS_THREADS), 0, s, p, st,
+                     c, (const double2 *)v, (double2 *)r, with_rbe, (const double2 *)v2old, (const double2 *)vold,
+                     (const double2 *)forcing, nullptr, nullptr, 0);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
@@ -2042,16 +2101,16 @@ struct StepBatchItem {
   Stencil st;
   Coeffs c;
   AsmCtx ax, ay;
-  double2 *buf[6];     // v, dv, rhs, t1, t2, work
+  double2 *buf[5];     // v, dv, rhs, t1, t2
   long P;
   double *norm;        // residual-norm slots (or null), as StepBatchMember
   int norm_count;
   long norm_idx;
 };
 
-__device__ __forceinline__ int step_member(const int *off, int count) {
+__device__ __forceinline__ int step_member(const int *off, int count, long bid) {
   int lo = 0, hi = count;
-  const int b = (int)blockIdx.x;
+  const int b = (int)bid;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (off[mid] <= b) lo = mid;
@@ -2059,25 +2118,13 @@ __device__ __forceinline__ int step_member(const int *off, int count) {
   }
   return lo;
 }
+__device__ __forceinline__ int step_member(const int *off, int count) { return step_member(off, count, blockIdx.x); }
 
-__global__ void kb_rhs_d1x(const StepBatchItem *items, const int *off, int count) {
-  const int k = step_member(off, count);
+__device__ __forceinline__ RhsMember rhs_member(const StepBatchItem *items, const int *off, int count, long &bid) {
+  const int k = step_member(off, count, bid);
   const StepBatchItem &b = items[k];
-  rhs_d1x((long)blockIdx.x - off[k], b.p.nx, b.p.ny, b.p.xper, b.st, b.buf[SB_V], b.buf[SB_WORK]);
-}
-
-__device__ __forceinline__ void batch_point_args(const StepBatchItem *items, const int *off, int count,
-                                                 lns3d_params &p, Stencil &st, Coeffs &c, const double2 *&v,
-                                                 const double2 *&c1a, double2 *&r, long &tile) {
-  const int k = step_member(off, count);
-  const StepBatchItem &b = items[k];
-  p = b.p;
-  st = b.st;
-  c = b.c;
-  v = b.buf[SB_V];
-  c1a = b.buf[SB_WORK];
-  r = b.buf[SB_RHS];
-  tile = (long)blockIdx.x - off[k];
+  bid -= off[k];
+  return RhsMember{&b.p, &b.st, &b.c, b.buf[SB_V], b.buf[SB_RHS]};
 }
 
 // y = L_dir x with x, y chosen among the member's buffers
@@ -2143,8 +2190,7 @@ __global__ __launch_bounds__(256) void kb_norm_final(const StepBatchItem *items,
 static long stage_blocks(int stage, const lns3d_params &p) {
   const long P = (long)p.nx * p.ny;
   switch (stage) {
-    case SB_STAGE_D1X: return nblocks(5 * P, 256);
-    case SB_STAGE_POINT: return nblocks(P, RT);
+    case SB_STAGE_RHS: return (long)rhs_row_tiles(p.nx) * p.ny;
     case SB_STAGE_LINE: return nblocks(P, 256);
     case SB_STAGE_VEC: return nblocks(5 * P, 256);
     case SB_STAGE_LR: return bc_after_update(p) ? nblocks(p.ny, 128) : 0;
@@ -2169,7 +2215,6 @@ int step_batch_build(const StepBatchMember *m, int count, StepBatch &out, std::v
     it.buf[SB_RHS] = a.rhs;
     it.buf[SB_T1] = a.t1;
     it.buf[SB_T2] = a.t2;
-    it.buf[SB_WORK] = a.work;
     it.P = (long)a.p.nx * a.p.ny;
     it.norm = a.norm;
     it.norm_count = a.norm ? a.norm_count : 0;
@@ -2220,11 +2265,9 @@ void step_batch_free(StepBatch &b) {
 
 int step_batch_rhs(const StepBatch &b, hipStream_t s) {
   const auto *it = (const StepBatchItem *)b.items;
-  hipLaunchKernelGGL(kb_rhs_d1x, dim3((unsigned)b.blocks[SB_STAGE_D1X]), dim3(256), 0, s, it, b.off[SB_STAGE_D1X],
+  hipLaunchKernelGGL(k_rhs<true>, dim3((unsigned)b.blocks[SB_STAGE_RHS]), dim3(RHS_THREADS), 0, s, lns3d_params{},
+                     Stencil{}, Coeffs{}, nullptr, nullptr, 1, nullptr, nullptr, nullptr, it, b.off[SB_STAGE_RHS],
                      b.count);
-  hipLaunchKernelGGL(k_rhs_point_t<true>, dim3((unsigned)b.blocks[SB_STAGE_POINT]), dim3(5 * 64), 0, s,
-                     lns3d_params{}, Stencil{}, Coeffs{}, nullptr, nullptr, nullptr, 1, nullptr, nullptr, nullptr,
-                     it, b.off[SB_STAGE_POINT], b.count);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }

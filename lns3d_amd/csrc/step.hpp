@@ -84,13 +84,13 @@ int launch_top_forcing(const lns3d_params &p, const Coeffs &c, const double *xto
 int launch_assemble(const lns3d_params &p, const Coeffs &c, int dir, PentaPlan &plan, hipStream_t s);
 // assembled LHS in the reference layout mat(5,5,5,nx,ny) (testing)
 int launch_assemble_ref(const lns3d_params &p, const Coeffs &c, int dir, void *mat, hipStream_t s);
-// r = -dtl * L(v) with the boundary rows of rhsBC3D; work holds 5P complex
+// r = -dtl * L(v) with the boundary rows of rhsBC3D
 // with_rbe: 0 the operator only, 1 backward Euler (rbe3D), 2 two-step
 // backward (rtb3D) with v2old, the field at the start of the previous step,
 // both with vold = v; 3 and 4 the same with vold given (corrector iterations);
 // 5 the forced form vold - v - dtl (L(v) - f) of the shift-invert driver
 int launch_rhs(const lns3d_params &p, const Stencil &st, const Coeffs &c, const void *v, void *r,
-               void *work, int with_rbe, hipStream_t s, const void *v2old = nullptr,
+               int with_rbe, hipStream_t s, const void *v2old = nullptr,
                const void *vold = nullptr, const void *forcing = nullptr);
 // the residual norm sqrt(sum |r|^2 / dtl^2) into *out (device), its
 // per-block partials in part (NORM_BLOCKS doubles); no host synchronisation
@@ -123,11 +123,11 @@ int launch_copy(void *dst, const void *src, long n, hipStream_t s);   // complex
 
 // batched steps: one launch per stage over the members of a batch (device
 // tables built once).  Buffers of a member: v, dv, rhs (the step's
-// residual), t1, t2 (the correction), work (U_xi)
-enum { SB_V = 0, SB_DV, SB_RHS, SB_T1, SB_T2, SB_WORK };
+// residual), t1, t2 (the correction)
+enum { SB_V = 0, SB_DV, SB_RHS, SB_T1, SB_T2 };
 // elementwise stages: dv = rhs; t2 = rhs - t2; dv += t2
 enum { SB_COPY = 0, SB_SUB, SB_ADD_DV };
-enum { SB_STAGE_D1X = 0, SB_STAGE_POINT, SB_STAGE_LINE, SB_STAGE_VEC, SB_STAGE_UPDATE, SB_STAGE_LR, SB_STAGE_NORM,
+enum { SB_STAGE_RHS = 0, SB_STAGE_LINE, SB_STAGE_VEC, SB_STAGE_UPDATE, SB_STAGE_LR, SB_STAGE_NORM,
        SB_STAGE_BCFIX, SB_NSTAGE };
 // norm (optional): the member's residual-norm output of norm_count slots;
 // step k of a captured sequence writes slot (norm_idx + k) mod norm_count
@@ -135,7 +135,7 @@ struct StepBatchMember {
   lns3d_params p;
   Stencil st;
   Coeffs c;
-  double2 *v, *dv, *rhs, *t1, *t2, *work;
+  double2 *v, *dv, *rhs, *t1, *t2;
   double *norm = nullptr;
   int norm_count = 0;
   long norm_idx = 0;
