@@ -64,24 +64,6 @@ __device__ __forceinline__ cx<float> bcast(cx<float> v, int lane) {
   return {a.f, b.f};
 }
 
-// broadcast lane q's complex value to the 16 lanes of its DPP row
-// (v_mov_b64_dpp row_newbcast:q); q must be a compile-time constant.  Every
-// lane receives a value, so bound_ctrl spares the old-value operand.
-template <int Q> __device__ __forceinline__ cx<double> row_bcast(cx<double> v) {
-  long a = __builtin_bit_cast(long, v.re), b = __builtin_bit_cast(long, v.im);
-  a = __builtin_amdgcn_update_dpp(0L, a, 0x150 + Q, 0xF, 0xF, true);
-  b = __builtin_amdgcn_update_dpp(0L, b, 0x150 + Q, 0xF, 0xF, true);
-  return {__builtin_bit_cast(double, a), __builtin_bit_cast(double, b)};
-}
-template <int Q> __device__ __forceinline__ cx<float> row_bcast(cx<float> v) {
-  long a = __builtin_bit_cast(long, v);
-  a = __builtin_amdgcn_update_dpp(0L, a, 0x150 + Q, 0xF, 0xF, true);
-  return __builtin_bit_cast(cx<float>, a);
-}
-template <typename T> __device__ __forceinline__ void row_bcast5(cx<T> v, cx<T> (&y)[5]) {
-  y[0] = row_bcast<0>(v); y[1] = row_bcast<1>(v); y[2] = row_bcast<2>(v);
-  y[3] = row_bcast<3>(v); y[4] = row_bcast<4>(v);
-}
 // The chip places workgroup b of a launch on XCD b % 8 (round robin over its
 // eight XCDs, each with its own L2).  xcd_tile(b, nb) numbers the tiles so
 // that each XCD works through a contiguous range of them (a bijection of

@@ -1,4 +1,4 @@
-// Streaming solve of non-periodic lines from their records.
+// Streaming solve of lines from their records.
 //
 // A workgroup of four waves runs two chains of block rows in lockstep: the
 // two halves of a twisted line (TW: chain 0 rows 0..h+1 top-down, chain 1 rows
@@ -108,18 +108,41 @@ template <int N, int U = 0, typename F> __device__ __forceinline__ void static_f
 // T: record precision; R: rows of a chunk (a multiple of three); NBUF: LDS
 // buffers; TW: twisted lines, one per workgroup, else two plain lines; RES:
 // the lines' right-hand sides stay in LDS from the first row to the last.
-template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
+//
+// PER: periodic lines (plain pairs).  Their bordered LU has the same band, so
+// rows 0 .. n-3 are a chain without boundary blocks; the last two rows meet
+// every other one:
+//   p2[row i]: what y_i adds to rows n-2 and n-1, summed by the waves that
+//     otherwise only write out, from the results in LDS;
+//   qp[row i]: what x_{n-2} and x_{n-1} add to row i, added where Uinv y is
+//     formed.
+// They ride through a ring of their own, whose buffers live as long as the
+// staged right-hand sides.  Between the passes one
+// wave solves rows n-2 and n-1 of both lines.  Bound by the memory from about
+// 400 lines (512 lines of 1023 rows, 3760 bytes a row: 382 us, 5.2 TB/s), by
+// the waves that prepare and sum below (97 of 256 rows 65 us, 0.76 us a chunk
+// where the chain takes 0.48).  Before, one line or four per workgroup, its
+// recurrence by broadcasts and the border blocks read from memory where they
+// were used: 474 and 92 us.  Border blocks held in registers two chunks ahead
+// were slower (473 and 99): the compiler copies them once loaded, and waits.
+template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> struct LineSolve {
+  static_assert(!(TW && PER), "periodic lines are plain");
   static_assert(R % 3 == 0, "three rotating register sets");
   static_assert(NBUF >= 4, "a chunk computed, one being prepared, two in flight");
   static constexpr int NROW = NBUF + 2;      // staged right-hand sides: two chunks more until they are copied out
   // LDS layout in bytes
   static constexpr unsigned CS = sizeof(cx<T>);
   static constexpr unsigned CHB = R * 66 * CS, BUFB = 2 * CHB;   // a chunk's records: one chain, both
-  static constexpr unsigned TAIL = NBUF * BUFB, TAILB = (150 * CS + 15) & ~15u;   // boundary blocks of a pass
+  // boundary blocks of a pass; PER: of both lines, the records of rows n-2
+  // and n-1 (60 and 66 values a row), their right-hand sides (80 bytes a
+  // row), the border sums (20 values) and the waves' shares of them
+  static constexpr unsigned TAIL = NBUF * BUFB, BREC = 2 * 2 * 126 * CS, BSUM = BREC + 4 * 80, BPART = BSUM + 20 * CS,
+                            TAILB = PER ? (BPART + 200 * CS + 15) & ~15u : (150 * CS + 15) & ~15u;
   static constexpr unsigned SV = TAIL + TAILB, SVB = (20 * CS + 15) & ~15u;       // rows kept for them
   static constexpr unsigned ROWB = 80;                           // a right-hand-side row
   static constexpr unsigned ZERO = SV + SVB, DUMMY = ZERO + R * ROWB;
-  static constexpr unsigned ROWS = DUMMY + R * ROWB;             // right-hand-side rows
+  static constexpr unsigned BORD = DUMMY + R * ROWB, BORDB = PER ? R * 50 * CS : 0;    // PER: a chunk's p2 or qp of one chain
+  static constexpr unsigned ROWS = BORD + NROW * 2 * BORDB;      // right-hand-side rows
   // rows of a resident right-hand side: a twisted line's inactive steps
   // touch one row before chain 1 and three after it
   static __host__ __device__ unsigned rows(int n) { return RES ? (TW ? n + 4 : 2 * n) : NROW * 2 * R; }
@@ -127,7 +150,11 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
 
   static __device__ __forceinline__ void run(char *sm, long bid, int n, int h, long L, const cx<T> *__restrict__ fwd,
                                              const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ tail,
-                                             double2 *rhs, long sL, long sR) {
+                                             double2 *rhs, long sL, long sR, const cx<T> *__restrict__ p2 = nullptr,
+                                             const cx<T> *__restrict__ qp = nullptr) {
+    // rows of a line in memory; of its chain (PER: without the last two)
+    const int nmem = n;
+    if (PER) n -= 2;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int len0 = TW ? h + 2 : n, len1 = TW ? n - h - 2 : n;
     // by chain, in arithmetic form: a select here becomes a per-lane table
@@ -168,7 +195,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
           for (int c = 0; c < 2; c++) {
             const int jb = first_row(fw, k, c), a = max(0, -jb), b = min(R, len(c) - jb);
             const char *src = reinterpret_cast<const char *>(fw ? fwd : bwd) +
-                              (line_of(c) * n + (TW ? c * len0 : 0) + jb) * ROW + lane * 16;
+                              (line_of(c) * nmem + (TW ? c * len0 : 0) + jb) * ROW + lane * 16;
             char *dst = sm + (buf * BUFB + c * CHB);
             if (a == 0 && b == R) {
               // 1 KB an instruction (16 B a lane); the last one ends with the
@@ -187,6 +214,27 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
         };
         if (fw) records(std::true_type{});
         else records(std::false_type{});
+        if constexpr (PER) {
+          constexpr int ROW = 50 * CS, FULL = R * ROW;
+          static_assert(FULL >= 1024 && FULL % 16 == 0, "as the records");
+#pragma unroll
+          for (int c = 0; c < 2; c++) {
+            const int jb = first_row(fw, k, c), a = max(0, -jb), b = min(R, len(c) - jb);
+            const char *src = reinterpret_cast<const char *>(fw ? p2 : qp) + (line_of(c) * nmem + jb) * ROW + lane * 16;
+            char *dst = sm + (BORD + (rb * 2 + c) * BORDB);
+            if (a == 0 && b == R) {
+              static_for<(FULL + 1023) / 1024>([&](auto I) {
+                constexpr int at = decltype(I)::value * 1024 + 1024 <= FULL ? decltype(I)::value * 1024 : FULL - 1024;
+                constexpr int base = at & ~4095;
+                __builtin_amdgcn_global_load_lds((const void *)(src + base), (lds_void *)(dst + base), 16, at - base, NT);
+              });
+            } else {
+              for (int o = a * ROW; o < b * ROW; o += 1024)
+                if (o + lane * 16 < b * ROW)
+                  __builtin_amdgcn_global_load_lds((const void *)(src + o), (lds_void *)(dst + o), 16, 0, NT);
+            }
+          }
+        }
         if (!RES) {
 #pragma unroll
           for (int rnd = 0; rnd < ROUNDS; rnd++) {
@@ -208,6 +256,23 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
           }
       };
       auto load_tail = [&](bool fw) {                  // boundary blocks of a pass
+        if constexpr (PER) {
+          if (!fw) return;                             // both passes' at the start
+          cx<T> v[8];
+          const int e20 = min(lane, 19);
+          const double2 b = rhs[(line_of(e20 / 10) * sL + (long)(n + e20 / 5 % 2) * sR) * 5 + e20 % 5];
+#pragma unroll
+          for (int i = 0; i < 8; i++) {                // line, row, value
+            const int e = min(i * 64 + lane, 503), c = e / 252, r = e / 126 % 2, k = e % 126;
+            const long row = line_of(c) * nmem + n + r;
+            v[i] = *(k < 60 ? fwd + (row * 60 + k) : bwd + (row * 66 + k - 60));
+          }
+#pragma unroll
+          for (int i = 0; i < 8; i++)
+            if (i * 64 + lane < 504) reinterpret_cast<cx<T> *>(sm + TAIL)[i * 64 + lane] = v[i];
+          if (lane < 20) *reinterpret_cast<double2 *>(sm + (TAIL + BREC + lane * 16)) = b;
+          return;
+        }
         cx<T> v[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
@@ -217,6 +282,95 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
 #pragma unroll
         for (int i = 0; i < 3; i++)
           if (i * 64 + lane < 150) reinterpret_cast<cx<T> *>(sm + TAIL)[i * 64 + lane] = v[i];
+      };
+      // PER, forward: the border sums of a finished chunk.  Lane e of 50 takes
+      // entry e of every row's p2 (border row, component, column e % 5) and
+      // sums its product with the row's y; the columns are added at the end
+      cx<T> bacc[2] = {{0, 0}, {0, 0}};
+      auto border_sum = [&](int k, int rb) {
+        if constexpr (PER) {
+          const int e = min(lane, 49), nr = min(R, n - k * R);
+#pragma unroll
+          for (int c = 0; c < 2; c++) {
+            const char *row = sm + (row_off(rb, c, k * R) + e % 5 * 16);
+            const cx<T> *blk = reinterpret_cast<const cx<T> *>(sm + (BORD + (rb * 2 + c) * BORDB)) + e;
+            if (nr == R) {
+#pragma unroll
+              for (int u = 0; u < R; u++)
+                bacc[c] = cfma(blk[u * 50], *reinterpret_cast<const cx<T> *>(row + u * ROWB), bacc[c]);
+            } else {
+              for (int u = 0; u < nr; u++)
+                bacc[c] = cfma(blk[u * 50], *reinterpret_cast<const cx<T> *>(row + u * ROWB), bacc[c]);
+            }
+          }
+        }
+      };
+      // rows n-2 and n-1 of both lines (one wave; lane a of ten has line a / 5
+      // and component a % 5): the forward rows with the border sums, then the
+      // backward ones, which become the chain's start and the qp terms' x
+      auto border_rows = [&]() {
+        if constexpr (PER) {
+          auto *bs = reinterpret_cast<cx<T> *>(sm + TAIL + BSUM);
+          const auto *part = reinterpret_cast<const cx<T> *>(sm + TAIL + BPART);
+          if (lane < 20) {
+            cx<T> t{0, 0};                             // over two waves and five columns
+#pragma unroll 1
+            for (int k = 0; k < 10; k++) t = t + part[k / 5 * 100 + lane * 5 + k % 5];
+            bs[lane] = t;
+          }
+          wave_sync();
+          const int c = min(lane / 5, 1), mm = lane % 5;
+          auto *xs = reinterpret_cast<cx<T> *>(sm + SV) + c * 10;      // y_{n-3}, y_{n-4}; then x_{n-2}, x_{n-1}
+          const auto *rec = reinterpret_cast<const cx<T> *>(sm + TAIL) + c * 252;
+          auto entry = [&](const cx<T> *r, int older, int q) {
+            const T *w = reinterpret_cast<const T *>(r) + mm * 20 + rec_pos(older, q);
+            return cx<T>{w[0], w[10]};
+          };
+          auto linv_b = [&](int r) {                   // Linv b, component mm
+            const cx<T> *L = rec + r * 126 + 50;
+            const double2 *b = reinterpret_cast<const double2 *>(sm + (TAIL + BREC)) + (c * 2 + r) * 5;
+            cx<T> acc{(T)b[mm].x, (T)b[mm].y};
+#pragma unroll 1
+            for (int q = 0; q < mm; q++) acc = cfma(L[mm * (mm - 1) / 2 + q], cx<T>{(T)b[q].x, (T)b[q].y}, acc);
+            return acc;
+          };
+          auto uinv = [&](int r, const cx<T> *y) {
+            const cx<T> *U = rec + r * 126 + 110 + mm * 5 - mm * (mm - 1) / 2;
+            cx<T> acc{0, 0};
+#pragma unroll 1
+            for (int q = mm; q < 5; q++) acc = cfma(U[q - mm], y[q], acc);
+            return acc;
+          };
+          cx<T> y0 = linv_b(0) + bs[c * 10 + mm], y1 = linv_b(1) + bs[c * 10 + 5 + mm];
+#pragma unroll 1
+          for (int q = 0; q < 5; q++) {
+            y0 = cfma(entry(rec, 0, q), xs[q], y0);
+            y0 = cfma(entry(rec, 1, q), xs[5 + q], y0);
+            y1 = cfma(entry(rec + 126, 1, q), xs[q], y1);
+          }
+          // y_{n-2}, y_{n-1} take the place of the border sums
+          wave_sync();
+          if (lane < 10) bs[c * 10 + mm] = y0;
+          wave_sync();
+#pragma unroll 1
+          for (int q = 0; q < 5; q++) y1 = cfma(entry(rec + 126, 0, q), bs[c * 10 + q], y1);
+          if (lane < 10) bs[c * 10 + 5 + mm] = y1;
+          wave_sync();
+          const cx<T> x1 = uinv(1, bs + c * 10 + 5);
+          cx<T> x0 = uinv(0, bs + c * 10);
+          if (lane < 10) xs[5 + mm] = x1;
+          wave_sync();
+#pragma unroll 1
+          for (int q = 0; q < 5; q++) x0 = cfma(entry(rec + 60, 0, q), xs[5 + q], x0);
+          if (lane < 10) {
+            xs[mm] = x0;
+            if (2 * bid + c < L) {
+              double2 *at = rhs + (line_of(c) * sL + (long)n * sR) * 5 + mm;
+              at[0] = make_double2(x0.re, x0.im);
+              at[sR * 5] = make_double2(x1.re, x1.im);
+            }
+          }
+        }
       };
       // c = Linv b or Uinv y in place, component lq of a row per lane (a
       // row's five lanes are in one wave: all have read before any writes)
@@ -261,6 +415,17 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
                 const cx<T> t = cfma(v[q], x[q], acc);
                 if (q < 5 - lq) acc = t;
               }
+              if constexpr (PER) {                     // what x_{n-2}, x_{n-1} add
+                const cx<T> *xb = reinterpret_cast<const cx<T> *>(sm + SV) + c * 10;
+                const cx<T> *blk = reinterpret_cast<const cx<T> *>(sm + (BORD + (rb * 2 + c) * BORDB)) + u * 50 + lq * 5;
+                cx<T> e{0, 0};
+#pragma unroll
+                for (int q = 0; q < 5; q++) {
+                  acc = cfma(blk[q], xb[q], acc);
+                  e = cfma(blk[25 + q], xb[5 + q], e);
+                }
+                acc = acc + e;
+              }
             }
             *reinterpret_cast<cx<T> *>(row + lq * 16) = acc;
           }
@@ -275,6 +440,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
             const cx<T> x =
                 *reinterpret_cast<const cx<T> *>(sm + (row_off(rb, c, first_row(fw, k, c)) + u * ROWB + lq * 16));
             *value_at(c, j) = make_double2(x.re, x.im);
+            if (PER && !fw && j == 0) rhs[(line_of(c) * sL + (long)nmem * sR) * 5 + lq] = make_double2(x.re, x.im);
           }
         }
       };
@@ -284,7 +450,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
       // iterations.  Waves 2 and 3 take turns to prepare the chunk one ahead
       // of the compute wave and to copy out the chunk two behind it (the
       // compute wave's barriers don't wait for its last write).
-      constexpr int OPS = 2 * ((R * 60 * (int)CS + 1023) / 1024) + (RES ? 0 : ROUNDS);   // copies of a full chunk, at least
+      constexpr int OPS = 2 * ((R * 60 * (int)CS + 1023) / 1024 + (PER ? (R * 50 * (int)CS + 1023) / 1024 : 0)) + (RES ? 0 : ROUNDS);   // copies of a full chunk, at least
       constexpr int AHEAD = (NBUF - 3) * OPS < 63 ? (NBUF - 3) * OPS : 63;   // copies younger than those waited for (a six-bit counter)
       // both passes are one stream of chunks where the right-hand sides are
       // resident (the backward pass's first chunk is prepared between them);
@@ -313,17 +479,39 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
           loader_barrier();
           int buf = NBUF - 1, rb = NBUF - 1;
           for (int K = 0; K < M; K++) {
-            if (RES && K == N) loader_barrier();
+            if (RES && K == N) {
+              if (PER) {
+                loader_barrier();
+                loader_barrier();
+              }
+              loader_barrier();
+            }
             if (K + NBUF - 1 < M) issue(is_fw(K + NBUF - 1), kk(K + NBUF - 1), buf, rb);
             wait_for(K);
             buf = buf + 1 == NBUF ? 0 : buf + 1;
             rb = rb + 1 == NROW ? 0 : rb + 1;
             loader_barrier();
           }
+          if (PER && !RES && pass == 0) {
+            loader_barrier();
+            loader_barrier();
+          }
         } else {
+          // wave p prepares, sums and writes out the chunks of its parity
           const int p = w - 1;
+          // PER: the border between the passes; the last two chunks' sums are
+          // still to be added
+          auto border = [&]() {
+            const int last = ((N - 1) & 1) == p ? N - 1 : N - 2;
+            if (last >= 0) border_sum(last, last % NROW);
+            if (lane < 50)
+              for (int c = 0; c < 2; c++) reinterpret_cast<cx<T> *>(sm + TAIL + BPART)[p * 100 + c * 50 + lane] = bacc[c];
+            loader_barrier();
+            if (p == 0) border_rows();
+            loader_barrier();
+          };
           if (RES) load_rhs(p, 2);
-          if (p == 1) load_tail(is_fw(0));
+          if (p == 1 && (!PER || pass == 0)) load_tail(is_fw(0));
           __builtin_amdgcn_s_waitcnt(0);
           loader_barrier();
           if (p == 0) prep(is_fw(0), 0, 0, 0);
@@ -331,14 +519,16 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
           int buf = 1, rb = 1, ro = 0;                  // buffers of chunks K + 1, staging of K - 2
           for (int K = 0; K < M; K++) {
             if (RES && K == N) {
-              if (p == 0) prep(false, 0, N % NBUF, 0);
+              if (PER) border();
+              if (p == 0) prep(false, 0, N % NBUF, N % NROW);
               else load_tail(false);
               loader_barrier();
             }
             if (((K + 1) & 1) == p) {
               if (K + 1 < M && !(RES && K + 1 == N)) prep(is_fw(K + 1), kk(K + 1), buf, rb);
-            } else if (K >= 2 && (!RES || K - 2 >= N)) {
-              copy_out(is_fw(K - 2), kk(K - 2), ro);
+            } else if (K >= 2) {
+              if (PER && is_fw(K - 2) && !(RES && K >= N)) border_sum(kk(K - 2), ro);
+              if (!RES || K - 2 >= N) copy_out(is_fw(K - 2), kk(K - 2), ro);
             }
             buf = buf + 1 == NBUF ? 0 : buf + 1;
             rb = rb + 1 == NROW ? 0 : rb + 1;
@@ -346,6 +536,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
             loader_barrier();
           }
           if (N - 2 + p >= 0) copy_out(is_fw(M - 1), N - 2 + p, (N - 2 + p) % NROW);
+          if (PER && !RES && pass == 0) border();
           __builtin_amdgcn_s_waitcnt(0);                // a forward pass's results are in memory
         }
         if (!RES) loader_barrier();
@@ -392,12 +583,12 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
     auto pass = [&](auto FWT, int K0) {
       constexpr bool FW = decltype(FWT)::value;
       constexpr unsigned ROW = (FW ? 60 : 66) * CS;
-      V = 0;
+      V = PER && !FW ? sv_lane(ch, hq) : T(0);      // PER: the backward chain starts from x_{n-2}, x_{n-1}
       const int jt = jtop(ch);
       // chunks of ordinary steps only: both chains active, no hand-off, no
       // boundary block, no value to keep
       const int main_lo = (!FW && TW) ? 1 : 0;
-      const int main_hi = FW ? (TW ? len1 : n - 3) : min(jtop(0), jtop(1)) - 2;
+      const int main_hi = PER ? n : FW ? (TW ? len1 : n - 3) : min(jtop(0), jtop(1)) - 2;
       // LDS offsets of a chunk for this lane: records (real, imaginary
       // broadcasts; their last columns), c read, result written
       struct At { unsigned a, a4, b, b4, c, y; };
@@ -443,7 +634,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
             if (ch == 1) sv_lane(0, hq) = V;
             wave_sync();
           }
-          if (FW && !TW && s == n - 3) {             // rows n-5, n-4
+          if (FW && !TW && !PER && s == n - 3) {     // rows n-5, n-4
             sv_lane(ch, 1 - hq) = V;
             wave_sync();
           }
@@ -453,13 +644,13 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
             if (ch == 1) V = sv_lane(1, 1 - hq);
             wave_sync();
           }
-          if (!FW && j == 2) sv_lane(ch, hq) = V;    // chain rows 3, 4
+          if (!FW && !PER && j == 2) sv_lane(ch, hq) = V;    // chain rows 3, 4
           if (!FW) wave_sync();
           T a[5], b[5];
           load(now, slot, a, b);
           T c = load_c(now, slot);
           // blocks of the pass's last two rows outside the band
-          const bool ends = FW ? (s >= len0 - 2 && (!TW || ch == 0)) : (j == 0 || j == 1);
+          const bool ends = PER ? false : FW ? (s >= len0 - 2 && (!TW || ch == 0)) : (j == 0 || j == 1);
           if (ends && hq == 0) {
             const int from = FW && TW ? 0 : ch;
             const bool end = FW ? s == len0 - 1 : j == 0;
@@ -513,6 +704,11 @@ template <typename T, int R, int NBUF, bool TW, bool RES> struct LineSolve {
     loader_barrier();
     loader_barrier();
     pass(std::true_type{}, 0);
+    if (PER) {
+      sv_lane(ch, hq) = V;    // y_{n-3}, y_{n-4}, for the rows the loader waves solve now
+      loader_barrier();
+      loader_barrier();
+    }
     loader_barrier();         // RES: the backward pass's first chunk is prepared; else the results are in memory
     if (!RES) {
       loader_barrier();
@@ -531,6 +727,16 @@ __global__ __launch_bounds__(256, 2) void k_line_solve(int n, int h, long L, con
                                                       double2 *rhs, long sL, long sR) {
   extern __shared__ __attribute__((aligned(16))) char sm[];
   LineSolve<T, R, NBUF, TW, RES>::run(sm, xcd_tile(blockIdx.x, gridDim.x), n, h, L, fwd, bwd, tail, rhs, sL, sR);
+}
+
+// periodic lines
+template <typename T, int R, int NBUF, bool RES>
+__global__ __launch_bounds__(256, 2) void k_line_solve_per(int n, long L, const cx<T> *__restrict__ fwd,
+                                                          const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ p2,
+                                                          const cx<T> *__restrict__ qp, double2 *rhs, long sL, long sR) {
+  extern __shared__ __attribute__((aligned(16))) char sm[];
+  LineSolve<T, R, NBUF, false, RES, true>::run(sm, xcd_tile(blockIdx.x, gridDim.x), n, -1, L, fwd, bwd, nullptr, rhs, sL,
+                                               sR, p2, qp);
 }
 
 }  // namespace lns3d

@@ -30,8 +30,8 @@
 //     ring and compute the parallel parts (Linv b, Uinv y).
 //  Periodic lines: k_records_per forms the same records from the bordered
 //  LU plus two border blocks per row (p2: rows n-2, n-1 in column i; qp:
-//  row i in columns n-2, n-1), and k_solve_per streams them through a ring
-//  with the border sums formed by the loader waves.  k_solve_lines (one lane
+//  row i in columns n-2, n-1), and k_line_solve_per streams them in pairs of
+//  lines with the border sums formed by the loader waves.  k_solve_lines (one lane
 //  per line, the reference's substitution order on the LU working copy) is
 //  kept as the order-exact solve behind lns3d_penta_solve_reference_order.
 #include <algorithm>
@@ -883,113 +883,12 @@ __global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *l
 }
 
 // ---------------------------------------------------------------------------
-// stage 3: streaming solve of non-periodic lines
-//
-// A workgroup of four waves.  Wave 0 runs the recurrences; waves 1-3 stream
-// the records through a ring of NBUF = 4 LDS buffers.  Chunk k (R rows of
-// each line or chain of the workgroup) belongs to loader wave 1 + k % 3,
-// which
-//   * in iteration k - 3 starts its copies: the record rows verbatim
-//     (global_load_lds_dwordx4, no VGPR round trip; fwd 60, bwd 66 complex
-//     per row) and the right-hand-side rows gathered into a staging buffer;
-//   * in iteration k - 1 waits for them (the only copies it has in flight)
-//     and replaces each staged row by its parallel part c_i = Linv_i b_i
-//     (forward) or d_i = Uinv_i y_i (backward).
-// A chunk's copies so have two iterations to arrive while the compute wave
-// works through the chunks before it.
-
-template <typename T>
-__device__ __forceinline__ void copy_rows_to_lds(const cx<T> *src, long src_elems_left, cx<T> *dst,
-                                                 int nelem, int wave_in, int nwaves, int lane) {
-  // copy nelem complex values src[0..nelem) -> dst[0..nelem) in 1 KB blocks
-  // per wave instruction; lanes past the end read a clamped (valid) address
-  // and write into the buffer's padding
-  constexpr int PER_LANE = 16 / sizeof(cx<T>);          // complex values per 16 B
-  const int nblk = (nelem * (int)sizeof(cx<T>) + 1023) / 1024;
-  for (int b = wave_in; b < nblk; b += nwaves) {
-    long e = (long)b * 64 * PER_LANE + (long)lane * PER_LANE;
-    long ec = e < src_elems_left - PER_LANE ? e : src_elems_left - PER_LANE;
-    if (ec < 0) ec = 0;
-    __builtin_amdgcn_global_load_lds((const void *)(src + ec),
-                                     (lds_void *)(dst + (long)b * 64 * PER_LANE), 16, 0, 0);
-  }
-}
-
-// the parallel part of one row, in place: bp[0..5) holds the row's
-// right-hand side (forward) or forward result (backward) in complex double,
-// rp the row's record.  Lane mm of the row overwrites bp[mm] with component
-// mm of c = Linv b (forward) or d = Uinv y (backward), as cx<T>.  The five
-// lanes of a row sit in one wave, so all of them have read the row before
-// any writes to it.
-template <typename T>
-__device__ __forceinline__ void parallel_part(double2 *bp, const cx<T> *rp, int mm, bool fw) {
-  cx<T> acc{0, 0};
-  if (fw) {
-    const cx<T> *Li = rp + 50 + mm * (mm - 1) / 2;
-    const double2 bm = bp[mm];
-    acc = cx<T>{(T)bm.x, (T)bm.y};
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-      if (q < mm) {
-        const double2 bq = bp[q];
-        acc = cfma(Li[q], cx<T>{(T)bq.x, (T)bq.y}, acc);
-      }
-  } else {
-    const cx<T> *Ui = rp + 50 + mm * 5 - mm * (mm - 1) / 2;
-#pragma unroll
-    for (int q = 0; q < 5; q++)
-      if (q < 5 - mm) {
-        const double2 yq = bp[mm + q];
-        acc = cfma(Ui[q], cx<T>{(T)yq.x, (T)yq.y}, acc);
-      }
-  }
-  *reinterpret_cast<cx<T> *>(bp + mm) = acc;
-}
-
-// The loader side of one pass over nchunk chunks (loader wave w = 0, 1, 2)
-// with a ring of NBUF (4 or 5) buffers.  Chunk k belongs to wave k % 3,
-// which starts its copies in iteration k - (NBUF - 1) and, in iteration
-// k - 1, waits for them and prepares the chunk before it starts any further
-// copies.  So a wave has one chunk's copies in flight when it waits, and
-// vmcnt(0) waits for exactly those (with NBUF = 5 the wave preparing chunk
-// k + 1 is the one that then starts chunk k + 4; in the prologue wave 0
-// waits for chunks 0 and 3).  One barrier after the prologue and one per
-// chunk, as in compute_pass.
-template <int NBUF, typename Issue, typename Prep>
-__device__ __forceinline__ void stream_pass(int nchunk, int w, Issue issue, Prep prep) {
-  static_assert(NBUF == 4 || NBUF == 5, "one chunk in flight per wave when it waits");
-  for (int c = w; c < NBUF - 1 && c < nchunk; c += 3) issue(c);
-  if (w == 0) {
-    __builtin_amdgcn_s_waitcnt(0);
-    prep(0);
-  }
-  loader_barrier();
-  for (int k = 0; k < nchunk; k++) {
-    if (k + 1 < nchunk && (k + 1) % 3 == w) {
-      __builtin_amdgcn_s_waitcnt(0);      // this wave's copies of chunk k + 1
-      prep(k + 1);
-    }
-    if (k + NBUF - 1 < nchunk && (k + NBUF - 1) % 3 == w) issue(k + NBUF - 1);   // buffer of chunk k - 1
-    loader_barrier();
-  }
-}
-
-template <typename Body>
-__device__ __forceinline__ void compute_pass(int nchunk, Body body) {
-  __syncthreads();
-  for (int k = 0; k < nchunk; k++) {
-    body(k);
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------------------------------------------
 // periodic lines (cpenta1p.f / cpenta2p.f): records from the bordered LU of
 // k_lu_per and a streaming solve.  The LU's band gives the same recurrence
 // as non-periodic lines; the border (rows n-2, n-1 in every column: per2;
 // columns n-2, n-1 in every row: per) becomes two more per-row records:
 //   p2[row c] = (Linv_{n-2} per2(n-2,c), Linv_{n-1} per2(n-1,c)): the forward
-//     contributions of y_c to the last two rows, summed by the loader waves;
+//     contributions of y_c to the last two rows;
 //   qp[row i] = (-Uinv_i per(i,n-2), -Uinv_i per(i,n-1)): the backward terms
 //     in x_{n-2}, x_{n-1}, which are known first, folded into d_i.
 __device__ __forceinline__ void inblock_inverses(const Blk<double> &D, cx<double> (&Li)[5][5],
@@ -1018,322 +917,62 @@ __device__ __noinline__ void records_per_row(LineGeom g, cx<double> *mat, cx<dou
   blk(g, mat, per, per2, line, i, i, D);
   inblock_inverses(D, Li, Ui);
   cx<double> *F = fwd + idx * 60, *B = bwd + idx * 66, *P2 = p2 + idx * 50, *QP = qp + idx * 50;
-  auto lmul = [&](const cx<double> (&A)[5][5], int row, int col, cx<double> *dst, int ld) {
+  // entry (m, q) of a block of the recurrence (rec_pos), of a border block
+  auto in_record = [](cx<double> *rec, int older) {
+    return [=](int m, int q, cx<double> v) {
+      double *w = reinterpret_cast<double *>(rec) + m * 20 + rec_pos(older, q);
+      w[0] = v.re;
+      w[10] = v.im;
+    };
+  };
+  auto in_block = [](cx<double> *dst) { return [=](int m, int q, cx<double> v) { dst[m * 5 + q] = v; }; };
+  auto lmul = [&](const cx<double> (&A)[5][5], int row, int col, auto put) {
     bool ok = col >= 0 && col < n && blk(g, mat, per, per2, line, row, col, M);
     for (int m = 0; m < 5; m++)
       for (int q = 0; q < 5; q++) {
         cx<double> acc{0, 0};
         if (ok)
           for (int k = 0; k <= m; k++) acc = cfma(A[m][k], M(k, q), acc);
-        dst[m * ld + q] = acc;
+        put(m, q, acc);
       }
   };
-  auto umul = [&](int col, cx<double> *dst, int ld) {
+  auto umul = [&](int col, auto put) {
     bool ok = col >= 0 && col < n && blk(g, mat, per, per2, line, i, col, M);
     for (int m = 0; m < 5; m++)
       for (int q = 0; q < 5; q++) {
         cx<double> acc{0, 0};
         if (ok)
           for (int k = m; k < 5; k++) acc = cfma(Ui[m][k], M(k, q), acc);
-        dst[m * ld + q] = cx<double>{-acc.re, -acc.im};
+        put(m, q, cx<double>{-acc.re, -acc.im});
       }
   };
   // band blocks only (columns i-1, i-2 / i+1, i+2 within the line)
-  if (i >= 1) lmul(Li, i, i - 1, F, 10); else lmul(Li, i, -1, F, 10);
-  if (i >= 2) lmul(Li, i, i - 2, F + 5, 10); else lmul(Li, i, -1, F + 5, 10);
+  lmul(Li, i, i >= 1 ? i - 1 : -1, in_record(F, 0));
+  lmul(Li, i, i >= 2 ? i - 2 : -1, in_record(F, 1));
   for (int l = 1, k = 0; l < 5; l++)
     for (int q = 0; q < l; q++, k++) F[50 + k] = Li[l][q];
-  umul(i + 1 < n ? i + 1 : -1, B, 10);
-  umul(i + 2 < n ? i + 2 : -1, B + 5, 10);
+  umul(i + 1 < n ? i + 1 : -1, in_record(B, 0));
+  umul(i + 2 < n ? i + 2 : -1, in_record(B, 1));
   for (int m = 0, k = 0; m < 5; m++)
     for (int q = m; q < 5; q++, k++) B[50 + k] = Ui[m][q];
   B[65] = cx<double>{0, 0};
   // border columns of row i (per exists for i < col-2)
-  umul(i < n - 4 ? n - 2 : -1, QP, 5);
-  umul(i < n - 3 ? n - 1 : -1, QP + 25, 5);
+  umul(i < n - 4 ? n - 2 : -1, in_block(QP));
+  umul(i < n - 3 ? n - 1 : -1, in_block(QP + 25));
   // border rows in column i (per2 exists for i < row-2), with those rows' Linv
   cx<double> Lb[5][5], Ub[5][5];
   blk(g, mat, per, per2, line, n - 2, n - 2, D);
   inblock_inverses(D, Lb, Ub);
-  lmul(Lb, n - 2, i < n - 4 ? i : -1, P2, 5);
+  lmul(Lb, n - 2, i < n - 4 ? i : -1, in_block(P2));
   blk(g, mat, per, per2, line, n - 1, n - 1, D);
   inblock_inverses(D, Lb, Ub);
-  lmul(Lb, n - 1, i < n - 3 ? i : -1, P2 + 25, 5);
+  lmul(Lb, n - 1, i < n - 3 ? i : -1, in_block(P2 + 25));
 }
 
 __global__ __launch_bounds__(128) void k_records_per(LineGeom g, cx<double> *mat, cx<double> *per, cx<double> *per2,
                               cx<double> *fwd, cx<double> *bwd, cx<double> *p2, cx<double> *qp) {
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx < g.L * g.n) records_per_row(g, mat, per, per2, fwd, bwd, p2, qp, idx);
-}
-
-// streaming solve of periodic lines: G lines per workgroup, one per DPP row
-// of the compute wave; rows 0..n-3 in chunks of R through the LDS ring.
-//   forward: rows 0..n-3 on the band, then rows n-2, n-1 with the border sums
-//            the loaders formed from p2 and the computed y;
-//   backward: rows n-1, n-2 first, then rows n-3..0 with d_i including
-//            qp_i (x_{n-2}, x_{n-1}); finally x(np) = x(1) (cpenta1p.f:1037).
-// T: the records' precision (complex float records are the complex-double
-// ones rounded; the right-hand side and solution stay complex double).
-// Workgroup bid takes lines bid*G .. bid*G + G - 1.
-template <typename T, int R, int G>
-__device__ __forceinline__ void solve_per(long bid, int n, long L, const cx<T> *__restrict__ fwd,
-                                          const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ p2,
-                                          const cx<T> *__restrict__ qp, double2 *rhs, long sL, long sR) {
-  constexpr int RECW = 66;
-  constexpr int BUFE = ((R * RECW * (int)sizeof(cx<T>) + 1023) / 1024) * 1024 / (int)sizeof(cx<T>);
-  __shared__ __attribute__((aligned(1024))) cx<T> rec[2][G][BUFE];
-  __shared__ cx<T> cb[2][G][R][5];
-  __shared__ cx<T> bsum[G][2][5];     // forward border sums into rows n-2, n-1
-  constexpr int NSUB = 192 / (10 * G);  // loader threads per border sum
-  __shared__ cx<T> bpart[NSUB][10 * G];
-  __shared__ cx<T> xb[G][2][5];       // x_{n-2}, x_{n-1}
-  const long line0 = bid * G;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int g = (lane >> 4) % G;
-  const int m = min(lane & 15, 4);
-  auto line_of = [&](int gg) { return min(line0 + gg, L - 1); };
-  const long line = line_of(g);
-  const long rs = sR * 5;
-  double2 *X = rhs + line * sL * 5;
-  const int nreg = n - 2;                         // rows 0..n-3: band recurrence only
-  const int nck = (nreg + R - 1) / R;
-  auto zx = [](double2 a) { return cx<T>{(T)a.x, (T)a.y}; };
-
-  // ---- loaders: record rows [r0, r0+nr) of pass fw into buffer kk, with
-  // c = Linv b (forward) or d = Uinv y + qp (x_{n-2}, x_{n-1}) (backward)
-  auto load = [&](int kk, int r0, int nr, bool fw, bool border) {
-    const int stride = fw ? 60 : 66;
-    const cx<T> *base = fw ? fwd : bwd;
-#pragma unroll
-    for (int gg = 0; gg < G; gg++) {
-      const long r = line_of(gg) * n + r0;
-      copy_rows_to_lds(base + r * stride, (L * n - r) * stride, rec[kk][gg], nr * stride, wave - 1, 3, lane);
-    }
-    for (int t = tid - 64; t < G * nr * 5; t += 192) {
-      const int gg = t / (nr * 5), rem = t - gg * nr * 5, row = rem / 5, mm = rem - row * 5;
-      const long ln = line_of(gg), ri = ln * n + r0 + row;
-      const double2 *xr = rhs + ln * sL * 5 + (long)(r0 + row) * rs;
-      cx<T> acc{0, 0};
-      if (fw) {
-        const cx<T> *Li = fwd + ri * 60 + 50 + mm * (mm - 1) / 2;
-        acc = zx(xr[mm]);
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (q < mm) acc = cfma(Li[q], zx(xr[q]), acc);
-      } else {
-        const cx<T> *Ui = bwd + ri * 66 + 50 + mm * 5 - mm * (mm - 1) / 2;
-#pragma unroll
-        for (int q = 0; q < 5; q++)
-          if (q < 5 - mm) acc = cfma(Ui[q], zx(xr[mm + q]), acc);
-        if (border) {
-          const cx<T> *Q = qp + ri * 50 + mm * 5;
-#pragma unroll
-          for (int q = 0; q < 5; q++) acc = cfma(Q[q], xb[gg][0][q], acc);
-#pragma unroll
-          for (int q = 0; q < 5; q++) acc = cfma(Q[25 + q], xb[gg][1][q], acc);
-        }
-      }
-      cb[kk][gg][row][mm] = acc;
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-  };
-  // loader threads keep partial forward border sums of (line gg, border row
-  // bt, component mm) over the rows the compute wave finished: NSUB threads
-  // per sum, each taking every NSUB-th row of a chunk
-  const int at = tid - 64;
-  const bool acc_thread = at >= 0 && at < NSUB * 10 * G;
-  const int aid = acc_thread ? at % (10 * G) : 0, asub = acc_thread ? at / (10 * G) : 0;
-  const int agg = aid / 10, abt = (aid / 5) % 2, amm = aid % 5;
-  cx<T> bacc{0, 0};
-  auto accumulate = [&](int r0, int nr) {
-    if (!acc_thread) return;
-    const long ln = line_of(agg);
-    for (int row = asub; row < nr; row += NSUB) {
-      const long ri = ln * n + r0 + row;
-      const double2 *yr = rhs + ln * sL * 5 + (long)(r0 + row) * rs;
-      const cx<T> *P = p2 + ri * 50 + abt * 25 + amm * 5;
-#pragma unroll
-      for (int q = 0; q < 5; q++) bacc = cfma(P[q], zx(yr[q]), bacc);
-    }
-  };
-
-  // ---- compute wave
-  cx<T> yA[5], yB[5];
-  cx<T> w2s[3][5], w1s[3][5], cs[3];
-  // the term in the newest value: two FMA accumulators (four independent
-  // chains over re and im), 22 instructions
-  auto crit = [&](const cx<T> (&w)[5], const cx<T> (&yn)[5], cx<T> a0) -> cx<T> {
-    cx<T> a = cfma(w[0], yn[0], a0), b = cmul(w[1], yn[1]);
-    a = cfma(w[2], yn[2], a);
-    b = cfma(w[3], yn[3], b);
-    a = cfma(w[4], yn[4], a);
-    return a + b;
-  };
-  auto pre0 = [&](const cx<T> (&w)[5], cx<T> c, const cx<T> (&yo)[5]) -> cx<T> {
-    cx<T> a = cfma(w[0], yo[0], c), b = cmul(w[1], yo[1]);
-    a = cfma(w[2], yo[2], a);
-    b = cfma(w[3], yo[3], b);
-    a = cfma(w[4], yo[4], a);
-    return a + b;
-  };
-  // rows of buffer kk in processing order j (buffer row = j forward,
-  // nr-1-j backward); extra(j) is added to the row's known part
-  // two rows on the plain path: the border rows of either pass; extra adds
-  // the forward border sums
-  auto border_rows = [&](int kk, int ibase, bool fw, bool extra) {
-    const int stride = fw ? 60 : 66;
-    const cx<T> *B = rec[kk][g];
-    for (int j = 0; j < 2; j++) {
-      const int r = fw ? j : 1 - j;
-      cx<T> w1[5], w2[5];
-#pragma unroll
-      for (int q = 0; q < 5; q++) { w2[q] = B[r * stride + m * 10 + q]; w1[q] = B[r * stride + m * 10 + 5 + q]; }
-      cx<T> a = pre0(w1, cb[kk][g][r][m], yA);
-      if (extra) a = a + bsum[g][j][m];
-      cx<T> y = crit(w2, yB, a);
-      X[(long)(fw ? ibase + j : ibase - j) * rs + m] = make_double2(y.re, y.im);
-      row_bcast5(y, yA);
-#pragma unroll
-      for (int q = 0; q < 5; q++) { cx<T> t = yA[q]; yA[q] = yB[q]; yB[q] = t; }
-    }
-  };
-  auto run_chunk = [&](int kk, int nr, int ibase, bool fw) {
-    const int stride = fw ? 60 : 66;
-    const cx<T> *B = rec[kk][g];
-    auto rix = [&](int j) { j = min(j, nr - 1); return fw ? j : nr - 1 - j; };
-    auto ldW2 = [&](int j, cx<T> (&w)[5]) {
-      const cx<T> *pp = B + rix(j) * stride + m * 10;
-#pragma unroll
-      for (int q = 0; q < 5; q++) w[q] = pp[q];
-    };
-    auto ldW1 = [&](int j, cx<T> (&w)[5], cx<T> &c) {
-      const int r = rix(j);
-      const cx<T> *pp = B + r * stride + m * 10 + 5;
-#pragma unroll
-      for (int q = 0; q < 5; q++) w[q] = pp[q];
-      c = cb[kk][g][r][m];
-    };
-    const long xstep = fw ? rs : -rs;
-    double2 *xp = X + (long)(fw ? ibase : ibase) * rs + m;
-    const int nmain = (nr / 6) * 6;
-    if (nmain > 0) {
-      ldW2(0, w2s[0]);
-      ldW2(1, w2s[1]);
-      ldW1(0, w1s[0], cs[0]);
-      ldW1(1, w1s[1], cs[1]);
-      ldW1(2, w1s[2], cs[2]);
-      cx<T> a0 = pre0(w1s[0], cs[0], yA);
-      auto sub = [&](int j, auto U) {
-        constexpr int u = decltype(U)::value;
-        constexpr int u0 = u % 3, u1 = (u + 1) % 3, u2 = (u + 2) % 3;
-        cx<T>(&yn)[5] = (u % 2 == 0) ? yB : yA;
-        cx<T>(&yd)[5] = (u % 2 == 0) ? yA : yB;
-        cx<T> y = crit(w2s[u0], yn, a0);
-        a0 = pre0(w1s[u1], cs[u1], yn);
-        *xp = make_double2(y.re, y.im);
-        xp += xstep;
-        ldW2(j + 2, w2s[u2]);
-        ldW1(j + 3, w1s[u0], cs[u0]);
-        row_bcast5(y, yd);
-      };
-      for (int j = 0; j < nmain; j += 6) {
-        sub(j, std::integral_constant<int, 0>());
-        sub(j + 1, std::integral_constant<int, 1>());
-        sub(j + 2, std::integral_constant<int, 2>());
-        sub(j + 3, std::integral_constant<int, 3>());
-        sub(j + 4, std::integral_constant<int, 4>());
-        sub(j + 5, std::integral_constant<int, 5>());
-      }
-    }
-    for (int j = nmain; j < nr; j++) {
-      cx<T> w1[5], w2[5], c;
-      ldW1(j, w1, c);
-      ldW2(j, w2);
-      cx<T> y = crit(w2, yB, pre0(w1, c, yA));
-      *xp = make_double2(y.re, y.im);
-      xp += xstep;
-      row_bcast5(y, yA);
-#pragma unroll
-      for (int q = 0; q < 5; q++) { cx<T> t = yA[q]; yA[q] = yB[q]; yB[q] = t; }
-    }
-  };
-
-  // ================= forward
-#pragma unroll
-  for (int q = 0; q < 5; q++) { yA[q] = cx<T>{0, 0}; yB[q] = cx<T>{0, 0}; }
-  if (wave != 0) load(0, 0, min(R, nreg), true, false);
-  __syncthreads();
-  for (int k = 0; k < nck; k++) {
-    const int r0 = k * R, nr = min(R, nreg - r0);
-    if (wave == 0) {
-      run_chunk(k & 1, nr, r0, true);
-    } else {
-      if (k >= 1) accumulate(r0 - R, R);
-      if (k + 1 < nck) load((k + 1) & 1, r0 + R, min(R, nreg - r0 - R), true, false);
-    }
-    __syncthreads();
-  }
-  // the last regular chunk's sums, the records of rows n-2, n-1
-  if (wave != 0) {
-    const int r0 = (nck - 1) * R;
-    accumulate(r0, nreg - r0);
-    if (acc_thread) bpart[asub][aid] = bacc;
-    load(nck & 1, nreg, 2, true, false);
-  }
-  __syncthreads();
-  if (tid >= 64 && tid < 64 + 10 * G) {
-    const int id = tid - 64;
-    cx<T> t{0, 0};
-    for (int k = 0; k < NSUB; k++) t = t + bpart[k][id];
-    bsum[id / 10][(id / 5) % 2][id % 5] = t;
-  }
-  __syncthreads();
-  if (wave == 0) border_rows(nck & 1, nreg, true, true);
-  __syncthreads();
-
-  // ================= backward
-#pragma unroll
-  for (int q = 0; q < 5; q++) { yA[q] = cx<T>{0, 0}; yB[q] = cx<T>{0, 0}; }
-  if (wave != 0) load(0, nreg, 2, false, false);
-  __syncthreads();
-  if (wave == 0) {
-    border_rows(0, n - 1, false, false);
-    // x_{n-1} is yA, x_{n-2} is yB (all components on every lane); pick
-    // component m with constant indices (a runtime index would move the
-    // arrays out of registers)
-    cx<T> xa = yB[0], xc = yA[0];
-#pragma unroll
-    for (int q = 1; q < 5; q++)
-      if (m == q) { xa = yB[q]; xc = yA[q]; }
-    if ((lane & 15) < 5) { xb[g][0][m] = xa; xb[g][1][m] = xc; }
-  }
-  __syncthreads();
-  if (wave != 0) {
-    const int rtop = nreg - 1, nr = min(R, rtop + 1);
-    load(1, rtop - nr + 1, nr, false, true);
-  }
-  __syncthreads();
-  for (int k = 1; k <= nck; k++) {
-    const int rtop = nreg - 1 - (k - 1) * R, nr = min(R, rtop + 1);
-    if (wave == 0) {
-      run_chunk(k & 1, nr, rtop, false);
-    } else if (k < nck) {
-      const int rt2 = rtop - nr, nr2 = min(R, rt2 + 1);
-      load((k + 1) & 1, rt2 - nr2 + 1, nr2, false, true);
-    }
-    __syncthreads();
-  }
-  // x(np) = x(1)
-  if (wave == 0 && (lane & 15) < 5) X[(long)n * rs + m] = X[m];
-}
-template <typename T, int R, int G>
-__global__ __launch_bounds__(256) void k_solve_per(int n, long L, const cx<T> *__restrict__ fwd,
-                                                  const cx<T> *__restrict__ bwd,
-                                                  const cx<T> *__restrict__ p2,
-                                                  const cx<T> *__restrict__ qp, double2 *rhs,
-                                                  long sL, long sR) {
-  solve_per<T, R, G>(blockIdx.x, n, L, fwd, bwd, p2, qp, rhs, sL, sR);
 }
 
 // ---------------------------------------------------------------------------
@@ -1657,7 +1296,21 @@ template <typename F> static auto with_line_form(int form, int prec, bool tw, F 
     default: return prec ? fam(float{}, LineForm<6, 4, false>()) : fam(double{}, LineForm<6, 4, false>());
   }
 }
-static unsigned line_lds(int form, int prec, bool tw, int n) {
+// the same for periodic lines, which have six of them
+template <typename F> static auto with_per_form(int form, int prec, F f) {
+  switch (form) {
+    case LINES_RES6: return prec ? f(float{}, LineForm<6, 4, true>()) : f(double{}, LineForm<6, 4, true>());
+    case LINES_RES3: return f(double{}, LineForm<3, 4, true>());
+    case LINES_RES12: return f(float{}, LineForm<12, 4, true>());
+    case LINES_RING12: return f(float{}, LineForm<12, 4, false>());
+    default: return f(double{}, LineForm<6, 4, false>());
+  }
+}
+static unsigned line_lds(int form, int prec, bool tw, int n, bool per = false) {
+  if (per)
+    return with_per_form(form, prec, [&](auto t, auto lf) {
+      return LineSolve<decltype(t), lf.R, lf.NBUF, false, lf.RES, true>::lds_bytes(n);
+    });
   return with_line_form(form, prec, tw, [&](auto t, auto lf, auto TW) {
     return LineSolve<decltype(t), lf.R, lf.NBUF, TW.value, lf.RES>::lds_bytes(n);
   });
@@ -1698,6 +1351,23 @@ static int line_form(int variant, int n, long lines, int prec, bool tw) {
   return tw && fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING3;
 }
 
+// The form of periodic lines, two per workgroup: resident right-hand sides
+// while one workgroup per CU holds every line and its LDS them (they spare
+// 160 of 3920 bytes a row); with more lines the chunks of half the rows, of
+// which two workgroups fit a CU (up to about 100 rows; the prologues of short
+// lines overlap then: 1025 lines of 33 rows 47 us, with six-row chunks 58);
+// rings of twelve (complex float) or six rows else.
+static int per_form(int n, long lines, int prec) {
+  auto fit = [&](int form) { return (int)(LDS_PER_CU / line_lds(form, prec, false, n, true)); };
+  const int res = prec ? LINES_RES12 : LINES_RES6, small = prec ? LINES_RES6 : LINES_RES3;
+  if ((lines + 1) / 2 <= 256) {
+    if (fit(res) >= 1) return res;
+  } else if (fit(small) >= 2) {
+    return small;
+  }
+  return prec ? LINES_RING12 : LINES_RING6;
+}
+
 // a kernel's dynamic LDS above the default 64 KB has to be asked for
 template <typename K> static int allow_lds(K k, unsigned lds) {
   if (lds > 64 * 1024)
@@ -1721,28 +1391,23 @@ static int launch_line_solve(const PentaPlan *pl, void *rhs, long sL, long sR, h
   });
 }
 
-int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
-  LineGeom g{pl->n, pl->periodic, pl->exact, pl->L};
-  if (pl->periodic) {
-    (void)g;
-    auto per = [&](auto tag) {
-      using T = decltype(tag);
-      auto *f = (const cx<T> *)pl->fwd; auto *b = (const cx<T> *)pl->bwd;
-      auto *p2 = (const cx<T> *)pl->p2; auto *qp = (const cx<T> *)pl->qp;
-      // one line per workgroup while two workgroups per CU hold every line
-      if (pl->L > 512)
-        hipLaunchKernelGGL((k_solve_per<T, 6, 4>), dim3((unsigned)((pl->L + 3) / 4)), dim3(256), 0, s, pl->n, pl->L,
-                           f, b, p2, qp, (double2 *)rhs, sL, sR);
-      else
-        hipLaunchKernelGGL((k_solve_per<T, 30, 1>), dim3((unsigned)pl->L), dim3(256), 0, s, pl->n, pl->L, f, b, p2,
-                           qp, (double2 *)rhs, sL, sR);
-    };
-    if (pl->prec) per(float{});
-    else per(double{});
-  } else {
-    const int rc = launch_line_solve(pl, rhs, sL, sR, s);
+static int launch_per_solve(const PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
+  const int form = per_form(pl->n, pl->L, pl->prec);
+  return with_per_form(form, pl->prec, [&](auto t, auto lf) {
+    using T = decltype(t);
+    auto k = k_line_solve_per<T, lf.R, lf.NBUF, lf.RES>;
+    const unsigned lds = line_lds(form, pl->prec, false, pl->n, true);
+    const int rc = allow_lds(k, lds);
     if (rc) return rc;
-  }
+    hipLaunchKernelGGL(k, dim3((unsigned)((pl->L + 1) / 2)), dim3(256), lds, s, pl->n, pl->L, (const cx<T> *)pl->fwd,
+                       (const cx<T> *)pl->bwd, (const cx<T> *)pl->p2, (const cx<T> *)pl->qp, (double2 *)rhs, sL, sR);
+    return 0;
+  });
+}
+
+int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
+  const int rc = pl->periodic ? launch_per_solve(pl, rhs, sL, sR, s) : launch_line_solve(pl, rhs, sL, sR, s);
+  if (rc) return rc;
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
@@ -1772,21 +1437,19 @@ __global__ __launch_bounds__(256, 2) void kb_line_solve(const PentaBatchItem *it
                                       (const cx<T> *)b.bwd, (const cx<T> *)b.tail, b.rhs[which], b.sL, b.sR);
 }
 
-template <typename T, int R, int G>
-__global__ __launch_bounds__(256) void kb_solve_per(const PentaBatchItem *items, const int *off, int count,
-                                                   int which) {
+template <typename T, int R, int NBUF, bool RES>
+__global__ __launch_bounds__(256, 2) void kb_line_solve_per(const PentaBatchItem *items, const int *off, int count,
+                                                           int which) {
+  extern __shared__ __attribute__((aligned(16))) char sm[];
   const int k = batch_member(off, count);
   const PentaBatchItem &b = items[k];
-  solve_per<T, R, G>((long)blockIdx.x - off[k], b.n, b.L, (const cx<T> *)b.fwd, (const cx<T> *)b.bwd,
-                     (const cx<T> *)b.p2, (const cx<T> *)b.qp, b.rhs[which], b.sL, b.sR);
+  LineSolve<T, R, NBUF, false, RES, true>::run(sm, (long)blockIdx.x - off[k], b.n, -1, b.L, (const cx<T> *)b.fwd,
+                                               (const cx<T> *)b.bwd, nullptr, b.rhs[which], b.sL, b.sR,
+                                               (const cx<T> *)b.p2, (const cx<T> *)b.qp);
 }
 
-// batch groups of periodic lines, by their solve kernel (as penta_solve
-// chooses it: four lines per workgroup above 512 lines, else one)
-constexpr int BATCH_PERIODIC1 = 1001, BATCH_PERIODIC4 = 1004;
-
 // lines per workgroup of a batch group's solve kernel
-static int group_lines(const PentaBatchGroup &g) { return g.form < 0 ? (g.variant == BATCH_PERIODIC4 ? 4 : 1) : g.tw ? 1 : 2; }
+static int group_lines(const PentaBatchGroup &g) { return g.tw ? 1 : 2; }
 
 int stage_upload(void *dev, const void *src, size_t bytes, std::vector<TableUpload> &ups) {
   void *h = nullptr;
@@ -1802,13 +1465,12 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
   out.clear();
   long lines = 0;              // solved by one launch or another at a time
   for (int k = 0; k < count; k++) lines += plans[k]->L;
-  // members that share a kernel: periodic lines by their kernel, the others
-  // by form and family (form -1: periodic)
-  std::map<std::tuple<int, int, int, int>, std::vector<int>> by;   // (form, variant of periodic lines, twisted, precision)
+  // members that share a kernel: by form, family and precision
+  std::map<std::tuple<int, int, int, int>, std::vector<int>> by;   // (form, periodic, twisted, precision)
   for (int k = 0; k < count; k++) {
     const PentaPlan *pl = plans[k];
     const bool tw = pl->h >= 0;
-    if (pl->periodic) by[{-1, pl->L > 512 ? BATCH_PERIODIC4 : BATCH_PERIODIC1, 0, pl->prec}].push_back(k);
+    if (pl->periodic) by[{per_form(pl->n, lines, pl->prec), 1, 0, pl->prec}].push_back(k);
     else by[{line_form(pl->variant, pl->n, lines, pl->prec, tw), 0, tw, pl->prec}].push_back(k);
   }
   for (auto &kv : by) {
@@ -1818,7 +1480,7 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
                      [&](int a, int b) { return plans[a]->n > plans[b]->n; });
     PentaBatchGroup g;
     g.form = std::get<0>(kv.first);
-    g.variant = std::get<1>(kv.first);
+    g.per = std::get<1>(kv.first);
     g.tw = std::get<2>(kv.first);
     g.prec = std::get<3>(kv.first);
     g.count = (int)kv.second.size();
@@ -1841,7 +1503,7 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
       it.sR = sR[k];
       items.push_back(it);
       const long wg = (pl->L + group_lines(g) - 1) / group_lines(g);
-      if (g.form >= 0) g.lds = std::max(g.lds, line_lds(g.form, g.prec, g.tw, pl->n));
+      g.lds = std::max(g.lds, line_lds(g.form, g.prec, g.tw, pl->n, g.per));
       if ((long)off.back() + wg > 0x7fffffffL) return set_error(__FILE__, __LINE__, "batch too large");
       off.push_back(off.back() + (int)wg);
     }
@@ -1867,24 +1529,19 @@ void penta_batch_free(std::vector<PentaBatchGroup> &groups) {
 static int launch_batch_group(const PentaBatchGroup &g, int which, hipStream_t s) {
   const auto *it = (const PentaBatchItem *)g.items;
   const dim3 grid((unsigned)g.blocks), blk(256);
-  if (g.form >= 0)
-    return with_line_form(g.form, g.prec, g.tw, [&](auto t, auto lf, auto TW) {
-      auto k = kb_line_solve<decltype(t), lf.R, lf.NBUF, TW.value, lf.RES>;
-      const int rc = allow_lds(k, g.lds);
-      if (rc) return rc;
-      hipLaunchKernelGGL(k, grid, blk, g.lds, s, it, g.off, g.count, which);
-      return 0;
-    });
-  auto per = [&](auto t) {
-    using T = decltype(t);
-    if (g.variant == BATCH_PERIODIC4)
-      hipLaunchKernelGGL((kb_solve_per<T, 6, 4>), grid, blk, 0, s, it, g.off, g.count, which);
-    else
-      hipLaunchKernelGGL((kb_solve_per<T, 30, 1>), grid, blk, 0, s, it, g.off, g.count, which);
+  auto launch = [&](auto k) {
+    const int rc = allow_lds(k, g.lds);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k, grid, blk, g.lds, s, it, g.off, g.count, which);
+    return 0;
   };
-  if (g.prec) per(float{});
-  else per(double{});
-  return 0;
+  if (g.per)
+    return with_per_form(g.form, g.prec, [&](auto t, auto lf) {
+      return launch(kb_line_solve_per<decltype(t), lf.R, lf.NBUF, lf.RES>);
+    });
+  return with_line_form(g.form, g.prec, g.tw, [&](auto t, auto lf, auto TW) {
+    return launch(kb_line_solve<decltype(t), lf.R, lf.NBUF, TW.value, lf.RES>);
+  });
 }
 
 int penta_batch_solve(const std::vector<PentaBatchGroup> &groups, int which, hipStream_t s) {

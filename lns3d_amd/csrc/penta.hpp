@@ -48,8 +48,8 @@ struct PentaBatchItem {
 };
 // the members of a batch that share a solve kernel; device tables
 struct PentaBatchGroup {
-  int form = -1;           // form of the line solve; -1: periodic lines
-  int variant = 0;         // periodic lines: their kernel
+  int form = 0;            // form of the line solve
+  int per = 0;             // periodic lines
   int tw = 0, prec = 0, count = 0;
   unsigned lds = 0;        // the most a member needs
   long blocks = 0;
