@@ -134,10 +134,10 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
   static constexpr unsigned CS = sizeof(cx<T>);
   static constexpr unsigned CHB = R * 66 * CS, BUFB = 2 * CHB;   // a chunk's records: one chain, both
   // boundary blocks of a pass; PER: of both lines, the records of rows n-2
-  // and n-1 (60 and 66 values a row), their right-hand sides (80 bytes a
+  // (60 and 66 values) and n-1 (60, and 16 without its recurrence), their right-hand sides (80 bytes a
   // row), the border sums (20 values) and the waves' shares of them
-  static constexpr unsigned TAIL = NBUF * BUFB, BREC = 2 * 2 * 126 * CS, BSUM = BREC + 4 * 80, BPART = BSUM + 20 * CS,
-                            TAILB = PER ? (BPART + 200 * CS + 15) & ~15u : (150 * CS + 15) & ~15u;
+  static constexpr unsigned TAIL = NBUF * BUFB, BREC = 2 * 202 * CS, BSUM = BREC + 4 * 80, BPART = BSUM + 20 * CS,
+                            TAILB = PER ? (BPART + 400 * CS + 15) & ~15u : (150 * CS + 15) & ~15u;
   static constexpr unsigned SV = TAIL + TAILB, SVB = (20 * CS + 15) & ~15u;       // rows kept for them
   static constexpr unsigned ROWB = 80;                           // a right-hand-side row
   static constexpr unsigned ZERO = SV + SVB, DUMMY = ZERO + R * ROWB;
@@ -145,7 +145,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
   static constexpr unsigned ROWS = BORD + NROW * 2 * BORDB;      // right-hand-side rows
   // rows of a resident right-hand side: a twisted line's inactive steps
   // touch one row before chain 1 and three after it
-  static __host__ __device__ unsigned rows(int n) { return RES ? (TW ? n + 4 : 2 * n) : NROW * 2 * R; }
+  static __host__ __device__ unsigned rows(int n) { return RES ? (TW ? n + 4 : PER ? 2 * (n - 2) : 2 * n) : NROW * 2 * R; }
   static __host__ __device__ unsigned lds_bytes(int n) { return ROWS + rows(n) * ROWB; }
 
   static __device__ __forceinline__ void run(char *sm, long bid, int n, int h, long L, const cx<T> *__restrict__ fwd,
@@ -258,18 +258,18 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
       auto load_tail = [&](bool fw) {                  // boundary blocks of a pass
         if constexpr (PER) {
           if (!fw) return;                             // both passes' at the start
-          cx<T> v[8];
+          cx<T> v[7];
           const int e20 = min(lane, 19);
           const double2 b = rhs[(line_of(e20 / 10) * sL + (long)(n + e20 / 5 % 2) * sR) * 5 + e20 % 5];
 #pragma unroll
-          for (int i = 0; i < 8; i++) {                // line, row, value
-            const int e = min(i * 64 + lane, 503), c = e / 252, r = e / 126 % 2, k = e % 126;
+          for (int i = 0; i < 7; i++) {                // line, row, value
+            const int e = min(i * 64 + lane, 403), c = e / 202, r = e % 202 >= 126, k = e % 202 - 126 * r;
             const long row = line_of(c) * nmem + n + r;
-            v[i] = *(k < 60 ? fwd + (row * 60 + k) : bwd + (row * 66 + k - 60));
+            v[i] = *(k < 60 ? fwd + (row * 60 + k) : bwd + (row * 66 + k - 60 + 50 * r));
           }
 #pragma unroll
-          for (int i = 0; i < 8; i++)
-            if (i * 64 + lane < 504) reinterpret_cast<cx<T> *>(sm + TAIL)[i * 64 + lane] = v[i];
+          for (int i = 0; i < 7; i++)
+            if (i * 64 + lane < 404) reinterpret_cast<cx<T> *>(sm + TAIL)[i * 64 + lane] = v[i];
           if (lane < 20) *reinterpret_cast<double2 *>(sm + (TAIL + BREC + lane * 16)) = b;
           return;
         }
@@ -285,23 +285,36 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
       };
       // PER, forward: the border sums of a finished chunk.  Lane e of 50 takes
       // entry e of every row's p2 (border row, component, column e % 5) and
-      // sums its product with the row's y; the columns are added at the end
-      cx<T> bacc[2] = {{0, 0}, {0, 0}};
+      // sums its product with the row's y.  Rows are summed in four classes,
+      // (row / G) % 4 with G the shortest chunk of the precision, a class by
+      // one wave; classes and columns are added at the end: so all forms of
+      // the kernel round alike
+      constexpr int G = sizeof(T) == 8 ? 3 : 6;
+      static_assert(!PER || R == G || R == 2 * G, "a wave's chunks hold two classes");
+      cx<T> bacc[2][2] = {{{0, 0}, {0, 0}}, {{0, 0}, {0, 0}}};      // the wave's classes, the lines
       auto border_sum = [&](int k, int rb) {
         if constexpr (PER) {
           const int e = min(lane, 49), nr = min(R, n - k * R);
-#pragma unroll
-          for (int c = 0; c < 2; c++) {
-            const char *row = sm + (row_off(rb, c, k * R) + e % 5 * 16);
-            const cx<T> *blk = reinterpret_cast<const cx<T> *>(sm + (BORD + (rb * 2 + c) * BORDB)) + e;
-            if (nr == R) {
-#pragma unroll
-              for (int u = 0; u < R; u++)
-                bacc[c] = cfma(blk[u * 50], *reinterpret_cast<const cx<T> *>(row + u * ROWB), bacc[c]);
-            } else {
-              for (int u = 0; u < nr; u++)
-                bacc[c] = cfma(blk[u * 50], *reinterpret_cast<const cx<T> *>(row + u * ROWB), bacc[c]);
-            }
+          const char *row = sm + (row_off(rb, 0, k * R) + e % 5 * 16);
+          const char *row1 = sm + (row_off(rb, 1, k * R) + e % 5 * 16);
+          const cx<T> *blk = reinterpret_cast<const cx<T> *>(sm + (BORD + rb * 2 * BORDB)) + e;
+          auto add = [&](auto H, int u) {              // row u of both lines, class H of the wave
+            cx<T>(&acc)[2] = bacc[decltype(H)::value];
+            acc[0] = cfma(blk[u * 50], *reinterpret_cast<const cx<T> *>(row + u * ROWB), acc[0]);
+            acc[1] = cfma(blk[u * 50 + R * 50], *reinterpret_cast<const cx<T> *>(row1 + u * ROWB), acc[1]);
+          };
+          if (R == 2 * G) {
+            if (nr == R)
+              static_for<R>([&](auto U) { add(idx_t<(decltype(U)::value >= G)>(), decltype(U)::value); });
+            else
+              for (int u = 0; u < nr; u++) {
+                if (u < G) add(idx_t<0>(), u);
+                else add(idx_t<1>(), u);
+              }
+          } else if ((k >> 1) & 1) {
+            for (int u = 0; u < nr; u++) add(idx_t<1>(), u);
+          } else {
+            for (int u = 0; u < nr; u++) add(idx_t<0>(), u);
           }
         }
       };
@@ -313,15 +326,15 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           auto *bs = reinterpret_cast<cx<T> *>(sm + TAIL + BSUM);
           const auto *part = reinterpret_cast<const cx<T> *>(sm + TAIL + BPART);
           if (lane < 20) {
-            cx<T> t{0, 0};                             // over two waves and five columns
+            cx<T> t{0, 0};                             // over four classes and five columns
 #pragma unroll 1
-            for (int k = 0; k < 10; k++) t = t + part[k / 5 * 100 + lane * 5 + k % 5];
+            for (int k = 0; k < 20; k++) t = t + part[k / 5 * 100 + lane * 5 + k % 5];
             bs[lane] = t;
           }
           wave_sync();
           const int c = min(lane / 5, 1), mm = lane % 5;
           auto *xs = reinterpret_cast<cx<T> *>(sm + SV) + c * 10;      // y_{n-3}, y_{n-4}; then x_{n-2}, x_{n-1}
-          const auto *rec = reinterpret_cast<const cx<T> *>(sm + TAIL) + c * 252;
+          const auto *rec = reinterpret_cast<const cx<T> *>(sm + TAIL) + c * 202;
           auto entry = [&](const cx<T> *r, int older, int q) {
             const T *w = reinterpret_cast<const T *>(r) + mm * 20 + rec_pos(older, q);
             return cx<T>{w[0], w[10]};
@@ -335,7 +348,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
             return acc;
           };
           auto uinv = [&](int r, const cx<T> *y) {
-            const cx<T> *U = rec + r * 126 + 110 + mm * 5 - mm * (mm - 1) / 2;
+            const cx<T> *U = rec + (r ? 186 : 110) + mm * 5 - mm * (mm - 1) / 2;
             cx<T> acc{0, 0};
 #pragma unroll 1
             for (int q = mm; q < 5; q++) acc = cfma(U[q - mm], y[q], acc);
@@ -505,7 +518,10 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
             const int last = ((N - 1) & 1) == p ? N - 1 : N - 2;
             if (last >= 0) border_sum(last, last % NROW);
             if (lane < 50)
-              for (int c = 0; c < 2; c++) reinterpret_cast<cx<T> *>(sm + TAIL + BPART)[p * 100 + c * 50 + lane] = bacc[c];
+              for (int h = 0; h < 2; h++)
+                for (int c = 0; c < 2; c++)
+                  reinterpret_cast<cx<T> *>(sm + TAIL + BPART)[(R == G ? p + 2 * h : 2 * p + h) * 100 + c * 50 + lane] =
+                      bacc[h][c];
             loader_barrier();
             if (p == 0) border_rows();
             loader_barrier();
