@@ -632,9 +632,10 @@ extern "C" int lns3d_ctx_set_residual_output(lns3d_ctx *c, double *norms_dev, in
   return 0;
 }
 
-static int solve_xy(lns3d_ctx *c, PentaPlan &px, PentaPlan &py, void *r) {
+// both directions' solves of r, in place, or of `in` with the solution in r
+static int solve_xy(lns3d_ctx *c, PentaPlan &px, PentaPlan &py, void *r, const void *in = nullptr) {
   // xi lines: line j, row i at (i + nx*j); eta lines: line i, row j
-  int rc = penta_solve(&px, r, c->p.nx, 1, c->stream);
+  int rc = penta_solve(&px, r, c->p.nx, 1, c->stream, in);
   if (!rc) rc = penta_solve(&py, r, 1, c->p.nx, c->stream);
   return rc;
 }
@@ -803,17 +804,14 @@ extern "C" int lns3d_step_refined(lns3d_ctx *c, void *v_dev, void *dv_dev, doubl
   int rc = refactor_for(c, 1);
   if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, rhs, 1, c->stream);
   if (rc) return rc;
-  rc = launch_copy(dv, rhs, n, c->stream);
-  if (rc) return rc;
-  rc = solve_xy(c, c->px32, c->py32, dv);
+  rc = solve_xy(c, c->px32, c->py32, dv, rhs);
   if (rc) return rc;
   // max_iters <= 0: no caller limit; the loop still stops after 64 solves
   const int cap = max_iters > 0 ? max_iters : 64;
   int it = 1;
   double nr[2] = {0, 0};
   for (;; it++) {
-    rc = launch_af_matvec(c->p, c->c, dv, c->t2, c->t1, c->stream);       // t2 = M dv
-    if (!rc) rc = launch_residual_norms(rhs, c->t2, n, c->scal + 8, c->stream);   // t2 = rhs - M dv
+    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, c->scal + 8, c->stream);   // t2 = rhs - M dv
     if (rc) return rc;
     LNS3D_CHECK(hipMemcpyAsync(nr, c->scal + 8, 16, hipMemcpyDeviceToHost, c->stream));
     LNS3D_CHECK(hipStreamSynchronize(c->stream));
@@ -865,20 +863,17 @@ extern "C" int lns3d_step_refined_fixed(lns3d_ctx *c, void *v_dev, void *dv_dev,
   int rc = refactor_for(c, 1);
   if (!rc) rc = launch_rhs(c->p, c->st, c->c, v_dev, rhs, 1, c->stream);
   if (!rc) rc = record_norm(c, rhs);
-  if (!rc) rc = launch_copy(dv, rhs, n, c->stream);
-  if (!rc) rc = solve_xy(c, c->px32, c->py32, dv);
+  if (!rc) rc = solve_xy(c, c->px32, c->py32, dv, rhs);
   // the last correction is added with the update of v, unless the check's
   // residual needs dv whole before it
   const void *last = corrections > 0 && !check ? c->t2 : nullptr;
   for (int k = 0; k < corrections && !rc; k++) {
-    rc = launch_af_matvec(c->p, c->c, dv, c->t2, c->t1, c->stream);
-    if (!rc) rc = launch_residual_norms(rhs, c->t2, n, c->scal + 8, c->stream);
+    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, c->scal + 8, c->stream);
     if (!rc) rc = solve_xy(c, c->px32, c->py32, c->t2);
     if (!rc && (k < corrections - 1 || !last)) rc = launch_axpy(dv, c->t2, n, c->stream);
   }
   if (!rc && check) {
-    rc = launch_af_matvec(c->p, c->c, dv, c->t2, c->t1, c->stream);
-    if (!rc) rc = launch_residual_norms(rhs, c->t2, n, c->scal + 8, c->stream);
+    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, c->scal + 8, c->stream);
   }
   if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, dv, last, c->stream);
   if (!rc) c->lstep++;
@@ -955,6 +950,7 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
   std::vector<StepBatchMember> m((size_t)count);
   std::vector<const PentaPlan *> px((size_t)count), py((size_t)count);
   std::vector<double2 *> r0((size_t)count), r1((size_t)count);
+  std::vector<const double2 *> in((size_t)count);
   std::vector<long> sx1((size_t)count), sx2((size_t)count), sy1((size_t)count), sy2((size_t)count);
   for (int i = 0; i < count; i++) {
     lns3d_ctx *c = ctxs[i];
@@ -972,6 +968,7 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
     a.norm_idx = c->norm_idx;
     px[(size_t)i] = &c->px32;
     py[(size_t)i] = &c->py32;
+    in[(size_t)i] = a.rhs;      // the xi solve reads the residual and leaves dv
     r0[(size_t)i] = a.dv;
     r1[(size_t)i] = a.t2;
     sx1[(size_t)i] = c->p.nx;   // xi lines: line j, row i at (i + nx j)
@@ -981,8 +978,8 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
   }
   int rc = hipStreamCreateWithFlags(&gr->s, hipStreamNonBlocking) != hipSuccess ? fail(LNS3D_EHIP, "stream") : 0;
   if (!rc) rc = step_batch_build(m.data(), count, gr->sb, gr->ups);
-  if (!rc) rc = penta_batch_build(px.data(), r0.data(), r1.data(), sx1.data(), sx2.data(), count, gr->gx, gr->ups);
-  if (!rc) rc = penta_batch_build(py.data(), r0.data(), r1.data(), sy1.data(), sy2.data(), count, gr->gy, gr->ups);
+  if (!rc) rc = penta_batch_build(px.data(), in.data(), r0.data(), r1.data(), sx1.data(), sx2.data(), count, gr->gx, gr->ups);
+  if (!rc) rc = penta_batch_build(py.data(), r0.data(), r0.data(), r1.data(), sy1.data(), sy2.data(), count, gr->gy, gr->ups);
   if (!rc && hipEventCreateWithFlags(&gr->up_ev, hipEventDisableTiming) != hipSuccess) rc = fail(LNS3D_EHIP, "event");
   if (!rc && hipStreamBeginCapture(gr->s, hipStreamCaptureModeThreadLocal) != hipSuccess)
     rc = fail(LNS3D_EHIP, "hipStreamBeginCapture");
@@ -994,15 +991,13 @@ static int graph_create_batched(lns3d_ctx **ctxs, void **v_dev, void **dv_dev, i
   for (int k = 0; k < nsteps && !rc; k++) {
     rc = step_batch_rhs(gr->sb, s);
     if (!rc) rc = step_batch_norm(gr->sb, k, s);
-    if (!rc) rc = step_batch_vec(gr->sb, SB_COPY, s);
     if (!rc) rc = penta_batch_solve(gr->gx, 0, s);
     if (!rc) rc = penta_batch_solve(gr->gy, 0, s);
     for (int q = 0; q < corrections && !rc; q++) {
-      rc = step_batch_matvec(gr->sb, s);
-      if (!rc) rc = step_batch_vec(gr->sb, SB_SUB, s);
+      rc = step_batch_residual(gr->sb, s);
       if (!rc) rc = penta_batch_solve(gr->gx, 1, s);
       if (!rc) rc = penta_batch_solve(gr->gy, 1, s);
-      if (!rc && (q < corrections - 1 || fix)) rc = step_batch_vec(gr->sb, SB_ADD_DV, s);
+      if (!rc && (q < corrections - 1 || fix)) rc = step_batch_add(gr->sb, s);
     }
     if (!rc && fix) rc = step_batch_bcfix(gr->sb, s);
     if (!rc) rc = step_batch_update(gr->sb, corrections > 0 && !fix, s);

@@ -109,6 +109,12 @@ template <int N, int U = 0, typename F> __device__ __forceinline__ void static_f
 // buffers; TW: twisted lines, one per workgroup, else two plain lines; RES:
 // the lines' right-hand sides stay in LDS from the first row to the last.
 //
+// The right-hand sides are read from `in` and the solutions left in rhs, of the
+// same layout (in == rhs: in place; non-resident lines pass through rhs); a
+// refined step's first solve reads the residual so, which was copied before
+// (a step of 257x129 142 -> 138 us with the residual formed in the operator's
+// kernel, 1025x257 527 -> 517).
+//
 // PER: periodic lines (plain pairs).  Their bordered LU has the same band, so
 // rows 0 .. n-3 are a chain without boundary blocks; the last two rows meet
 // every other one:
@@ -150,7 +156,8 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
 
   static __device__ __forceinline__ void run(char *sm, long bid, int n, int h, long L, const cx<T> *__restrict__ fwd,
                                              const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ tail,
-                                             double2 *rhs, long sL, long sR, const cx<T> *__restrict__ p2 = nullptr,
+                                             const double2 *in, double2 *rhs, long sL, long sR,
+                                             const cx<T> *__restrict__ p2 = nullptr,
                                              const cx<T> *__restrict__ qp = nullptr) {
     // rows of a line in memory; of its chain (PER: without the last two)
     const int nmem = n;
@@ -186,7 +193,8 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
         j = first_row(fw, k, c) + u;
         return lane < 60 && rr < 2 * R && j >= 0 && j < len(c);
       };
-      auto value_at = [&](int c, int j) { return rhs + (line_of(c) * sL + (long)real_row(c, j) * sR) * 5 + lq; };
+      const long to_in = reinterpret_cast<const char *>(in) - reinterpret_cast<const char *>(rhs);   // no select: see above
+      auto value_of = [&](auto *v, int c, int j) { return v + (line_of(c) * sL + (long)real_row(c, j) * sR) * 5 + lq; };
       auto issue = [&](bool fw, int k, int buf, int rb) {
         auto records = [&](auto FWT) {
           constexpr int ROW = (decltype(FWT)::value ? 60 : 66) * CS, FULL = R * ROW;   // bytes of a row, a chunk
@@ -240,7 +248,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           for (int rnd = 0; rnd < ROUNDS; rnd++) {
             int c, u, j;
             if (my_row(fw, k, rnd, c, u, j))
-              __builtin_amdgcn_global_load_lds((const void *)value_at(c, j),
+              __builtin_amdgcn_global_load_lds((const void *)(reinterpret_cast<const char *>(value_of(rhs, c, j)) + to_in * fw),
                                                (lds_void *)(sm + (ROWS + rb * 2 * R * ROWB + rnd * 960)), 16, 0, 0);
           }
         }
@@ -251,7 +259,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           for (int b = part; b * 12 < len(c); b += parts) {
             const int j = b * 12 + l5;
             if (lane < 60 && j < len(c))
-              __builtin_amdgcn_global_load_lds((const void *)value_at(c, j), (lds_void *)(sm + (row_off(0, c, 0) + b * 960)),
+              __builtin_amdgcn_global_load_lds((const void *)value_of(in, c, j), (lds_void *)(sm + (row_off(0, c, 0) + b * 960)),
                                                16, 0, 0);
           }
       };
@@ -260,7 +268,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           if (!fw) return;                             // both passes' at the start
           cx<T> v[7];
           const int e20 = min(lane, 19);
-          const double2 b = rhs[(line_of(e20 / 10) * sL + (long)(n + e20 / 5 % 2) * sR) * 5 + e20 % 5];
+          const double2 b = in[(line_of(e20 / 10) * sL + (long)(n + e20 / 5 % 2) * sR) * 5 + e20 % 5];
 #pragma unroll
           for (int i = 0; i < 7; i++) {                // line, row, value
             const int e = min(i * 64 + lane, 403), c = e / 202, r = e % 202 >= 126, k = e % 202 - 126 * r;
@@ -452,7 +460,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           if (my_row(fw, k, rnd, c, u, j) && (TW || 2 * bid + c < L)) {
             const cx<T> x =
                 *reinterpret_cast<const cx<T> *>(sm + (row_off(rb, c, first_row(fw, k, c)) + u * ROWB + lq * 16));
-            *value_at(c, j) = make_double2(x.re, x.im);
+            *value_of(rhs, c, j) = make_double2(x.re, x.im);
             if (PER && !fw && j == 0) rhs[(line_of(c) * sL + (long)nmem * sR) * 5 + lq] = make_double2(x.re, x.im);
           }
         }
@@ -740,19 +748,20 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
 template <typename T, int R, int NBUF, bool TW, bool RES>
 __global__ __launch_bounds__(256, 2) void k_line_solve(int n, int h, long L, const cx<T> *__restrict__ fwd,
                                                       const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ tail,
-                                                      double2 *rhs, long sL, long sR) {
+                                                      const double2 *in, double2 *rhs, long sL, long sR) {
   extern __shared__ __attribute__((aligned(16))) char sm[];
-  LineSolve<T, R, NBUF, TW, RES>::run(sm, xcd_tile(blockIdx.x, gridDim.x), n, h, L, fwd, bwd, tail, rhs, sL, sR);
+  LineSolve<T, R, NBUF, TW, RES>::run(sm, xcd_tile(blockIdx.x, gridDim.x), n, h, L, fwd, bwd, tail, in, rhs, sL, sR);
 }
 
 // periodic lines
 template <typename T, int R, int NBUF, bool RES>
 __global__ __launch_bounds__(256, 2) void k_line_solve_per(int n, long L, const cx<T> *__restrict__ fwd,
                                                           const cx<T> *__restrict__ bwd, const cx<T> *__restrict__ p2,
-                                                          const cx<T> *__restrict__ qp, double2 *rhs, long sL, long sR) {
+                                                          const cx<T> *__restrict__ qp, const double2 *in,
+                                                          double2 *rhs, long sL, long sR) {
   extern __shared__ __attribute__((aligned(16))) char sm[];
-  LineSolve<T, R, NBUF, false, RES, true>::run(sm, xcd_tile(blockIdx.x, gridDim.x), n, -1, L, fwd, bwd, nullptr, rhs, sL,
-                                               sR, p2, qp);
+  LineSolve<T, R, NBUF, false, RES, true>::run(sm, xcd_tile(blockIdx.x, gridDim.x), n, -1, L, fwd, bwd, nullptr, in, rhs,
+                                               sL, sR, p2, qp);
 }
 
 }  // namespace lns3d

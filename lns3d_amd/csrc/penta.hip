@@ -1375,7 +1375,7 @@ template <typename K> static int allow_lds(K k, unsigned lds) {
   return 0;
 }
 
-static int launch_line_solve(const PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
+static int launch_line_solve(const PentaPlan *pl, const void *in, void *rhs, long sL, long sR, hipStream_t s) {
   const bool tw = pl->h >= 0;
   const int form = line_form(pl->variant, pl->n, pl->L, pl->prec, tw);
   return with_line_form(form, pl->prec, tw, [&](auto t, auto lf, auto TW) {
@@ -1386,12 +1386,13 @@ static int launch_line_solve(const PentaPlan *pl, void *rhs, long sL, long sR, h
     if (rc) return rc;
     const long wg = tw ? pl->L : (pl->L + 1) / 2;
     hipLaunchKernelGGL(k, dim3((unsigned)wg), dim3(256), lds, s, pl->n, pl->h, pl->L,
-                       (const cx<T> *)pl->fwd, (const cx<T> *)pl->bwd, (const cx<T> *)pl->tail, (double2 *)rhs, sL, sR);
+                       (const cx<T> *)pl->fwd, (const cx<T> *)pl->bwd, (const cx<T> *)pl->tail, (const double2 *)in,
+                       (double2 *)rhs, sL, sR);
     return 0;
   });
 }
 
-static int launch_per_solve(const PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
+static int launch_per_solve(const PentaPlan *pl, const void *in, void *rhs, long sL, long sR, hipStream_t s) {
   const int form = per_form(pl->n, pl->L, pl->prec);
   return with_per_form(form, pl->prec, [&](auto t, auto lf) {
     using T = decltype(t);
@@ -1400,13 +1401,15 @@ static int launch_per_solve(const PentaPlan *pl, void *rhs, long sL, long sR, hi
     const int rc = allow_lds(k, lds);
     if (rc) return rc;
     hipLaunchKernelGGL(k, dim3((unsigned)((pl->L + 1) / 2)), dim3(256), lds, s, pl->n, pl->L, (const cx<T> *)pl->fwd,
-                       (const cx<T> *)pl->bwd, (const cx<T> *)pl->p2, (const cx<T> *)pl->qp, (double2 *)rhs, sL, sR);
+                       (const cx<T> *)pl->bwd, (const cx<T> *)pl->p2, (const cx<T> *)pl->qp, (const double2 *)in,
+                       (double2 *)rhs, sL, sR);
     return 0;
   });
 }
 
-int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s) {
-  const int rc = pl->periodic ? launch_per_solve(pl, rhs, sL, sR, s) : launch_line_solve(pl, rhs, sL, sR, s);
+int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s, const void *in) {
+  if (!in) in = rhs;
+  const int rc = pl->periodic ? launch_per_solve(pl, in, rhs, sL, sR, s) : launch_line_solve(pl, in, rhs, sL, sR, s);
   if (rc) return rc;
   LNS3D_CHECK(hipGetLastError());
   return 0;
@@ -1434,7 +1437,7 @@ __global__ __launch_bounds__(256, 2) void kb_line_solve(const PentaBatchItem *it
   const int k = batch_member(off, count);
   const PentaBatchItem &b = items[k];
   LineSolve<T, R, NBUF, TW, RES>::run(sm, (long)blockIdx.x - off[k], b.n, b.h, b.L, (const cx<T> *)b.fwd,
-                                      (const cx<T> *)b.bwd, (const cx<T> *)b.tail, b.rhs[which], b.sL, b.sR);
+                                      (const cx<T> *)b.bwd, (const cx<T> *)b.tail, b.in[which], b.rhs[which], b.sL, b.sR);
 }
 
 template <typename T, int R, int NBUF, bool RES>
@@ -1444,7 +1447,7 @@ __global__ __launch_bounds__(256, 2) void kb_line_solve_per(const PentaBatchItem
   const int k = batch_member(off, count);
   const PentaBatchItem &b = items[k];
   LineSolve<T, R, NBUF, false, RES, true>::run(sm, (long)blockIdx.x - off[k], b.n, -1, b.L, (const cx<T> *)b.fwd,
-                                               (const cx<T> *)b.bwd, nullptr, b.rhs[which], b.sL, b.sR,
+                                               (const cx<T> *)b.bwd, nullptr, b.in[which], b.rhs[which], b.sL, b.sR,
                                                (const cx<T> *)b.p2, (const cx<T> *)b.qp);
 }
 
@@ -1459,9 +1462,9 @@ int stage_upload(void *dev, const void *src, size_t bytes, std::vector<TableUplo
   return 0;
 }
 
-int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, double2 *const *rhs1, const long *sL,
-                      const long *sR, int count, std::vector<PentaBatchGroup> &out,
-                      std::vector<TableUpload> &ups) {
+int penta_batch_build(const PentaPlan *const *plans, const double2 *const *in0, double2 *const *rhs0,
+                      double2 *const *rhs1, const long *sL, const long *sR, int count,
+                      std::vector<PentaBatchGroup> &out, std::vector<TableUpload> &ups) {
   out.clear();
   long lines = 0;              // solved by one launch or another at a time
   for (int k = 0; k < count; k++) lines += plans[k]->L;
@@ -1497,6 +1500,8 @@ int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, doubl
       it.tail = pl->tail;
       it.p2 = pl->p2;
       it.qp = pl->qp;
+      it.in[0] = in0[k];
+      it.in[1] = rhs1[k];
       it.rhs[0] = rhs0[k];
       it.rhs[1] = rhs1[k];
       it.sL = sL[k];

@@ -43,6 +43,7 @@ struct PentaBatchItem {
   long L;
   const void *fwd, *bwd, *tail;
   const void *p2, *qp;     // periodic lines: the border records
+  const double2 *in[2];    // where each right-hand side is read
   double2 *rhs[2];
   long sL, sR;
 };
@@ -91,16 +92,18 @@ int penta_factor_records_only(PentaPlan *pl, hipStream_t s);
 // periodic lines: the complex-float records of dst, rounded from the
 // complex-double records of src (same shape, factored)
 int penta_records_narrow(PentaPlan *dst, const PentaPlan *src, hipStream_t s);
-// in-place solve of rhs (complex double); component d of (line l, row i) at
-// complex offset (l*sL + i*sR)*5 + d
-int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s);
+// in-place solve of rhs (complex double), or of the right-hand side `in` with
+// the solution in rhs; component d of (line l, row i) at complex offset
+// (l*sL + i*sR)*5 + d
+int penta_solve(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s, const void *in = nullptr);
 int penta_solve_reference_order(PentaPlan *pl, void *rhs, long sL, long sR, hipStream_t s);
 // batched solves: the plans grouped by solve kernel, with right-hand sides
-// rhs0[k], rhs1[k] of strides sL[k], sR[k]; penta_batch_solve launches one
-// kernel per group on right-hand side `which` (0 or 1) of every member
-int penta_batch_build(const PentaPlan *const *plans, double2 *const *rhs0, double2 *const *rhs1, const long *sL,
-                      const long *sR, int count, std::vector<PentaBatchGroup> &out,
-                      std::vector<TableUpload> &ups);
+// rhs0[k] (read from in0[k]), rhs1[k] of strides sL[k], sR[k];
+// penta_batch_solve launches one kernel per group on right-hand side `which`
+// (0 or 1) of every member
+int penta_batch_build(const PentaPlan *const *plans, const double2 *const *in0, double2 *const *rhs0,
+                      double2 *const *rhs1, const long *sL, const long *sR, int count,
+                      std::vector<PentaBatchGroup> &out, std::vector<TableUpload> &ups);
 int penta_batch_solve(const std::vector<PentaBatchGroup> &groups, int which, hipStream_t s);
 void penta_batch_free(std::vector<PentaBatchGroup> &groups);
 // factor health: flag the lines whose LU (and border fill) holds a

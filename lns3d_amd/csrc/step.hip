@@ -1826,8 +1826,10 @@ __device__ __forceinline__ int slot_col(int N, int per, int pos, int k) {
 // V the compact viscous entries and AB the spanwise cross entries of the
 // direction; boundary-condition rows as lhs_entry.  Equal to the assembled
 // block rows up to rounding.
+// With b, y is the residual b - L x, and my, mb take the largest parts of y
+// and b at this thread's point.
 __device__ __forceinline__ void line_op(long bid, const AsmCtx &A, const Coeffs &c, int dir, const double2 *x,
-                                        double2 *y) {
+                                        double2 *y, const double2 *b, double &my, double &mb) {
   using namespace st;
   const lns3d_params &p = A.p;
   const int nx = p.nx, ny = p.ny;
@@ -2008,43 +2010,32 @@ __device__ __forceinline__ void line_op(long bid, const AsmCtx &A, const Coeffs 
   for (int r = 0; r < 5; r++) {
     if (ident[r]) out[r] = xc[r];
     if (holdrow) out[r] = z{-xc[r].re, -xc[r].im};
-    y[5 * q + r] = dup ? make_double2(0.0, 0.0) : make_double2(out[r].re, out[r].im);
+    z o = dup ? z{0.0, 0.0} : out[r];
+    if (b) {
+      const z v = ld(b + 5 * q + r);
+      o = v - o;
+      my = fmax(my, fmax(fabs(o.re), fabs(o.im)));
+      mb = fmax(mb, fmax(fabs(v.re), fabs(v.im)));
+    }
+    y[5 * q + r] = make_double2(o.re, o.im);
   }
 }
 __global__ __launch_bounds__(256) void k_line_op(AsmCtx A, Coeffs c, int dir, const double2 *x, double2 *y) {
-  line_op(xcd_tile(blockIdx.x, gridDim.x), A, c, dir, x, y);
+  double my, mb;
+  line_op(xcd_tile(blockIdx.x, gridDim.x), A, c, dir, x, y, nullptr, my, mb);
 }
-
-int launch_af_matvec(const lns3d_params &p, const Coeffs &c, const void *x, void *y, void *tmp,
-                     hipStream_t s) {
-  long P = (long)p.nx * p.ny;
-  AsmCtx Ax = make_asm(p, c, 1), Ay = make_asm(p, c, 2);
-  hipLaunchKernelGGL(k_line_op, dim3(nblocks(P, 256)), dim3(256), 0, s, Ay, c, 2,
-                     (const double2 *)x, (double2 *)tmp);
-  hipLaunchKernelGGL(k_line_op, dim3(nblocks(P, 256)), dim3(256), 0, s, Ax, c, 1,
-                     (const double2 *)tmp, (double2 *)y);
-  LNS3D_CHECK(hipGetLastError());
-  return 0;
-}
-
-// y = b - y and the max norms |y|, |b| (of real and imaginary parts): one
-// partial pair per block, then one block reduces the partials
-constexpr int RES_BLOCKS = 512;
-
-__global__ __launch_bounds__(256) void k_residual(const double2 *b, double2 *y, long n, double *part) {
-  double ay = 0.0, abv = 0.0;
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-    double2 bb = b[t], yy = y[t];
-    double2 rr = make_double2(bb.x - yy.x, bb.y - yy.y);
-    y[t] = rr;
-    ay = fmax(ay, fmax(fabs(rr.x), fabs(rr.y)));
-    abv = fmax(abv, fmax(fabs(bb.x), fabs(bb.y)));
-  }
+// y = b - L x and the max norms |y|, |b| (of real and imaginary parts): one
+// partial pair per block, which k_residual_final reduces.  The residual cost
+// a pass of its own before (1025x257 13 us, 257x129 4 us).
+__global__ __launch_bounds__(256) void k_line_residual(AsmCtx A, Coeffs c, int dir, const double2 *x, const double2 *b,
+                                                       double2 *y, double *part) {
+  double my = 0.0, mb = 0.0;
+  line_op(xcd_tile(blockIdx.x, gridDim.x), A, c, dir, x, y, b, my, mb);
   __shared__ double s1[256], s2[256];
-  s1[threadIdx.x] = ay;
-  s2[threadIdx.x] = abv;
+  s1[threadIdx.x] = my;
+  s2[threadIdx.x] = mb;
   __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+  for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) {
       s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + w]);
       s2[threadIdx.x] = fmax(s2[threadIdx.x], s2[threadIdx.x + w]);
@@ -2080,13 +2071,14 @@ __global__ __launch_bounds__(256) void k_residual_final(const double *part, int 
   }
 }
 
-// norms: 2 doubles of results followed by 2*RES_BLOCKS of partials
-int launch_residual_norms(const void *b, void *y, long n, double *norms, hipStream_t s) {
-  const int nb = (int)std::min<long>(RES_BLOCKS, (n + 255) / 256);
-  hipLaunchKernelGGL(k_residual, dim3(nb), dim3(256), 0, s, (const double2 *)b, (double2 *)y, n,
-                     norms + 2);
-  hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(256), 0, s, (const double *)(norms + 2), nb,
-                     norms);
+int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, const void *b, void *y, void *tmp,
+                       void *part, double *norms, hipStream_t s) {
+  const int nb = nblocks((long)p.nx * p.ny, 256);
+  AsmCtx Ax = make_asm(p, c, 1), Ay = make_asm(p, c, 2);
+  hipLaunchKernelGGL(k_line_op, dim3(nb), dim3(256), 0, s, Ay, c, 2, (const double2 *)x, (double2 *)tmp);
+  hipLaunchKernelGGL(k_line_residual, dim3(nb), dim3(256), 0, s, Ax, c, 1, (const double2 *)tmp, (const double2 *)b,
+                     (double2 *)y, (double *)part);
+  hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(256), 0, s, (const double *)part, nb, norms);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
@@ -2127,12 +2119,15 @@ __device__ __forceinline__ RhsMember rhs_member(const StepBatchItem *items, cons
   return RhsMember{&b.p, &b.st, &b.c, b.buf[SB_V], b.buf[SB_RHS]};
 }
 
-// y = L_dir x with x, y chosen among the member's buffers
-__global__ __launch_bounds__(256) void kb_line_op(const StepBatchItem *items, const int *off, int count, int dir,
-                                                  int xs, int ys) {
-  const int k = step_member(off, count);
+// t1 = Ly dv (dir 2), t2 = rhs - Lx t1 (dir 1); neighbouring rows on one L2
+__global__ __launch_bounds__(256) void kb_line_op(const StepBatchItem *__restrict__ items,
+                                                  const int *__restrict__ off, int count, int dir) {
+  const long bid = xcd_tile(blockIdx.x, gridDim.x);
+  const int k = step_member(off, count, bid);
   const StepBatchItem &b = items[k];
-  line_op((long)blockIdx.x - off[k], dir == 1 ? b.ax : b.ay, b.c, dir, b.buf[xs], b.buf[ys]);
+  double my = 0.0, mb = 0.0;
+  if (dir == 2) line_op(bid - off[k], b.ay, b.c, 2, b.buf[SB_DV], b.buf[SB_T1], nullptr, my, mb);
+  else line_op(bid - off[k], b.ax, b.c, 1, b.buf[SB_T1], b.buf[SB_T2], b.buf[SB_RHS], my, mb);
 }
 
 // the end of a step (update_bc), with the last correction t2 or without
@@ -2143,22 +2138,15 @@ __global__ __launch_bounds__(256) void kb_update_bc(const StepBatchItem *items, 
             b.c.whi, b.c.bnb, b.buf[SB_V], b.buf[SB_DV], with_t2 ? b.buf[SB_T2] : nullptr);
 }
 
-// elementwise stages over the 5P values of a member
-__global__ void kb_vec(const StepBatchItem *items, const int *off, int count, int op) {
+// dv += t2 over the 5P values of a member
+__global__ void kb_add(const StepBatchItem *items, const int *off, int count) {
   const int k = step_member(off, count);
   const StepBatchItem &b = items[k];
   const long t = ((long)blockIdx.x - off[k]) * blockDim.x + threadIdx.x;
   if (t >= 5 * b.P) return;
-  double2 *dv = b.buf[SB_DV], *rhs = b.buf[SB_RHS], *t2 = b.buf[SB_T2];
-  if (op == SB_COPY) {
-    dv[t] = rhs[t];
-  } else if (op == SB_SUB) {
-    const double2 bb = rhs[t], yy = t2[t];
-    t2[t] = make_double2(bb.x - yy.x, bb.y - yy.y);
-  } else {   // SB_ADD_DV
-    const double2 a = dv[t], c = t2[t];
-    dv[t] = make_double2(a.x + c.x, a.y + c.y);
-  }
+  double2 *dv = b.buf[SB_DV];
+  const double2 a = dv[t], c = b.buf[SB_T2][t];
+  dv[t] = make_double2(a.x + c.x, a.y + c.y);
 }
 
 __global__ void kb_itrbc_lr(const StepBatchItem *items, const int *off, int count) {
@@ -2272,11 +2260,11 @@ int step_batch_rhs(const StepBatch &b, hipStream_t s) {
   return 0;
 }
 
-int step_batch_matvec(const StepBatch &b, hipStream_t s) {
+int step_batch_residual(const StepBatch &b, hipStream_t s) {
   const auto *it = (const StepBatchItem *)b.items;
   const dim3 g((unsigned)b.blocks[SB_STAGE_LINE]);
-  hipLaunchKernelGGL(kb_line_op, g, dim3(256), 0, s, it, b.off[SB_STAGE_LINE], b.count, 2, (int)SB_DV, (int)SB_T1);
-  hipLaunchKernelGGL(kb_line_op, g, dim3(256), 0, s, it, b.off[SB_STAGE_LINE], b.count, 1, (int)SB_T1, (int)SB_T2);
+  hipLaunchKernelGGL(kb_line_op, g, dim3(256), 0, s, it, b.off[SB_STAGE_LINE], b.count, 2);
+  hipLaunchKernelGGL(kb_line_op, g, dim3(256), 0, s, it, b.off[SB_STAGE_LINE], b.count, 1);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
@@ -2296,9 +2284,9 @@ int step_batch_bcfix(const StepBatch &b, hipStream_t s) {
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
-int step_batch_vec(const StepBatch &b, int op, hipStream_t s) {
-  hipLaunchKernelGGL(kb_vec, dim3((unsigned)b.blocks[SB_STAGE_VEC]), dim3(256), 0, s,
-                     (const StepBatchItem *)b.items, b.off[SB_STAGE_VEC], b.count, op);
+int step_batch_add(const StepBatch &b, hipStream_t s) {
+  hipLaunchKernelGGL(kb_add, dim3((unsigned)b.blocks[SB_STAGE_VEC]), dim3(256), 0, s, (const StepBatchItem *)b.items,
+                     b.off[SB_STAGE_VEC], b.count);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }

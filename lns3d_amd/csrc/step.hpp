@@ -111,13 +111,11 @@ int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, 
 int launch_itrbc(const lns3d_params &p, const Coeffs &c, void *v, hipStream_t s);
 // the wall normals bnb [2][nx] from the metric's n1, n2 on the wall row
 int launch_wall_normals(const lns3d_params &p, const Coeffs &c, double *bnb, hipStream_t s);
-// y = M x with M = Lx * Ly the approximate-factorization operator (FP64,
-// blocks regenerated from the coefficients); tmp holds 5P complex
-int launch_af_matvec(const lns3d_params &p, const Coeffs &c, const void *x, void *y, void *tmp,
-                     hipStream_t s);
-// y = b - y (complex, n values) and the max norms of y and b into norms[0..1];
-// norms holds 2 + 2*512 doubles (the rest is per-block partials)
-int launch_residual_norms(const void *b, void *y, long n, double *norms, hipStream_t s);
+// y = b - M x with M = Lx * Ly the approximate-factorization operator (FP64,
+// blocks regenerated from the coefficients) and the max norms of y and b into
+// norms[0..1]; tmp holds 5P complex, part two doubles per 256 points
+int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, const void *b, void *y, void *tmp,
+                       void *part, double *norms, hipStream_t s);
 int launch_axpy(void *x, const void *d, long n, hipStream_t s);   // x += d
 int launch_copy(void *dst, const void *src, long n, hipStream_t s);   // complex n values
 
@@ -125,8 +123,6 @@ int launch_copy(void *dst, const void *src, long n, hipStream_t s);   // complex
 // tables built once).  Buffers of a member: v, dv, rhs (the step's
 // residual), t1, t2 (the correction)
 enum { SB_V = 0, SB_DV, SB_RHS, SB_T1, SB_T2 };
-// elementwise stages: dv = rhs; t2 = rhs - t2; dv += t2
-enum { SB_COPY = 0, SB_SUB, SB_ADD_DV };
 enum { SB_STAGE_RHS = 0, SB_STAGE_LINE, SB_STAGE_VEC, SB_STAGE_UPDATE, SB_STAGE_LR, SB_STAGE_NORM,
        SB_STAGE_BCFIX, SB_NSTAGE };
 // norm (optional): the member's residual-norm output of norm_count slots;
@@ -153,9 +149,10 @@ int step_batch_build(const StepBatchMember *m, int count, StepBatch &out, std::v
 void step_batch_free(StepBatch &b);
 // rhs = the backward-Euler residual with the rhsBC3D rows (launch_rhs mode 1)
 int step_batch_rhs(const StepBatch &b, hipStream_t s);
-// t2 = Lx (Ly dv) through t1 (launch_af_matvec)
-int step_batch_matvec(const StepBatch &b, hipStream_t s);
-int step_batch_vec(const StepBatch &b, int op, hipStream_t s);
+// t2 = rhs - Lx (Ly dv) through t1 (launch_af_residual)
+int step_batch_residual(const StepBatch &b, hipStream_t s);
+// dv += t2
+int step_batch_add(const StepBatch &b, hipStream_t s);
 // dv += t2 (with_t2; no member with the inviscid wall rows then), v += dv and
 // itrBC3D of v (launch_update_bc)
 int step_batch_update(const StepBatch &b, bool with_t2, hipStream_t s);
