@@ -868,14 +868,16 @@ extern "C" int lns3d_step_refined_fixed(lns3d_ctx *c, void *v_dev, void *dv_dev,
   // residual needs dv whole before it
   const void *last = corrections > 0 && !check ? c->t2 : nullptr;
   for (int k = 0; k < corrections && !rc; k++) {
-    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, c->scal + 8, c->stream);
+    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, nullptr, c->stream);
     if (!rc) rc = solve_xy(c, c->px32, c->py32, c->t2);
     if (!rc && (k < corrections - 1 || !last)) rc = launch_axpy(dv, c->t2, n, c->stream);
   }
   if (!rc && check) {
-    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, c->scal + 8, c->stream);
+    rc = launch_af_residual(c->p, c->c, dv, rhs, c->t2, c->t1, c->work, nullptr, c->stream);
   }
-  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, dv, last, c->stream);
+  // the update's launch reduces the norms of the last residual formed
+  double *norms = corrections > 0 || check ? c->scal + 8 : nullptr;
+  if (!rc) rc = launch_update_bc(c->p, c->c, v_dev, dv, last, c->stream, c->work, norms);
   if (!rc) c->lstep++;
   return rc;
 }

@@ -1613,10 +1613,44 @@ __device__ __forceinline__ void update_bc(long t, const lns3d_params &p, const d
     for (int r = 1; r < 5; r++) put(r, d, u[r]);
   }
 }
+// the max norms of a refined step's residual from nb pairs of partial ones
+// (one workgroup of 256)
+__device__ __forceinline__ void residual_final(const double *part, int nb, double *norms) {
+  __shared__ double s1[256], s2[256];
+  double a = 0.0, b = 0.0;
+  for (int k = threadIdx.x; k < nb; k += blockDim.x) {
+    a = fmax(a, part[2 * k]);
+    b = fmax(b, part[2 * k + 1]);
+  }
+  s1[threadIdx.x] = a;
+  s2[threadIdx.x] = b;
+  __syncthreads();
+  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) {
+      s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + w]);
+      s2[threadIdx.x] = fmax(s2[threadIdx.x], s2[threadIdx.x + w]);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    norms[0] = s1[0];
+    norms[1] = s2[0];
+  }
+}
+// NORMS: workgroup 0 takes the refined step's residual norm, a launch of 4 us
+// by itself.
+template <bool NORMS>
 __global__ __launch_bounds__(256) void k_update_bc(lns3d_params p, const double *ftop, const double *fside,
                                                    const double *fwall, int wlo, int whi, const double *bnb,
-                                                   double2 *v, double2 *dv, const double2 *t2) {
-  update_bc((long)blockIdx.x * blockDim.x + threadIdx.x, p, ftop, fside, fwall, wlo, whi, bnb, v, dv, t2);
+                                                   double2 *v, double2 *dv, const double2 *t2, const double *part,
+                                                   int nb, double *norms) {
+  if constexpr (NORMS) {
+    if (blockIdx.x == 0) {
+      residual_final(part, nb, norms);
+      return;
+    }
+  }
+  update_bc((long)(blockIdx.x - NORMS) * blockDim.x + threadIdx.x, p, ftop, fside, fwall, wlo, whi, bnb, v, dv, t2);
 }
 
 __global__ void k_copy2(double2 *dst, const double2 *src, long n) {
@@ -1784,7 +1818,8 @@ int launch_axpy(void *x, const void *d, long n, hipStream_t s) {
   return 0;
 }
 
-int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, const void *t2, hipStream_t s) {
+int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, const void *t2, hipStream_t s,
+                     const void *part, double *norms) {
   const bool inviscid = c.bnb && !p.yper;
   if (inviscid) {              // the increment's wall row back to x, y components
     if (t2) {
@@ -1794,9 +1829,14 @@ int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, 
     }
     hipLaunchKernelGGL(k_bcfix, dim3(nblocks(p.nx, 128)), dim3(128), 0, s, p.nx, c.bnb, (double2 *)dv);
   }
-  hipLaunchKernelGGL(k_update_bc, dim3(nblocks(update_threads(p, inviscid), 256)), dim3(256), 0, s, p,
-                     (const double *)c.ftop, (const double *)c.fside, (const double *)c.fwall, c.wlo, c.whi, c.bnb,
-                     (double2 *)v, (double2 *)dv, (const double2 *)t2);
+  auto launch = [&](auto k, int extra) {
+    hipLaunchKernelGGL(k, dim3(nblocks(update_threads(p, inviscid), 256) + extra), dim3(256), 0, s, p,
+                       (const double *)c.ftop, (const double *)c.fside, (const double *)c.fwall, c.wlo, c.whi, c.bnb,
+                       (double2 *)v, (double2 *)dv, (const double2 *)t2, (const double *)part,
+                       nblocks((long)p.nx * p.ny, 256), norms);
+  };
+  if (norms) launch(k_update_bc<true>, 1);
+  else launch(k_update_bc<false>, 0);
   if (bc_after_update(p))
     hipLaunchKernelGGL(k_itrbc_lr, dim3(nblocks(p.ny, 128)), dim3(128), 0, s, p, (const double *)c.fside, (double2 *)v);
   LNS3D_CHECK(hipGetLastError());
@@ -2049,26 +2089,7 @@ __global__ __launch_bounds__(256) void k_line_residual(AsmCtx A, Coeffs c, int d
 }
 
 __global__ __launch_bounds__(256) void k_residual_final(const double *part, int nb, double *norms) {
-  __shared__ double s1[256], s2[256];
-  double a = 0.0, b = 0.0;
-  for (int k = threadIdx.x; k < nb; k += blockDim.x) {
-    a = fmax(a, part[2 * k]);
-    b = fmax(b, part[2 * k + 1]);
-  }
-  s1[threadIdx.x] = a;
-  s2[threadIdx.x] = b;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + w]);
-      s2[threadIdx.x] = fmax(s2[threadIdx.x], s2[threadIdx.x + w]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    norms[0] = s1[0];
-    norms[1] = s2[0];
-  }
+  residual_final(part, nb, norms);
 }
 
 int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, const void *b, void *y, void *tmp,
@@ -2078,7 +2099,7 @@ int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, co
   hipLaunchKernelGGL(k_line_op, dim3(nb), dim3(256), 0, s, Ay, c, 2, (const double2 *)x, (double2 *)tmp);
   hipLaunchKernelGGL(k_line_residual, dim3(nb), dim3(256), 0, s, Ax, c, 1, (const double2 *)tmp, (const double2 *)b,
                      (double2 *)y, (double *)part);
-  hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(256), 0, s, (const double *)part, nb, norms);
+  if (norms) hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(256), 0, s, (const double *)part, nb, norms);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }

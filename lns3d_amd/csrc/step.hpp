@@ -107,13 +107,16 @@ int launch_forced_norm(const lns3d_params &p, const Coeffs &c, const void *r, do
 // ftop: the top = 1 wave (Coeffs::ftop), null for top = 0
 // dv += t2 (unless null), v += dv and itrBC3D; for the inviscid deck bcfix
 // turns dv's wall row back to x, y components first (src/impdrv3d.f90:333-336)
-int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, const void *t2, hipStream_t s);
+// (with norms: launch_af_residual's norms from its part as well)
+int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, const void *t2, hipStream_t s,
+                     const void *part = nullptr, double *norms = nullptr);
 int launch_itrbc(const lns3d_params &p, const Coeffs &c, void *v, hipStream_t s);
 // the wall normals bnb [2][nx] from the metric's n1, n2 on the wall row
 int launch_wall_normals(const lns3d_params &p, const Coeffs &c, double *bnb, hipStream_t s);
 // y = b - M x with M = Lx * Ly the approximate-factorization operator (FP64,
 // blocks regenerated from the coefficients) and the max norms of y and b into
-// norms[0..1]; tmp holds 5P complex, part two doubles per 256 points
+// norms[0..1] (null: left in part for launch_update_bc); tmp holds 5P complex,
+// part two doubles per 256 points
 int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, const void *b, void *y, void *tmp,
                        void *part, double *norms, hipStream_t s);
 int launch_axpy(void *x, const void *d, long n, hipStream_t s);   // x += d
