@@ -1310,6 +1310,7 @@ int launch_rhs(const lns3d_params &p, const Stencil &st, const Coeffs &c, const 
 
 // ==========================================================================
 // update and boundary conditions on v (src/impdrv3d.f90:340-356, itrbc3d.f90)
+constexpr int OP_T = 64;             // points of a workgroup of the line operator (k_line_op)
 __global__ void k_axpy(double2 *x, const double2 *d, long n) {
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
@@ -1833,7 +1834,7 @@ int launch_update_bc(const lns3d_params &p, const Coeffs &c, void *v, void *dv, 
     hipLaunchKernelGGL(k, dim3(nblocks(update_threads(p, inviscid), 256) + extra), dim3(256), 0, s, p,
                        (const double *)c.ftop, (const double *)c.fside, (const double *)c.fwall, c.wlo, c.whi, c.bnb,
                        (double2 *)v, (double2 *)dv, (const double2 *)t2, (const double *)part,
-                       nblocks((long)p.nx * p.ny, 256), norms);
+                       nblocks((long)p.nx * p.ny, OP_T), norms);
   };
   if (norms) launch(k_update_bc<true>, 1);
   else launch(k_update_bc<false>, 0);
@@ -2060,31 +2061,28 @@ __device__ __forceinline__ void line_op(long bid, const AsmCtx &A, const Coeffs 
     y[5 * q + r] = make_double2(o.re, o.im);
   }
 }
-__global__ __launch_bounds__(256) void k_line_op(AsmCtx A, Coeffs c, int dir, const double2 *x, double2 *y) {
+// Workgroups of one wave: a grid of 257x129 points is 130 workgroups of four,
+// half the CUs, and the last of a large grid's wait for room for four (us, L_y
+// and the residual with L_x: 1025x257 31 and 62 -> 28.5 and 59.5).
+__global__ __launch_bounds__(OP_T, 3) void k_line_op(AsmCtx A, Coeffs c, int dir, const double2 *x, double2 *y) {
   double my, mb;
   line_op(xcd_tile(blockIdx.x, gridDim.x), A, c, dir, x, y, nullptr, my, mb);
 }
 // y = b - L x and the max norms |y|, |b| (of real and imaginary parts): one
 // partial pair per block, which k_residual_final reduces.  The residual cost
 // a pass of its own before (1025x257 13 us, 257x129 4 us).
-__global__ __launch_bounds__(256) void k_line_residual(AsmCtx A, Coeffs c, int dir, const double2 *x, const double2 *b,
+__global__ __launch_bounds__(OP_T, 3) void k_line_residual(AsmCtx A, Coeffs c, int dir, const double2 *x, const double2 *b,
                                                        double2 *y, double *part) {
   double my = 0.0, mb = 0.0;
   line_op(xcd_tile(blockIdx.x, gridDim.x), A, c, dir, x, y, b, my, mb);
-  __shared__ double s1[256], s2[256];
-  s1[threadIdx.x] = my;
-  s2[threadIdx.x] = mb;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + w]);
-      s2[threadIdx.x] = fmax(s2[threadIdx.x], s2[threadIdx.x + w]);
-    }
-    __syncthreads();
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    my = fmax(my, __shfl_xor(my, w));
+    mb = fmax(mb, __shfl_xor(mb, w));
   }
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s1[0];
-    part[2 * blockIdx.x + 1] = s2[0];
+    part[2 * blockIdx.x] = my;
+    part[2 * blockIdx.x + 1] = mb;
   }
 }
 
@@ -2094,10 +2092,10 @@ __global__ __launch_bounds__(256) void k_residual_final(const double *part, int 
 
 int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, const void *b, void *y, void *tmp,
                        void *part, double *norms, hipStream_t s) {
-  const int nb = nblocks((long)p.nx * p.ny, 256);
+  const int nb = nblocks((long)p.nx * p.ny, OP_T);
   AsmCtx Ax = make_asm(p, c, 1), Ay = make_asm(p, c, 2);
-  hipLaunchKernelGGL(k_line_op, dim3(nb), dim3(256), 0, s, Ay, c, 2, (const double2 *)x, (double2 *)tmp);
-  hipLaunchKernelGGL(k_line_residual, dim3(nb), dim3(256), 0, s, Ax, c, 1, (const double2 *)tmp, (const double2 *)b,
+  hipLaunchKernelGGL(k_line_op, dim3(nb), dim3(OP_T), 0, s, Ay, c, 2, (const double2 *)x, (double2 *)tmp);
+  hipLaunchKernelGGL(k_line_residual, dim3(nb), dim3(OP_T), 0, s, Ax, c, 1, (const double2 *)tmp, (const double2 *)b,
                      (double2 *)y, (double *)part);
   if (norms) hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(256), 0, s, (const double *)part, nb, norms);
   LNS3D_CHECK(hipGetLastError());
@@ -2141,7 +2139,7 @@ __device__ __forceinline__ RhsMember rhs_member(const StepBatchItem *items, cons
 }
 
 // t1 = Ly dv (dir 2), t2 = rhs - Lx t1 (dir 1); neighbouring rows on one L2
-__global__ __launch_bounds__(256) void kb_line_op(const StepBatchItem *__restrict__ items,
+__global__ __launch_bounds__(OP_T, 3) void kb_line_op(const StepBatchItem *__restrict__ items,
                                                   const int *__restrict__ off, int count, int dir) {
   const long bid = xcd_tile(blockIdx.x, gridDim.x);
   const int k = step_member(off, count, bid);
@@ -2200,7 +2198,7 @@ static long stage_blocks(int stage, const lns3d_params &p) {
   const long P = (long)p.nx * p.ny;
   switch (stage) {
     case SB_STAGE_RHS: return (long)rhs_row_tiles(p.nx) * p.ny;
-    case SB_STAGE_LINE: return nblocks(P, 256);
+    case SB_STAGE_LINE: return nblocks(P, OP_T);
     case SB_STAGE_VEC: return nblocks(5 * P, 256);
     case SB_STAGE_LR: return bc_after_update(p) ? nblocks(p.ny, 128) : 0;
     default: return 0;
@@ -2284,8 +2282,8 @@ int step_batch_rhs(const StepBatch &b, hipStream_t s) {
 int step_batch_residual(const StepBatch &b, hipStream_t s) {
   const auto *it = (const StepBatchItem *)b.items;
   const dim3 g((unsigned)b.blocks[SB_STAGE_LINE]);
-  hipLaunchKernelGGL(kb_line_op, g, dim3(256), 0, s, it, b.off[SB_STAGE_LINE], b.count, 2);
-  hipLaunchKernelGGL(kb_line_op, g, dim3(256), 0, s, it, b.off[SB_STAGE_LINE], b.count, 1);
+  hipLaunchKernelGGL(kb_line_op, g, dim3(OP_T), 0, s, it, b.off[SB_STAGE_LINE], b.count, 2);
+  hipLaunchKernelGGL(kb_line_op, g, dim3(OP_T), 0, s, it, b.off[SB_STAGE_LINE], b.count, 1);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }

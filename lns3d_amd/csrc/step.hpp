@@ -116,7 +116,7 @@ int launch_wall_normals(const lns3d_params &p, const Coeffs &c, double *bnb, hip
 // y = b - M x with M = Lx * Ly the approximate-factorization operator (FP64,
 // blocks regenerated from the coefficients) and the max norms of y and b into
 // norms[0..1] (null: left in part for launch_update_bc); tmp holds 5P complex,
-// part two doubles per 256 points
+// part two doubles per 64 points
 int launch_af_residual(const lns3d_params &p, const Coeffs &c, const void *x, const void *b, void *y, void *tmp,
                        void *part, double *norms, hipStream_t s);
 int launch_axpy(void *x, const void *d, long n, hipStream_t s);   // x += d
