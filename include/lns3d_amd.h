@@ -383,8 +383,9 @@ int lns3d_step_fp32(lns3d_ctx *c, void *v_dev, void *dv_dev);
 
 /* The refined step with a fixed number of corrections and no host
  * synchronisation (graph-capturable); check = 1 adds one operator
- * application whose relative residual lns3d_last_residual returns.  No
- * counterpart in the reference (its step is complex double). */
+ * application whose relative residual lns3d_last_residual returns (not a
+ * number where the residual is not finite).  No counterpart in the reference
+ * (its step is complex double). */
 int lns3d_step_refined_fixed(lns3d_ctx *c, void *v_dev, void *dv_dev, int corrections, int check);
 int lns3d_last_residual(lns3d_ctx *c, double *rel);
 /* device bytes a factored context of these parameters holds (admission by

@@ -7,6 +7,7 @@
 #include <string.h>
 #include <string>
 #include <complex>
+#include <limits>
 #include <utility>
 #include <vector>
 
@@ -787,6 +788,13 @@ extern "C" int lns3d_set_time_history(lns3d_ctx *c, const void *vold_dev, long l
   return 0;
 }
 
+// the relative residual of the norms {|res|_max, |r|_max}: 0 where there is
+// none at all, not a number where either is not finite
+static double relative_residual(const double *nr) {
+  if (!std::isfinite(nr[0]) || !std::isfinite(nr[1])) return std::numeric_limits<double>::quiet_NaN();
+  return nr[1] > 0 ? nr[0] / nr[1] : 0.0;
+}
+
 // The same step with the line solves in complex float used as a
 // defect-correction preconditioner for the complex-double AF system
 // M dv = r, M = Lx Ly (M applied with blocks regenerated in double):
@@ -815,16 +823,16 @@ extern "C" int lns3d_step_refined(lns3d_ctx *c, void *v_dev, void *dv_dev, doubl
     if (rc) return rc;
     LNS3D_CHECK(hipMemcpyAsync(nr, c->scal + 8, 16, hipMemcpyDeviceToHost, c->stream));
     LNS3D_CHECK(hipStreamSynchronize(c->stream));
-    if (nr[0] <= tol * nr[1] || it >= cap || !(nr[0] == nr[0])) break;
+    if (nr[0] <= tol * nr[1] || it >= cap || !std::isfinite(nr[0])) break;
     rc = solve_xy(c, c->px32, c->py32, c->t2);
     if (!rc) rc = launch_axpy(dv, c->t2, n, c->stream);
     if (rc) return rc;
   }
   c->last_iters = it;
-  c->last_resid = nr[1] > 0 ? nr[0] / nr[1] : 0.0;
+  c->last_resid = relative_residual(nr);
   if (iters_out) *iters_out = it;
   if (resid_out) *resid_out = c->last_resid;
-  if (!(c->last_resid == c->last_resid)) return fail(LNS3D_ENONFINITE, "refinement produced NaN");
+  if (!(c->last_resid == c->last_resid)) return fail(LNS3D_ENONFINITE, "lns3d_step_refined: the residual is not finite");
   rc = launch_update_bc(c->p, c->c, v_dev, dv, nullptr, c->stream);
   if (!rc) c->lstep++;
   return rc;
@@ -887,7 +895,7 @@ extern "C" int lns3d_last_residual(lns3d_ctx *c, double *rel) {
   double nr[2];
   LNS3D_CHECK(hipMemcpyAsync(nr, c->scal + 8, 16, hipMemcpyDeviceToHost, c->stream));
   LNS3D_CHECK(hipStreamSynchronize(c->stream));
-  *rel = nr[1] > 0 ? nr[0] / nr[1] : 0.0;
+  *rel = relative_residual(nr);
   return 0;
 }
 
