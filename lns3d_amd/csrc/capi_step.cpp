@@ -899,19 +899,18 @@ extern "C" int lns3d_last_residual(lns3d_ctx *c, double *rel) {
   return 0;
 }
 
-// bytes of device memory a context of these parameters holds once factored
+// bytes of device memory a context of these parameters holds once factored:
+// coefficients, work and r, scalars, the inviscid deck's wall normals, the
+// plans of both directions; precision 1: the complex-float plans, t1 .. t3
 extern "C" int lns3d_ctx_bytes(const lns3d_params *p, size_t *bytes) {
   if (!p || !bytes) return fail(LNS3D_EINVAL, "lns3d_ctx_bytes: null argument");
   const size_t P = (size_t)p->nx * p->ny;
-  size_t b = P * (25 * 4 + 6 * 3 + 4 + 1 + 5 + 10) * 8 + P * 160 + 512;   // coefficients, work, r
-  auto plan = [&](int periodic, size_t es) {
-    size_t x = P * 125 * 16;                                  // LU working copy
-    if (periodic) x += 2 * P * 50 * 16;
-    else x += P * 126 * es + P * 2 * 150 * es / 32 + P * 100 * 16 / 32 + P * 26 * es;   // (26: room)
-    return x;
-  };
-  b += plan(p->xper, 16) + plan(p->yper, 16);
-  if (p->precision == 1) b += 2 * P * 126 * 8 + 3 * P * 80;
+  size_t b = P * (25 * 4 + 6 * 3 + 4 + 1 + 5 + 10) * 8 + P * 160 + 4096 * sizeof(double);
+  if (p->Re == 0.0 && p->mattyp == 0) b += (size_t)2 * p->nx * sizeof(double);
+  for (int prec = 0; prec <= (p->precision == 1); prec++)
+    b += penta_plan_bytes(p->xper, p->nx, p->ny, prec, false, !prec) +
+         penta_plan_bytes(p->yper, p->ny, p->nx, prec, false, !prec);
+  if (p->precision == 1) b += 3 * P * 80;
   *bytes = b;
   return 0;
 }

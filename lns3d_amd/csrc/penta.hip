@@ -1144,6 +1144,38 @@ int penta_plan_create(PentaPlan *pl, int periodic, int exact, int n_rows, long l
                                    periodic ? PENTA_PLAIN1 : penta_variant_for(n, lines, prec, row_order));
 }
 
+// what a plan holds on the device
+namespace {
+struct PlanBytes {
+  size_t lu, per, fwd, bwd, tail, mid, border;   // per: each of per, per2; border: each of p2, qp
+};
+}  // namespace
+static PlanBytes plan_bytes(int periodic, int n_rows, long lines, int prec, bool tw) {
+  const size_t es = prec ? sizeof(cx<float>) : sizeof(cx<double>), z = sizeof(cx<double>);
+  const size_t L = (size_t)lines, np = (size_t)n_rows, n = periodic ? np - 1 : np;
+  PlanBytes b{};
+  b.lu = np * 125 * L * z;
+  b.fwd = n * 60 * L * es;
+  b.bwd = n * 66 * L * es;
+  if (periodic) {
+    // complex-float plans take their records from a complex-double plan
+    // (penta_records_narrow): no bordered LU of their own
+    if (!prec) b.per = np * 50 * L * z;
+    b.border = n * 50 * L * es;
+  } else {
+    b.tail = 150 * L * (tw ? 2 : 1) * es;
+    if (tw) b.mid = 100 * L * z;
+  }
+  return b;
+}
+
+size_t penta_plan_bytes(int periodic, int n_rows, long lines, int prec, bool row_order, bool own_lu) {
+  const int n = periodic ? n_rows - 1 : n_rows;
+  const bool tw = !periodic && n >= 16 && penta_twisted(penta_variant_for(n, lines, 0, row_order));
+  const PlanBytes b = plan_bytes(periodic, n_rows, lines, prec, tw);
+  return (own_lu ? b.lu : 0) + 2 * b.per + b.fwd + b.bwd + b.tail + b.mid + 2 * b.border + (size_t)lines * sizeof(int);
+}
+
 int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec,
                               int variant) {
   pl->periodic = periodic;
@@ -1156,29 +1188,22 @@ int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows
   if (penta_twisted(variant) && pl->n < 16) variant = PENTA_PLAIN1;
   pl->variant = periodic ? PENTA_PLAIN1 : variant;
   pl->h = (!periodic && penta_twisted(pl->variant)) ? (pl->n - 1) / 2 : -1;
-  size_t ne = (size_t)pl->np * 125 * lines;
-  LNS3D_CHECK(hipMalloc(&pl->lu, ne * sizeof(cx<double>)));
+  const PlanBytes b = plan_bytes(periodic, n_rows, lines, prec, pl->h >= 0);
+  LNS3D_CHECK(hipMalloc(&pl->lu, b.lu));
   pl->per = pl->per2 = nullptr;
   pl->fwd = pl->bwd = pl->tail = pl->mid = pl->p2 = pl->qp = pl->flags = nullptr;
-  if (periodic) {
-    // complex-float plans take their records from a complex-double plan
-    // (penta_records_narrow): no bordered LU of their own
-    const size_t z = prec ? sizeof(cx<float>) : sizeof(cx<double>);
-    if (!prec) {
-      LNS3D_CHECK(hipMalloc(&pl->per, (size_t)pl->np * 50 * lines * z));
-      LNS3D_CHECK(hipMalloc(&pl->per2, (size_t)pl->np * 50 * lines * z));
-    }
-    LNS3D_CHECK(hipMalloc(&pl->fwd, (size_t)pl->n * 60 * lines * z));
-    LNS3D_CHECK(hipMalloc(&pl->bwd, (size_t)pl->n * 66 * lines * z));
-    LNS3D_CHECK(hipMalloc(&pl->p2, (size_t)pl->n * 50 * lines * z));
-    LNS3D_CHECK(hipMalloc(&pl->qp, (size_t)pl->n * 50 * lines * z));
-  } else {
-    size_t es = prec ? sizeof(cx<float>) : sizeof(cx<double>);
-    LNS3D_CHECK(hipMalloc(&pl->fwd, (size_t)pl->n * 60 * lines * es));
-    LNS3D_CHECK(hipMalloc(&pl->bwd, (size_t)pl->n * 66 * lines * es));
-    LNS3D_CHECK(hipMalloc(&pl->tail, (size_t)150 * lines * (pl->h >= 0 ? 2 : 1) * es));
-    if (pl->h >= 0) LNS3D_CHECK(hipMalloc(&pl->mid, (size_t)100 * lines * sizeof(cx<double>)));
+  if (b.per) {
+    LNS3D_CHECK(hipMalloc(&pl->per, b.per));
+    LNS3D_CHECK(hipMalloc(&pl->per2, b.per));
   }
+  LNS3D_CHECK(hipMalloc(&pl->fwd, b.fwd));
+  LNS3D_CHECK(hipMalloc(&pl->bwd, b.bwd));
+  if (b.border) {
+    LNS3D_CHECK(hipMalloc(&pl->p2, b.border));
+    LNS3D_CHECK(hipMalloc(&pl->qp, b.border));
+  }
+  if (b.tail) LNS3D_CHECK(hipMalloc(&pl->tail, b.tail));
+  if (b.mid) LNS3D_CHECK(hipMalloc(&pl->mid, b.mid));
   return 0;
 }
 

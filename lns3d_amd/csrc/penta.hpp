@@ -82,6 +82,10 @@ int penta_plan_create(PentaPlan *pl, int periodic, int exact, int n_rows, long l
 int penta_plan_create_variant(PentaPlan *pl, int periodic, int exact, int n_rows, long lines, int prec,
                               int variant);
 void penta_plan_destroy(PentaPlan *pl);
+// device bytes of a plan of this shape, its health flags included (own_lu: with
+// the LU working copy, which a context's complex-float plans borrow); the
+// family is the complex-double plan's in both precisions
+size_t penta_plan_bytes(int periodic, int n_rows, long lines, int prec, bool row_order, bool own_lu);
 // copy a device matrix in the reference's layout mat(5,5,5,...) into the
 // working copy; block (line l, row i) starts at complex offset (i*sRm + l*sLm)*125
 int penta_import(PentaPlan *pl, const void *ref_mat, long sLm, long sRm, hipStream_t s);
