@@ -677,14 +677,20 @@ __device__ __forceinline__ void eliminate_interior(cx<double> *mx, cx<double> *l
 // the partner's blocks updated.
 constexpr int FW = 5;
 
-__global__ __launch_bounds__(128) void k_factor_chains(LineGeom g, cx<double> *lu, cx<double> *mid) {
+// TW: twisted lines, two chains.  A plain line has one and half the LDS: ten
+// of its workgroups fit a CU, where four did with the LDS of two chains (a
+// factor with its import and records, us: 1300 lines of 7 rows 330 -> 191,
+// 2000 of 12 393 -> 244, 20000 of 33 4920 -> 2914; with rows updated task by
+// task in LDS, before, these took 241, 362 and 6666).
+template <bool TW>
+__global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<double> *lu, cx<double> *mid) {
   using T = double;
-  __shared__ cx<T> win[2][FW][125];
-  __shared__ cx<T> mx[2][MX_SIZE];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  __shared__ cx<T> win[TW ? 2 : 1][FW][125];
+  __shared__ cx<T> mx[TW ? 2 : 1][MX_SIZE];
+  const int wave = TW ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, lane = threadIdx.x & 63;
   const long line = blockIdx.x;
   const int n = g.n, h = g.h;
-  const bool tw = h >= 0;
+  constexpr bool tw = TW;
   cx<T> *lul = lu + line * n * 125;
   cx<T> *midl = mid ? mid + line * 4 * 25 : nullptr;
   auto wsync = [] { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); };
@@ -1290,8 +1296,9 @@ int penta_factor(PentaPlan *pl, hipStream_t s) {
     LNS3D_CHECK(hipGetLastError());
     return 0;
   }
-  hipLaunchKernelGGL(k_factor_chains, dim3((unsigned)pl->L), dim3(pl->h >= 0 ? 128 : 64), 0, s, g,
-                     (cx<double> *)pl->lu, (cx<double> *)pl->mid);
+  const bool tw = pl->h >= 0;
+  hipLaunchKernelGGL(tw ? k_factor_chains<true> : k_factor_chains<false>, dim3((unsigned)pl->L), dim3(tw ? 128 : 64),
+                     0, s, g, (cx<double> *)pl->lu, (cx<double> *)pl->mid);
   LNS3D_CHECK(hipGetLastError());
   const int rc = clear_flags(pl, s);
   return rc ? rc : records_launch(pl, (int *)pl->flags, s);
