@@ -1348,6 +1348,14 @@ static unsigned line_lds(int form, int prec, bool tw, int n, bool per = false) {
   });
 }
 
+// workgroups of a form that a CU holds.  The LDS is given out in pieces of 1280
+// bytes: three workgroups of 53,664 bytes share a CU, of 53,824 bytes two
+// (1025 plain lines of 157 and 158 rows, LINES_RES3: 80 and 128 us).
+static int cu_fit(int form, int prec, bool tw, int n, bool per = false) {
+  constexpr unsigned PIECE = 1280;
+  return (int)(LDS_PER_CU / ((line_lds(form, prec, tw, n, per) + PIECE - 1) / PIECE * PIECE));
+}
+
 // The form for `lines` lines of n rows solved by one launch.  What matters is
 // how many workgroups share a CU (256 CUs, LDS_PER_CU of LDS each): while all
 // lines run at once a solve takes as long as its chain, so one or two per CU
@@ -1358,13 +1366,21 @@ static unsigned line_lds(int form, int prec, bool tw, int n, bool per = false) {
 //            257x257 36 / 37; 1025 lines of 257: RES6 120, RES3 126, RING3 132;
 //            513 of 257: RES3 63, RES6 75; 700 of 600: RING3 189, RING6 207
 //   plain    1025 of 65: RES3 33, RES6 41; 513 of 257: RING6 73, RING3 79;
-//            1025 of 257: RING3 133, RING6 151
+//            1025 of 257: RING3 133, RING6 151; where three workgroups of RES3
+//            don't fit, RES6 / RING3: 1300 of 163 106 / 103, 2000 of 163
+//            124 / 148, 3000 of 170 194 / 229
 //   complex float, twisted: 257x1025 RING12 85, RING6 101; 127x384 RES12 35,
 //            RES6 41; 1025 of 257: RES6 74, RING6 83; 33x65 RES6 11.6, RES12 12.7
+//   complex float, more than two workgroups a CU, RES6 / RING6 / RING12:
+//            all at once with RES6, plain 1500 of 129 50 / 55 / 68; only with
+//            RING6, plain 1025 of 200 90 / 59 / 81, 1600 of 158 84 / 71 / 78,
+//            twisted 513 of 384 93 / 59 / 84, 769 of 200 59 / 45 / 55; with
+//            neither, plain 2500 of 158 98 / 120 / 116, of 257 178 / 190 / 169,
+//            3000 of 200 156 / 160 / 151
 static int line_form(int variant, int n, long lines, int prec, bool tw) {
-  // workgroups of a form that a CU holds
-  auto fit = [&](int form) { return (int)(LDS_PER_CU / line_lds(form, prec, tw, n)); };
+  auto fit = [&](int form) { return cu_fit(form, prec, tw, n); };
   const long wg = tw ? lines : (lines + 1) / 2;
+  auto at_once = [&](int form) { return wg <= 256L * fit(form); };
   const int need = wg <= 256 ? 1 : wg <= 512 ? 2 : 3;      // to run all at once, up to three
   // variants that pin a form
   const int small = prec ? (fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING6) : (fit(LINES_RES3) >= 3 ? LINES_RES3 : LINES_RING3);
@@ -1378,25 +1394,33 @@ static int line_form(int variant, int n, long lines, int prec, bool tw) {
     if (prec && n >= 96) return fit(LINES_RES12) >= need ? LINES_RES12 : LINES_RING12;
     return fit(LINES_RES6) >= need ? LINES_RES6 : LINES_RING6;
   }
-  if (prec) return fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING6;
+  if (prec) {
+    if (at_once(LINES_RES6)) return LINES_RES6;
+    if (at_once(LINES_RING6)) return LINES_RING6;
+    return fit(LINES_RES6) >= 3 ? LINES_RES6 : LINES_RING12;
+  }
   if (fit(LINES_RES3) >= 3 && (!tw || n < 128 || wg <= 768)) return LINES_RES3;
-  return tw && fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING3;
+  return (tw || wg > 768) && fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING3;
 }
 
 // The form of periodic lines, two per workgroup: resident right-hand sides
-// while one workgroup per CU holds every line and its LDS them (they spare
-// 160 of 3920 bytes a row); with more lines the chunks of half the rows, of
-// which two workgroups fit a CU (up to about 100 rows; the prologues of short
-// lines overlap then: 1025 lines of 33 rows 47 us, with six-row chunks 58);
-// rings of twelve (complex float) or six rows else.
+// where they fit (they spare 160 of 3920 bytes a row), with one workgroup per
+// CU the longer chunks, from about 48 rows on in complex float; with more
+// workgroups than CUs the shorter chunks while two of them fit a CU (up to
+// about 85 rows, complex float 120; the prologues of short lines overlap then).
+// Measured at lines x rows, us:
+//   complex double, RES6 / RES3 / RING6: 257 of 33 12 / 16 / 15, 1025 of 33
+//            41 / 38 / 52, of 65 70 / 73 / 82, of 100 100 / 136 / 113
+//   complex float, RES12 / RES6 / RING12: 257 of 24 12 / 10 / 15, of 48
+//            14.5 / 14.4 / 20, of 65 16 / 18 / 23, 513 of 100 46 / 30 / 65,
+//            of 129 58 / 63 / 77, of 300 - / 145 / 161
 static int per_form(int n, long lines, int prec) {
-  auto fit = [&](int form) { return (int)(LDS_PER_CU / line_lds(form, prec, false, n, true)); };
+  auto fit = [&](int form) { return cu_fit(form, prec, false, n, true); };
   const int res = prec ? LINES_RES12 : LINES_RES6, small = prec ? LINES_RES6 : LINES_RES3;
-  if ((lines + 1) / 2 <= 256) {
-    if (fit(res) >= 1) return res;
-  } else if (fit(small) >= 2) {
-    return small;
-  }
+  if ((lines + 1) / 2 > 256 && fit(small) >= 2) return small;
+  if (prec && n < 48) return LINES_RES6;
+  if (fit(res) >= 1) return res;
+  if (prec && fit(LINES_RES6) >= 1) return LINES_RES6;
   return prec ? LINES_RING12 : LINES_RING6;
 }
 
