@@ -328,14 +328,18 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
       };
       // rows n-2 and n-1 of both lines (one wave; lane a of ten has line a / 5
       // and component a % 5): the forward rows with the border sums, then the
-      // backward ones, which become the chain's start and the qp terms' x
+      // backward ones, which become the chain's start and the qp terms' x.
+      // Every line waits for it, so a loop's LDS reads are in flight together
+      // (one at a time they cost a solve 1.4 us: 1025 lines of 24 rows 35.5 ->
+      // 32.9 us with the copy of the right-hand side, a step of 257x97 with
+      // periodic xi lines 100.5 -> 99.0)
       auto border_rows = [&]() {
         if constexpr (PER) {
           auto *bs = reinterpret_cast<cx<T> *>(sm + TAIL + BSUM);
           const auto *part = reinterpret_cast<const cx<T> *>(sm + TAIL + BPART);
           if (lane < 20) {
             cx<T> t{0, 0};                             // over four classes and five columns
-#pragma unroll 1
+#pragma unroll 5
             for (int k = 0; k < 20; k++) t = t + part[k / 5 * 100 + lane * 5 + k % 5];
             bs[lane] = t;
           }
@@ -351,15 +355,21 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
             const cx<T> *L = rec + r * 126 + 50;
             const double2 *b = reinterpret_cast<const double2 *>(sm + (TAIL + BREC)) + (c * 2 + r) * 5;
             cx<T> acc{(T)b[mm].x, (T)b[mm].y};
-#pragma unroll 1
-            for (int q = 0; q < mm; q++) acc = cfma(L[mm * (mm - 1) / 2 + q], cx<T>{(T)b[q].x, (T)b[q].y}, acc);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              const cx<T> t = cfma(L[min(mm * (mm - 1) / 2 + q, 9)], cx<T>{(T)b[q].x, (T)b[q].y}, acc);
+              if (q < mm) acc = t;
+            }
             return acc;
           };
           auto uinv = [&](int r, const cx<T> *y) {
-            const cx<T> *U = rec + (r ? 186 : 110) + mm * 5 - mm * (mm - 1) / 2;
+            const cx<T> *U = rec + (r ? 186 : 110);
             cx<T> acc{0, 0};
-#pragma unroll 1
-            for (int q = mm; q < 5; q++) acc = cfma(U[q - mm], y[q], acc);
+#pragma unroll
+            for (int q = 0; q < 5; q++) {
+              const cx<T> t = cfma(U[min(mm * 5 - mm * (mm - 1) / 2 + q, 14)], y[min(mm + q, 4)], acc);
+              if (q < 5 - mm) acc = t;
+            }
             return acc;
           };
           cx<T> y0 = linv_b(0) + bs[c * 10 + mm], y1 = linv_b(1) + bs[c * 10 + 5 + mm];
@@ -373,7 +383,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           wave_sync();
           if (lane < 10) bs[c * 10 + mm] = y0;
           wave_sync();
-#pragma unroll 1
+#pragma unroll
           for (int q = 0; q < 5; q++) y1 = cfma(entry(rec + 126, 0, q), bs[c * 10 + q], y1);
           if (lane < 10) bs[c * 10 + 5 + mm] = y1;
           wave_sync();
@@ -381,7 +391,7 @@ template <typename T, int R, int NBUF, bool TW, bool RES, bool PER = false> stru
           cx<T> x0 = uinv(0, bs + c * 10);
           if (lane < 10) xs[5 + mm] = x1;
           wave_sync();
-#pragma unroll 1
+#pragma unroll
           for (int q = 0; q < 5; q++) x0 = cfma(entry(rec + 60, 0, q), xs[5 + q], x0);
           if (lane < 10) {
             xs[mm] = x0;
