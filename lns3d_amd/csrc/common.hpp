@@ -11,7 +11,6 @@ template <typename T> struct cx {
   T re, im;
 };
 
-template <typename T> __host__ __device__ __forceinline__ cx<T> mk(T r, T i) { return cx<T>{r, i}; }
 template <typename T> __host__ __device__ __forceinline__ cx<T> operator+(cx<T> a, cx<T> b) { return {a.re + b.re, a.im + b.im}; }
 template <typename T> __host__ __device__ __forceinline__ cx<T> operator-(cx<T> a, cx<T> b) { return {a.re - b.re, a.im - b.im}; }
 template <typename T> __host__ __device__ __forceinline__ cx<T> operator-(cx<T> a) { return {-a.re, -a.im}; }
@@ -44,24 +43,6 @@ template <typename T> __host__ __device__ __forceinline__ cx<T> cdiv(cx<T> a, cx
 }
 template <typename T> __host__ __device__ __forceinline__ cx<T> crecip(cx<T> b) {
   return cdiv(cx<T>{T(1), T(0)}, b);
-}
-
-// wave-uniform broadcast of a lane's complex value (one line per wave)
-__device__ __forceinline__ cx<double> bcast(cx<double> v, int lane) {
-  union { double d; int i[2]; } a, b;
-  a.d = v.re; b.d = v.im;
-  a.i[0] = __builtin_amdgcn_readlane(a.i[0], lane);
-  a.i[1] = __builtin_amdgcn_readlane(a.i[1], lane);
-  b.i[0] = __builtin_amdgcn_readlane(b.i[0], lane);
-  b.i[1] = __builtin_amdgcn_readlane(b.i[1], lane);
-  return {a.d, b.d};
-}
-__device__ __forceinline__ cx<float> bcast(cx<float> v, int lane) {
-  union { float f; int i; } a, b;
-  a.f = v.re; b.f = v.im;
-  a.i = __builtin_amdgcn_readlane(a.i, lane);
-  b.i = __builtin_amdgcn_readlane(b.i, lane);
-  return {a.f, b.f};
 }
 
 // The chip places workgroup b of a launch on XCD b % 8 (round robin over its

@@ -693,7 +693,6 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
   constexpr bool tw = TW;
   cx<T> *lul = lu + line * n * 125;
   cx<T> *midl = mid ? mid + line * 4 * 25 : nullptr;
-  auto wsync = [] { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); };
   // one chain on window w, chain direction tt, pivots [v0, v1), rows above
   // lim never touched
   auto chain = [&](int w, int tt, int v0, int v1, int lim, bool preloaded) {
@@ -735,7 +734,7 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
       for (int r = 0; r < FW; r++)
         if (v + r <= lim) put_row(v + r, x[r][0], x[r][1]);
     };
-    // write back a row: own = all slots (pivot rows) or the chain's share
+    // write back a row: all slots (pivot rows) or the chain's share
     auto store_row = [&](int vr, bool all) {
       cx<T> *dst = lul + (long)real(vr) * 125;
       if (all) {
@@ -747,9 +746,8 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
         int vcol = -1;
         for (int vc = vr - 4; vc <= vr + 4; vc++)
           if (slot(vr, vc) == sl) vcol = vc;
-        if (vcol < 0) { if (all) dst[e] = win[w][vr % FW][e]; continue; }
+        if (vcol < 0) continue;
         const int c = real(vcol);
-        if (all) { dst[e] = win[w][vr % FW][e]; continue; }
         if (middle(vr, vcol)) {
           if (tt == 0) dst[e] = win[w][vr % FW][e];
           else midl[((real(vr) - h) * 2 + (c - h)) * 25 + (e % 25)] = win[w][vr % FW][e];
@@ -759,7 +757,7 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
       }
     };
     if (!preloaded) load_window(v0);
-    wsync();
+    wave_sync();
     // Pivots from 2 on whose partner rows v+1 and v+2 are interior rows of the
     // line (and the chain's): the blocks right of them are columns v+1, v+2,
     // and they go through registers.  The rows beside them keep the window.
@@ -775,17 +773,17 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
           const int b = e / 25, vr = v + b / 2, vc = v - 2 + (b + 1) / 2, sl = slot(vr, vc);
           lul[(long)real(vr) * 125 + sl * 25 + e % 25] = B(vr, sl)[e % 25];
         }
-        wsync();
+        wave_sync();
         eliminate_interior(mx[w], lul, n, tt == 0 ? 1 : -1, v, vfast, tt == 1 && tw ? lim - 1 : n, lane);
         __threadfence_block();
         v = vfast;
         load_window(v);
-        wsync();
+        wave_sync();
         for (int e = lane; e < 100; e += 64) {
           const int r = e / 10, c = e % 10;
           B(v + r / 5, slot(v + r / 5, v + c / 5))[(r % 5) * 5 + c % 5] = mx[w][r * 16 + c];
         }
-        wsync();
+        wave_sync();
         if (v == v1) break;
       }
       // row v+5 comes into the window when row v leaves it; its loads are
@@ -824,14 +822,14 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
       for (int nc = 0; nc < 4; nc++) {
         const int l = nc + 1 + lane;
         if (l < 5) D[l * 5 + nc] = -cdiv(D[l * 5 + nc], D[nc * 6]);
-        wsync();
+        wave_sync();
 #pragma unroll 1
         for (int k = lane; k < (1 + nu) * 25; k += 64) {
           const int b = k / 25, e = k % 25, l = e / 5, q = e % 5;
           cx<T> *X = b == 0 ? D : B(v, pick(us, b - 1));
           if (l > nc && (b > 0 || q > nc)) X[e] = cfma(D[l * 5 + nc], X[nc * 5 + q], X[e]);
         }
-        wsync();
+        wave_sync();
       }
       // partner rows: the block in the pivot column becomes the multipliers
 #pragma unroll 1
@@ -841,7 +839,7 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
           cx<T> *x = B(p, slot(p, v)) + (lane % 5) * 5 + nc;
           *x = -(*x * crecip(D[nc * 6]));
         }
-        wsync();
+        wave_sync();
 #pragma unroll 1
         for (int k = lane; k < nparts * (1 + nu) * 25; k += 64) {
           const int pp = k / ((1 + nu) * 25), b = k / 25 - pp * (1 + nu), e = k % 25, q = e % 5, p = pick(pr, pp);
@@ -852,13 +850,13 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
           cx<T> *x = B(p, sdst) + e;
           *x = cfma(Lb[e - q + nc], X[nc * 5 + q], *x);
         }
-        wsync();
+        wave_sync();
       }
       // row v is final: write it back and bring in row v+5
       store_row(v, true);
-      wsync();
+      wave_sync();
       if (pf_ok) put_row(v + FW, pf0, pf1);
-      wsync();
+      wave_sync();
     }
     // rows the chain updated but did not pivot
     for (int vr = v1; vr <= min(v1 + FW - 1, lim); vr++) store_row(vr, !tw);
@@ -875,13 +873,13 @@ __global__ __launch_bounds__(TW ? 128 : 64) void k_factor_chains(LineGeom g, cx<
     // then their elimination
     for (int rr = h; rr <= h + 1; rr++)
       for (int e = lane; e < 125; e += 64) win[0][rr % FW][e] = lul[(long)rr * 125 + e];
-    wsync();
+    wave_sync();
     for (int e = lane; e < 100; e += 64) {
       const int b = e / 25, r = h + b / 2, c = h + b % 2;
       cx<T> &x = win[0][r % FW][bc_slot(n, r, c) * 25 + e % 25];
       x = x + midl[e];
     }
-    wsync();
+    wave_sync();
     v0 = h;
     v1 = h + 2;
     lim = h + 1;
