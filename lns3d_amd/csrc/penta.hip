@@ -582,9 +582,9 @@ struct PivotWindow {
 // in a row, the exchange through LDS, the multiply-adds of one wave.  Every
 // load and store of memory is unconditional (idle lanes repeat another's), so
 // that the wait for a window's entries counts past the stores in between.
-// 257 twisted lines of 513 rows: 1770 -> 530 to 660 us, 1.7 us a pivot (the same
-// elimination task by task in LDS took 5.8), of which its 450 vector
-// instructions take 1.0
+// 257 twisted lines of 513 rows: 1770 -> 680 us (562 to 706), 2.6 us a pivot;
+// one line of 2000 rows, with import and records, 5.86 -> 1.88 ms for a chain
+// of 1000 pivots.  A pivot's 450 vector instructions take 1.0 us
 constexpr int MX_OUT = 17 * 16, MX_SIZE = MX_OUT + 125;     // 17 rows of 16, the final entries
 __device__ __forceinline__ void eliminate_interior(cx<double> *mx, cx<double> *lul, int n, int dir, int vs, int ve,
                                                    int zero_from, int lane) {
@@ -1117,12 +1117,14 @@ int penta_check_result(PentaPlan *pl, hipStream_t s, long *bad_lines, long *firs
 static std::mutex g_tune_mu;
 static std::map<std::tuple<int, long, int>, int> g_tuned;
 
-// Twisted lines (two chains per line, one line per workgroup) up to 512
-// lines: below that the chain's length is what a solve takes.  Above, plain
-// lines (two per workgroup) where the caller may ask for the reference's
-// substitution order, which needs factors in row order; else twisted lines
-// from 160 rows on.  Measured, plain / twisted us: 513 lines of 257 rows
-// 73 / 63, 1025 of 257 133 / 120, 1025 of 129 62 / 69, 1025 of 65 33 / 40.
+// Twisted lines (two chains per line, one line per workgroup) under 512 lines:
+// there the chain's length is what a solve takes.  From 512 on plain lines (two
+// per workgroup) where the caller may ask for the reference's substitution
+// order, which needs factors in row order; else twisted lines from 160 rows on.
+// Measured, plain / twisted us: 511 lines of 65 rows 18 / 15, of 129 34 / 27,
+// 513 of 65 19 / 18, of 257 80 / 67, 1025 of 65 33 / 39, of 129 65 / 72, of 144
+// 72 / 80, of 160 89 / 86, of 257 142 / 128, 1500 of 144 88 / 95, of 160
+// 109 / 102.
 int penta_variant_for(int n, long lines, int prec, bool row_order) {
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -1367,8 +1369,13 @@ static int cu_fit(int form, int prec, bool tw, int n, bool per = false) {
 //            1025 of 257: RING3 133, RING6 151; where three workgroups of RES3
 //            don't fit, RES6 / RING3: 1300 of 163 106 / 103, 2000 of 163
 //            124 / 148, 3000 of 170 194 / 229
+//            twisted, RES3 / RES6: all at once 513 of 160 39 / 50, 769 of 129
+//            43 / 50; not, 1025 of 96 56 / 59, of 129 72 / 70, of 200 105 / 103
 //   complex float, twisted: 257x1025 RING12 85, RING6 101; 127x384 RES12 35,
-//            RES6 41; 1025 of 257: RES6 74, RING6 83; 33x65 RES6 11.6, RES12 12.7
+//            RES6 41; 1025 of 257: RES6 74, RING6 83
+//   complex float, RES6 / RES12: 257 twisted lines of 65 rows 9.6 / 10.6, of
+//            96 13.1 / 13.1, of 129 16.1 / 15.4; plain, of 33 7.9 / 7.9, of 65
+//            13.0 / 11.7, of 96 17.8 / 17.0
 //   complex float, more than two workgroups a CU, RES6 / RING6 / RING12:
 //            all at once with RES6, plain 1500 of 129 50 / 55 / 68; only with
 //            RING6, plain 1025 of 200 90 / 59 / 81, 1600 of 158 84 / 71 / 78,
@@ -1389,7 +1396,7 @@ static int line_form(int variant, int n, long lines, int prec, bool tw) {
     default: break;
   }
   if (need < 3) {
-    if (prec && n >= 96) return fit(LINES_RES12) >= need ? LINES_RES12 : LINES_RING12;
+    if (prec && n >= (tw ? 96 : 60)) return fit(LINES_RES12) >= need ? LINES_RES12 : LINES_RING12;
     return fit(LINES_RES6) >= need ? LINES_RES6 : LINES_RING6;
   }
   if (prec) {
@@ -1397,7 +1404,7 @@ static int line_form(int variant, int n, long lines, int prec, bool tw) {
     if (at_once(LINES_RING6)) return LINES_RING6;
     return fit(LINES_RES6) >= 3 ? LINES_RES6 : LINES_RING12;
   }
-  if (fit(LINES_RES3) >= 3 && (!tw || n < 128 || wg <= 768)) return LINES_RES3;
+  if (fit(LINES_RES3) >= 3 && (!tw || n < 128 || at_once(LINES_RES3))) return LINES_RES3;
   return (tw || wg > 768) && fit(LINES_RES6) >= 2 ? LINES_RES6 : LINES_RING3;
 }
 

@@ -32,8 +32,8 @@ def _torch():
 
 
 PLAIN = [(0, L, n) for L, n in ((1025, 157), (1025, 158), (1025, 162), (1537, 158), (1541, 172), (1541, 173))] + \
-        [(1, L, n) for L, n in ((1025, 163), (1025, 164), (1540, 84), (1600, 158), (2049, 163), (2050, 164))]
-TWISTED = [(0, 513, 311), (0, 513, 312), (0, 769, 160), (1, 513, 323), (1, 769, 200), (1, 1024, 163), (1, 1025, 322),
+        [(1, L, n) for L, n in ((600, 59), (600, 60), (1025, 163), (1025, 164), (1540, 84), (1600, 158), (2049, 163), (2050, 164))]
+TWISTED = [(0, 513, 311), (0, 513, 312), (0, 769, 129), (0, 769, 160), (0, 1025, 129), (1, 513, 323), (1, 769, 200), (1, 1024, 163), (1, 1025, 322),
            (1, 1025, 324)]
 
 
