@@ -53,16 +53,20 @@ def parse():
     return ap.parse_args()
 
 
+# the kernel of the xi solve at this size
+SOLVE_KERNEL = "k_line_solve<double,6,4,true,false>"
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_solve_xi_1025x257.json")
 
 
-def measured_traffic():
+def measured_traffic(kernel=SOLVE_KERNEL):
     """HBM bytes per xi-solve launch from the committed rocprofv3 --pmc runs
     (FETCH_SIZE + WRITE_SIZE of the solve kernel, each scaled by the counter's
-    reading for a copy of known size); None when that file is absent"""
+    reading for a copy of known size); None when that file is absent or holds
+    another kernel's reading"""
     try:
         with open(TRAFFIC_FILE) as f:
-            return json.load(f)["bytes_per_launch"]
+            d = json.load(f)
+        return d["bytes_per_launch"] if d["kernel"].split(" ")[0] == kernel else None
     except (OSError, KeyError, ValueError):
         return None
 
@@ -168,7 +172,7 @@ def main():
         "config": {"workload": "LNS3D implicit AF step: lrhs3D + xi/eta block-penta line solves + "
                                "update, complex double, factors formed once",
                    "nx": NX, "ny": NY, "beta": BETA, "Ma": p.Ma, "Re": p.Re, "cfl": p.cflmax},
-        "roofline": {"bound": "hbm", "kernel": "k_line_solve<double,6,4,true,false> (xi lines: 257 lines x 1025 rows, twisted)",
+        "roofline": {"bound": "hbm", "kernel": SOLVE_KERNEL + " (xi lines: 257 lines x 1025 rows, twisted)",
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic(),
                      "bytes_per_launch": bytes_launch,
@@ -253,7 +257,8 @@ def main():
         sw = sweep(count=nreq, seed=0, mode="fp32_outer")
         pk_b = peak(count=nreq, seed=0, mode="fp32_outer", batched=True)
         # many small requests: 2 nreq on the two smaller grids, with a graph
-        # per request and batched per grid with three lines per workgroup
+        # per request and batched per grid with plain lines of a small LDS
+        # footprint (line-solve variant 4)
         small = dict(count=2 * nreq, seed=0, mode="fp32_outer", grids=((129, 65), (257, 129)),
                      grid_weights=(0.6, 0.4))
         pk_s0 = peak(batched=False, **small)
@@ -277,7 +282,7 @@ def main():
                         "peak_batched_per_grid": rnd(pk_b),
                         "small_grids_peak": {"requests": 2 * nreq, "grids": "129x65 (0.6), 257x129 (0.4)",
                                              "graph_per_request": rnd(pk_s0),
-                                             "batched_per_grid_three_lines_per_workgroup": rnd(pk_s1)},
+                                             "batched_per_grid_plain_lines": rnd(pk_s1)},
                         "poisson": rnd(sw["open_loop"]),
                         "serial_fp64": dict(rnd(ser64), same_arrivals=fifo(ser64)),
                         "serial_fp32_outer": dict(rnd(ser32), same_arrivals=fifo(ser32)),
