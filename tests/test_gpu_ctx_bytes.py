@@ -3,6 +3,8 @@ which the serving loop admits requests.
 
 Tolerance: a context makes fewer than 32 allocations, each rounded up to a
 page of 2 MiB at most."""
+import gc
+
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -23,6 +25,7 @@ def test_ctx_bytes(kw, precision):
     x, y, met = make_grid(p)
     vm = make_mean(p, y)
     for measured in (False, True):     # the first one brings in the kernels' own memory
+        gc.collect()                   # contexts that other tests left behind give theirs back here, not below
         torch.cuda.synchronize()
         before = torch.cuda.mem_get_info()[0]
         st = Step(p, precision=precision)
