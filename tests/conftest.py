@@ -13,6 +13,13 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs on the GPU box)")
 
 
+def pytest_collection_modifyitems(items):
+    """The tests on a library linked from the reference's own sources come
+    last: where those sources are absent they fail, and a run that stops at the
+    first failure has then run everything else."""
+    items.sort(key=lambda item: "test_gpu_dropin" in item.nodeid)
+
+
 @pytest.fixture(scope="session")
 def orc():
     """The C restatement (oracle/liboracle.so), built on first use if absent."""
