@@ -1614,25 +1614,22 @@ __device__ __forceinline__ void update_bc(long t, const lns3d_params &p, const d
     for (int r = 1; r < 5; r++) put(r, d, u[r]);
   }
 }
-// the larger of two magnitudes, not a number if either is none (fmax returns
-// the other one then, and a field of NaN would have the norm 0)
-__device__ __forceinline__ double max_mag(double a, double b) { return a == a && !(b <= a) ? b : a; }
 // the max norms of a refined step's residual from nb pairs of partial ones
 // (one workgroup of 256)
 __device__ __forceinline__ void residual_final(const double *part, int nb, double *norms) {
   __shared__ double s1[256], s2[256];
   double a = 0.0, b = 0.0;
   for (int k = threadIdx.x; k < nb; k += blockDim.x) {
-    a = max_mag(a, part[2 * k]);
-    b = max_mag(b, part[2 * k + 1]);
+    a = fmax(a, part[2 * k]);
+    b = fmax(b, part[2 * k + 1]);
   }
   s1[threadIdx.x] = a;
   s2[threadIdx.x] = b;
   __syncthreads();
   for (int w = blockDim.x / 2; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) {
-      s1[threadIdx.x] = max_mag(s1[threadIdx.x], s1[threadIdx.x + w]);
-      s2[threadIdx.x] = max_mag(s2[threadIdx.x], s2[threadIdx.x + w]);
+      s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + w]);
+      s2[threadIdx.x] = fmax(s2[threadIdx.x], s2[threadIdx.x + w]);
     }
     __syncthreads();
   }
@@ -1871,7 +1868,9 @@ __device__ __forceinline__ int slot_col(int N, int per, int pos, int k) {
 // direction; boundary-condition rows as lhs_entry.  Equal to the assembled
 // block rows up to rounding.
 // With b, y is the residual b - L x, and my, mb take the largest parts of y
-// and b at this thread's point.
+// and b at this thread's point; my is infinite where a part of y is not a
+// number (fmax would drop it, and a field of NaN have the norm 0; it is one
+// wherever b holds one).
 __device__ __forceinline__ void line_op(long bid, const AsmCtx &A, const Coeffs &c, int dir, const double2 *x,
                                         double2 *y, const double2 *b, double &my, double &mb) {
   using namespace st;
@@ -2051,6 +2050,7 @@ __device__ __forceinline__ void line_op(long bid, const AsmCtx &A, const Coeffs 
   // the duplicate row of a periodic line is no unknown of the factor (its
   // solve copies row 0 there, its residual is zero): no operator row
   const bool dup = per && pos == N - 1;
+  bool bad = false;
   for (int r = 0; r < 5; r++) {
     if (ident[r]) out[r] = xc[r];
     if (holdrow) out[r] = z{-xc[r].re, -xc[r].im};
@@ -2058,11 +2058,13 @@ __device__ __forceinline__ void line_op(long bid, const AsmCtx &A, const Coeffs 
     if (b) {
       const z v = ld(b + 5 * q + r);
       o = v - o;
-      my = max_mag(my, max_mag(fabs(o.re), fabs(o.im)));
-      mb = max_mag(mb, max_mag(fabs(v.re), fabs(v.im)));
+      my = fmax(my, fmax(fabs(o.re), fabs(o.im)));
+      bad |= __builtin_isunordered(o.re, o.im);
+      mb = fmax(mb, fmax(fabs(v.re), fabs(v.im)));
     }
     y[5 * q + r] = make_double2(o.re, o.im);
   }
+  if (b && bad) my = __builtin_inf();
 }
 // Workgroups of one wave: a grid of 257x129 points is 130 workgroups of four,
 // half the CUs, and the last of a large grid's wait for room for four (us, L_y
@@ -2080,8 +2082,8 @@ __global__ __launch_bounds__(OP_T, 3) void k_line_residual(AsmCtx A, Coeffs c, i
   line_op(xcd_tile(blockIdx.x, gridDim.x), A, c, dir, x, y, b, my, mb);
 #pragma unroll
   for (int w = 32; w > 0; w >>= 1) {
-    my = max_mag(my, __shfl_xor(my, w));
-    mb = max_mag(mb, __shfl_xor(mb, w));
+    my = fmax(my, __shfl_xor(my, w));
+    mb = fmax(mb, __shfl_xor(mb, w));
   }
   if (threadIdx.x == 0) {
     part[2 * blockIdx.x] = my;
