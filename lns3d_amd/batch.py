@@ -50,9 +50,10 @@ def tune_shapes(params_list, precisions=(0, 1)):
 
 # line-solve variants (lns3d_tune_lines numbering) the batch-level tuner
 # tries for every line shape of a staged batch: plain lines (two per
-# workgroup) with a small LDS footprint or the smallest chunks.  A shape alone
-# is solved fastest by the variant that shortens the chain (twisted lines); a
-# staged launch over thousands of lines is bound by throughput.
+# workgroup) with a small LDS footprint, or in a ring of the smallest chunks
+# (complex float, which the staged steps solve in: of the longest).  A shape
+# alone is solved fastest by the variant that shortens the chain (twisted
+# lines); a staged launch over thousands of lines is bound by throughput.
 BATCH_CANDIDATES = (("plain3", 4), ("plain4", 1))
 
 

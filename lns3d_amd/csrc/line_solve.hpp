@@ -126,7 +126,7 @@ template <int N, int U = 0, typename F> __device__ __forceinline__ void static_f
 // staged right-hand sides.  Between the passes one
 // wave solves rows n-2 and n-1 of both lines.  Bound by the memory from about
 // 400 lines (512 lines of 1023 rows, 3760 bytes a row: 382 us, 5.2 TB/s), by
-// the waves that prepare and sum below (97 of 256 rows 65 us, 0.76 us a chunk
+// the waves that prepare and sum below (97 of 256 rows 64 us, 0.76 us a chunk
 // where the chain takes 0.48).  Before, one line or four per workgroup, its
 // recurrence by broadcasts and the border blocks read from memory where they
 // were used: 474 and 92 us.  Border blocks held in registers two chunks ahead

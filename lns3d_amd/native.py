@@ -387,7 +387,7 @@ def ctx_bytes(p, precision=0) -> int:
 
 # line-solve variants the autotuner times (LNS3D_TUNE_VARIANTS)
 TUNE_VARIANTS = 7
-VARIANT_NAMES = ("plain", "plain, smallest chunks", "twisted", "plain, six-row chunks",
+VARIANT_NAMES = ("plain", "plain, smallest (complex float: longest) chunks", "twisted", "plain, six-row chunks",
                  "plain, small footprint", "twisted, six-row chunks", "twisted, small footprint")
 
 
