@@ -939,8 +939,8 @@ int launch_assemble_ref(const lns3d_params &p, const Coeffs &c, int dir, void *m
 }
 
 // ==========================================================================
-// RHS: the point operator on tiles of up to RT points of one grid row, one
-// workgroup of eight waves each.
+// RHS: the point operator on tiles of one grid row, one workgroup of eight
+// waves each (four where rows fill such tiles badly: rhs_half_tiles).
 //
 // Phase 1, one lane per (column, component) of the tile and HALO columns to
 // either side: v and U_eta of the column into LDS, U_etaeta of the tile's own
@@ -957,15 +957,31 @@ int launch_assemble_ref(const lns3d_params &p, const Coeffs &c, int dir, void *m
 //
 // Bound by the coefficients' stream, 1000 bytes a point of 1224: 1025x257 in
 // 69 us, 4.7 TB/s (copies reach 6.1), 24 grids of 65x33 to 513x257 in 166 us;
-// small grids by one pass through the phases (65x33 10 us).  Before, U_xi was
+// small grids by one pass through the phases (65x33 9 us).  Before, U_xi was
 // stored by a kernel of its own, the operator read it over seven rows and its
 // coefficients' loads came behind the stencils: 101, 255 and 15 us.
 // Eight waves, so that two workgroups fill a CU at 128 registers (of five-wave
 // ones, one a row of the operator, a CU held two: its first SIMD takes two
-// waves of each); RT is the widest tile with one task a lane in phase 1.
-constexpr int RHS_THREADS = 512, HALO = 4, RT = RHS_THREADS / 5 - 2 * HALO;
+// waves of each); a tile is at most as wide as leaves one task a lane in phase
+// 1, 94 points (43 with four waves).
+constexpr int RHS_THREADS = 512, HALO = 4;
+__host__ __device__ constexpr int rhs_tile(int threads) { return threads / 5 - 2 * HALO; }
 // tiles of a row; they share its columns evenly
-__host__ __device__ __forceinline__ int rhs_row_tiles(int nx) { return (nx + RT - 1) / RT; }
+__host__ __device__ __forceinline__ int rhs_row_tiles(int nx, int threads) {
+  const int rt = rhs_tile(threads);
+  return (nx + rt - 1) / rt;
+}
+
+// Workgroups of half the lanes, of which twice as many share a CU, where they
+// leave no more lanes idle: a row's tiles share its columns evenly, and one
+// column more than a tile leaves two tiles half empty.  us, 512 / 256 lanes:
+// 33x257 11.2 / 9.3, 65x33 9.5 / 8.8, 95x600 27.0 / 21.0 (with a kernel for U_xi
+// before it, over runs of 64 points, 25), 129x257 16.5 / 12.6, 189x257
+// 21.1 / 17.2, 257x1000 63 / 58; not at 94x600 (one full tile) 20.1 / 21.1.  A
+// staged batch, one launch for members of all widths, keeps the full tiles
+static bool rhs_half_tiles(int nx) {
+  return rhs_row_tiles(nx, RHS_THREADS / 2) <= 2 * rhs_row_tiles(nx, RHS_THREADS);
+}
 
 struct StepBatchItem;
 struct RhsMember {           // what the kernel reads of a staged batch's member
@@ -981,8 +997,8 @@ __device__ __forceinline__ RhsMember rhs_member(const StepBatchItem *items, cons
 // buffers replace the arguments, from items; its workgroups are numbered
 // from off[member]).  Tiles are numbered per XCD: those of neighbouring rows,
 // which share v, on one L2.
-template <bool BATCH>
-__global__ __launch_bounds__(RHS_THREADS, 4) void k_rhs(lns3d_params p_, Stencil st_, Coeffs c_, const double2 *v_,
+template <bool BATCH, int THREADS>
+__global__ __launch_bounds__(THREADS, 4) void k_rhs(lns3d_params p_, Stencil st_, Coeffs c_, const double2 *v_,
                                                     double2 *r_, int with_rbe, const double2 *v2old,
                                                     const double2 *vold, const double2 *forcing,
                                                     const StepBatchItem *__restrict__ items, const int *__restrict__ off, int count) {
@@ -995,11 +1011,11 @@ __global__ __launch_bounds__(RHS_THREADS, 4) void k_rhs(lns3d_params p_, Stencil
   const Coeffs &c = *mb.c;
   const double2 *v = mb.v;
   double2 *r = mb.r;
-  constexpr int NC = RT + 2 * HALO;    // columns held
+  constexpr int NC = rhs_tile(THREADS) + 2 * HALO;    // columns held
   __shared__ double2 sv[5 * NC], su[5 * NC], s22[4 * NC], s1[5 * NC], s11[4 * NC], s12[4 * NC];
   const int nx = p.nx, ny = p.ny;
   const long P = (long)nx * ny;
-  const int nt = rhs_row_tiles(nx), j = (int)((unsigned)bid / (unsigned)nt), tt = (int)bid - j * nt;
+  const int nt = rhs_row_tiles(nx, THREADS), j = (int)((unsigned)bid / (unsigned)nt), tt = (int)bid - j * nt;
   const int wid = nx / nt, rem = nx - wid * nt;
   const int i0 = tt * wid + min(tt, rem), npt = wid + (tt < rem);
   const long q0 = (long)j * nx + i0;
@@ -1301,9 +1317,13 @@ __global__ __launch_bounds__(RHS_THREADS, 4) void k_rhs(lns3d_params p_, Stencil
 
 int launch_rhs(const lns3d_params &p, const Stencil &st, const Coeffs &c, const void *v, void *r, int with_rbe,
                hipStream_t s, const void *v2old, const void *vold, const void *forcing) {
-  hipLaunchKernelGGL(k_rhs<false>, dim3((unsigned)((long)rhs_row_tiles(p.nx) * p.ny)), dim3(RHS_THREADS), 0, s, p, st,
-                     c, (const double2 *)v, (double2 *)r, with_rbe, (const double2 *)v2old, (const double2 *)vold,
-                     (const double2 *)forcing, nullptr, nullptr, 0);
+  auto launch = [&](auto k, int threads) {
+    hipLaunchKernelGGL(k, dim3((unsigned)((long)rhs_row_tiles(p.nx, threads) * p.ny)), dim3(threads), 0, s, p, st, c,
+                       (const double2 *)v, (double2 *)r, with_rbe, (const double2 *)v2old, (const double2 *)vold,
+                       (const double2 *)forcing, nullptr, nullptr, 0);
+  };
+  if (rhs_half_tiles(p.nx)) launch(k_rhs<false, RHS_THREADS / 2>, RHS_THREADS / 2);
+  else launch(k_rhs<false, RHS_THREADS>, RHS_THREADS);
   LNS3D_CHECK(hipGetLastError());
   return 0;
 }
@@ -2202,7 +2222,7 @@ __global__ __launch_bounds__(256) void kb_norm_final(const StepBatchItem *items,
 static long stage_blocks(int stage, const lns3d_params &p) {
   const long P = (long)p.nx * p.ny;
   switch (stage) {
-    case SB_STAGE_RHS: return (long)rhs_row_tiles(p.nx) * p.ny;
+    case SB_STAGE_RHS: return (long)rhs_row_tiles(p.nx, RHS_THREADS) * p.ny;
     case SB_STAGE_LINE: return nblocks(P, OP_T);
     case SB_STAGE_VEC: return nblocks(5 * P, 256);
     case SB_STAGE_LR: return bc_after_update(p) ? nblocks(p.ny, 128) : 0;
@@ -2277,7 +2297,7 @@ void step_batch_free(StepBatch &b) {
 
 int step_batch_rhs(const StepBatch &b, hipStream_t s) {
   const auto *it = (const StepBatchItem *)b.items;
-  hipLaunchKernelGGL(k_rhs<true>, dim3((unsigned)b.blocks[SB_STAGE_RHS]), dim3(RHS_THREADS), 0, s, lns3d_params{},
+  hipLaunchKernelGGL((k_rhs<true, RHS_THREADS>), dim3((unsigned)b.blocks[SB_STAGE_RHS]), dim3(RHS_THREADS), 0, s, lns3d_params{},
                      Stencil{}, Coeffs{}, nullptr, nullptr, 1, nullptr, nullptr, nullptr, it, b.off[SB_STAGE_RHS],
                      b.count);
   LNS3D_CHECK(hipGetLastError());
